@@ -243,6 +243,11 @@ struct IgemmPlan {
   size_t staged_elems = 0;  // channels-last copy of the GEMM's input operand
   size_t table_bytes = 0;   // geometry tables (IgemmArgs::tables)
   PadArgs stage{};          // octet-major copy of the GEMM input (no padding)
+  // The GEMM input's channels per group are no whole octets: staged with zero channels up to
+  // the next octet. Calls that cannot have the staging scratch or the geometry tables (the
+  // allocation-free entry beyond its scratch, a first call under stream capture) run such a
+  // problem on the direct kernels, which need neither.
+  bool padded = false;
   int conflict = 1;         // lanes per 16-byte bank slot in a B-fragment read (1 = none)
   double cost = 0.0;
 };
@@ -436,11 +441,16 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   const int R = g.rank;
   const int real_cin = static_cast<int>(mode == 0 ? g.cin_g : g.cout_g);
   if (split && real_cin > kSplitMaxChannels) return plan;
-  const int gemm_cin = split ? (kSplit * real_cin + 7) / 8 * 8 : real_cin;
+  const int gemm_cin = ((split ? kSplit : 1) * real_cin + 7) / 8 * 8;
   const int gemm_cout = static_cast<int>(mode == 0 ? g.cout_g : g.cin_g);
-  if (gemm_cin % 8 != 0) return plan;
-  // The split copies multiply the staged input; keep it int32-addressable.
-  if (split && (int64_t)gemm_cin * g.groups * g.batch *
+  // 16-bit channel counts that are no whole octets run here too, on an octet-major copy with
+  // zero channels: at worst (one channel) seven eighths of the MFMA work is padding, which still
+  // beats the direct kernels' one serial chain of loads per output (3 -> 32 channels, 3^4 taps,
+  // 145,350 outputs: 3549 -> 34 us; 20 -> 36 channels on 9x13x11x14: 3637 -> 20 us).
+  const bool padded = !split && gemm_cin != real_cin;
+  // The split copies and the zero channels of partial octets multiply the staged input; keep it
+  // int32-addressable.
+  if ((split || padded) && (int64_t)gemm_cin * g.groups * g.batch *
                        (mode == 0 ? g.in_vol : g.out_vol) > kI32Safe / 2)
     return plan;
   const int out_es = split ? 4 : 2;
@@ -484,7 +494,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   // one so far, so they are tried only on request (nbuf=2).
   // Input gradients of strided convolutions (several stride phases) measured slower with
   // direct staging: octet copy there unless requested.
-  if (is_half(dt) && filter.ds != 0 && (nphase == 1 || filter.ds == 1)) {
+  if (is_half(dt) && !padded && filter.ds != 0 && (nphase == 1 || filter.ds == 1)) {
     if (filter.nbuf == 2) staging_options.push_back({true, 2});
     if (filter.nbuf != 2) staging_options.push_back({true, 1});
   }
@@ -704,8 +714,14 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   }
   if (plan.ok) {
     IgemmArgs& A = plan.args;
+    plan.padded = padded;
     plan.wpk_elems = (size_t)A.nphase * A.groups * A.nchunk * A.kc_max * A.mtiles_padded * 64 * 8;
     plan.staged_elems = (size_t)A.batch * A.in_vol * A.cin_total;
+    // The packing pass indexes weight elements with 32 bits.
+    if (padded && plan.wpk_elems > (size_t)kI32Safe) {
+      plan.ok = false;
+      return plan;
+    }
     // Byte offsets into the staged operand are 32-bit (buffer loads, an offset of 0xffffffe0
     // or more reads zero).
     if (plan.staged_elems * 2 > 0xffffffe0ull) {
@@ -1819,6 +1835,16 @@ int run_forward(const Geom& g, convnd_hip_dtype dtype, const ForwardSetup& f, co
   return st;
 }
 
+// The forward plan's geometry tables (kept null for the plans without any). A first call under
+// stream capture has none: a padded plan then becomes the direct kernel's, any other fails.
+bool forward_tables(const Geom& g, convnd_hip_dtype dtype, ForwardSetup* f, hipStream_t stream,
+                    TablesRef* tables) {
+  if (!f->ig.ok) return true;
+  *tables = igemm_device_tables(plan_key(g, dtype, 0), f->ig.args, stream);
+  if (*tables == nullptr && f->ig.padded) f->ig.ok = false;
+  return *tables != nullptr || !f->ig.ok;
+}
+
 // ---- channels-last I/O -----------------------------------------------------------------
 // The implicit GEMM with direct staging (16-bit data) reads [N][in...][C] and writes
 // [N][out...][Co] itself. Every other plan runs channels-first on copies in the workspace,
@@ -1854,7 +1880,8 @@ struct ClBackward {
 ClBackward cl_backward_plan(const Geom& g, convnd_hip_dtype dt, const BackwardSetup& b, bool gi,
                             bool gw, bool gb) {
   ClBackward c;
-  const bool mfma_dx = gi && g.batch > 0 && b.dg.ok;
+  // (A padded plan may become the direct kernel's, which writes channels-first only.)
+  const bool mfma_dx = gi && g.batch > 0 && b.dg.ok && !b.dg.padded;
   // The weight and bias gradients read a channels-first grad_output copy; the input gradient
   // then stages from it as well, and reads channels-last grad_output only when it is alone.
   c.dgrad_cl = mfma_dx && !gw && !gb && igemm_stages_cl(b.dg);
@@ -1912,7 +1939,14 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   // sums part of the same launch); otherwise grad_output is reduced on its own.
   const bool tiny_bias = gb && gw && b.tdw.ok;
   const bool cm_bias = gb && gw && b.wg.ok && b.wg.cm && is_half(dtype);
-  const bool fused_bias = gb && !cm_bias && !tiny_bias && gi && b.dg.ok && is_half(dtype);
+  TablesRef dx_tables, dw_tables;  // held until the kernels that read them are enqueued
+  bool mfma_dx = gi && b.dg.ok;
+  if (mfma_dx) {
+    dx_tables = igemm_device_tables(plan_key(g, dtype, 64), b.dg.args, stream);
+    if (dx_tables == nullptr && !b.dg.padded) return CONVND_HIP_LAUNCH_FAILED;
+    mfma_dx = dx_tables != nullptr;  // (a padded plan without tables: the direct kernel)
+  }
+  const bool fused_bias = gb && !cm_bias && !tiny_bias && mfma_dx && is_half(dtype);
   if (gb && !fused_bias && !cm_bias && !tiny_bias) {
     st = hip_check(launch_grad_bias(dtype, g.batch, g.out_channels, g.out_vol, grad_output,
                                     grad_bias, reinterpret_cast<float*>(ws + b.off_bias),
@@ -1923,17 +1957,17 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   // Staging passes of both MFMA gradients (grad_output channels-last copy with the bias
   // sums, input-gradient weight packing, octet-major input, padded grad_output) in one
   // launch.
-  const bool mfma_dx = gi && b.dg.ok, mfma_dw = gw && b.wg.ok;
+  const bool mfma_dw = gw && b.wg.ok;
   IgemmArgs DA{};
   WgradArgs WA{};
   WgradCmArgs CA{};
   float* sums = fused_bias ? reinterpret_cast<float*>(ws + b.off_bias) : nullptr;
   PrologueParts pp;
-  TablesRef dx_tables, dw_tables;  // held until the kernels that read them are enqueued
+  // Channel sums from the octet-major copy's blocks, or from a part of their own where the GEMM
+  // stages grad_output itself or the copy holds zero channels besides grad_output's.
+  const bool own_sums = mfma_dx && (b.dg.args.direct != 0 || b.dg.padded);
   if (mfma_dx) {
     DA = b.dg.args;
-    dx_tables = igemm_device_tables(plan_key(g, dtype, 64), DA, stream);
-    if (dx_tables == nullptr) return CONVND_HIP_LAUNCH_FAILED;
     DA.tables = dx_tables->dev;
     DA.in = DA.direct ? (dy_cl != nullptr ? dy_cl : grad_output)
                       : static_cast<const void*>(ws + b.off_dy_stage);
@@ -1942,19 +1976,18 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
     DA.wpk = ws + b.off_wpk;
     DA.bias = nullptr;
     DA.out = grad_input;
-    if (DA.direct) {
-      if (sums != nullptr) {
-        pp.sum_src = grad_output;
-        pp.sum_out = sums;
-        pp.sum_batch = g.batch;
-        pp.sum_channels = g.out_channels;
-        pp.sum_volume = g.out_vol;
-      }
-    } else {
+    if (own_sums && sums != nullptr) {
+      pp.sum_src = grad_output;
+      pp.sum_out = sums;
+      pp.sum_batch = g.batch;
+      pp.sum_channels = g.out_channels;
+      pp.sum_volume = g.out_vol;
+    }
+    if (!DA.direct) {
       pp.sa = &b.dg.stage;
       pp.src = grad_output;
       pp.staged = ws + b.off_dy_stage;
-      pp.sums = sums;
+      pp.sums = own_sums ? nullptr : sums;
       pp.batch = g.batch;
     }
     pp.ig = &DA;
@@ -2024,8 +2057,8 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   // The bias gradient from the staging sums rides in the weight-gradient reduction's launch
   // when there is one.
   const bool bias_in_reduce = fused_bias && mfma_dw;
-  const int64_t nsum = mfma_dx && DA.direct ? prologue_sum_blocks(g.batch, g.out_vol)
-                                            : octet_sum_blocks(g.batch, g.out_vol);
+  const int64_t nsum = own_sums ? prologue_sum_blocks(g.batch, g.out_vol)
+                                : octet_sum_blocks(g.batch, g.out_vol);
   if (fused_bias && !bias_in_reduce) {
     st = hip_check(launch_grad_bias_from_sums(dtype, sums, nsum, g.out_channels, grad_bias, stream),
                    "bias gradient");
@@ -2207,15 +2240,12 @@ int convnd_hip_forward_act(const convnd_hip_problem* problem, convnd_hip_dtype d
   if (st != CONVND_HIP_SUCCESS) return st;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   if (g.batch == 0) return CONVND_HIP_SUCCESS;
-  const ForwardSetup f = setup_forward(g, dtype);
+  ForwardSetup f = setup_forward(g, dtype);
   if (workspace_size < f.bytes || (f.bytes > 0 && workspace == nullptr))
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "device workspace is smaller than convnd_hip_forward_workspace_size");
   TablesRef tables;  // held until the kernels that read them are enqueued
-  if (f.ig.ok) {
-    tables = igemm_device_tables(plan_key(g, dtype, 0), f.ig.args, stream);
-    if (tables == nullptr) return CONVND_HIP_LAUNCH_FAILED;
-  }
+  if (!forward_tables(g, dtype, &f, stream, &tables)) return CONVND_HIP_LAUNCH_FAILED;
   return run_forward(g, dtype, f, input, weight, bias, output, activation,
                      static_cast<char*>(workspace), tables ? tables->dev : nullptr, nullptr, true,
                      stream);
@@ -2229,12 +2259,13 @@ int convnd_hip_forward_noalloc(const convnd_hip_problem* problem, convnd_hip_dty
   if (st != CONVND_HIP_SUCCESS) return st;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   if (g.batch == 0) return CONVND_HIP_SUCCESS;
-  const ForwardSetup f = setup_forward(g, dtype);
+  ForwardSetup f = setup_forward(g, dtype);
+  // Scratch: [geometry tables | the workspace regions of convnd_hip_forward].
+  const size_t tab = f.ig.ok ? align_up(static_cast<size_t>(f.ig.args.tab_bytes)) : 0;
+  if (f.ig.ok && f.ig.padded && tab + f.bytes > kNoAllocScratchBytes) f.ig.ok = false;
   if (!f.ig.ok)  // the direct kernels use no scratch
     return run_forward(g, dtype, f, input, weight, bias, output, CONVND_HIP_ACT_NONE, nullptr,
                        nullptr, nullptr, false, stream);
-  // Scratch: [geometry tables | the workspace regions of convnd_hip_forward].
-  const size_t tab = align_up(static_cast<size_t>(f.ig.args.tab_bytes));
   if (tab + f.bytes > kNoAllocScratchBytes)
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "convnd_hip_forward_noalloc: this problem needs " + std::to_string(tab + f.bytes) +
@@ -2307,16 +2338,13 @@ int convnd_hip_forward_layout(const convnd_hip_problem* problem, convnd_hip_dtyp
   if (st != CONVND_HIP_SUCCESS) return st;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   if (g.batch == 0) return CONVND_HIP_SUCCESS;
-  const ForwardSetup f = setup_forward(g, dtype);
+  ForwardSetup f = setup_forward(g, dtype);
   const size_t need = convnd_hip_forward_workspace_size_layout(problem, dtype, layout);
   if (workspace_size < need || (need > 0 && workspace == nullptr))
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "device workspace is smaller than convnd_hip_forward_workspace_size_layout");
   TablesRef tables;  // held until the kernels that read them are enqueued
-  if (f.ig.ok) {
-    tables = igemm_device_tables(plan_key(g, dtype, 0), f.ig.args, stream);
-    if (tables == nullptr) return CONVND_HIP_LAUNCH_FAILED;
-  }
+  if (!forward_tables(g, dtype, &f, stream, &tables)) return CONVND_HIP_LAUNCH_FAILED;
   char* ws = static_cast<char*>(workspace);
   const void* tab = tables ? tables->dev : nullptr;
   const bool out_cl = layout == CONVND_HIP_CHANNELS_LAST;

@@ -1,8 +1,8 @@
 // Direct N-d convolution kernels for gfx950 with 64-bit index arithmetic.
 //
-// They serve every shape the MFMA kernels do not: float64, channel counts that are not a
-// multiple of eight, ranks above eight, huge strides/dilations/padding, and tiny-channel
-// layers that are bound by memory latency rather than by matrix throughput. Each output
+// They serve every shape the MFMA and tiny-channel kernels do not: float64, ranks above eight,
+// huge strides/dilations/padding, and calls of other shapes that cannot have the MFMA kernels'
+// scratch or geometry tables. Each output
 // element is computed by one thread (forward, input gradient) or one workgroup
 // (weight gradient) in a fixed summation order, so results are deterministic.
 //

@@ -63,6 +63,9 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
       live = live && sp < kSplitProducts;
       ci -= sp * A.split_c;
       part = split_other_part(sp);
+    } else {
+      // Zero channels that fill the last octet of the GEMM input.
+      live = live && ci < (A.mode == 0 ? A.wk_cin_g : A.wk_cout_g);
     }
     unsigned short bits = 0;
     if (live) {
