@@ -243,11 +243,13 @@ struct IgemmPlan {
   size_t staged_elems = 0;  // channels-last copy of the GEMM's input operand
   size_t table_bytes = 0;   // geometry tables (IgemmArgs::tables)
   PadArgs stage{};          // octet-major copy of the GEMM input (no padding)
-  // The GEMM input's channels per group are no whole octets: staged with zero channels up to
-  // the next octet. Calls that cannot have the staging scratch or the geometry tables (the
-  // allocation-free entry beyond its scratch, a first call under stream capture) run such a
-  // problem on the direct kernels, which need neither.
+  // 16-bit GEMM input whose channels per group are no whole octets: staged with zero channels
+  // up to the next octet.
   bool padded = false;
+  // Problems that calls without scratch or geometry tables (the allocation-free entry beyond
+  // its scratch, a first call under stream capture) run on the direct kernels, which need
+  // neither, instead of being refused: padded ones, and wide or large split-precision ones.
+  bool or_direct = false;
   int conflict = 1;         // lanes per 16-byte bank slot in a B-fragment read (1 = none)
   double cost = 0.0;
 };
@@ -363,7 +365,7 @@ int64_t choose_pitches(int R, const int* box, const int* sigma, const int* hext,
 // Any subset of the keys may be given; the planner then searches only plans matching it and
 // ignores the override when none does.
 struct PlanFilter {
-  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0;
+  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0;
   std::vector<int> box;
   bool active = false;
 };
@@ -400,6 +402,7 @@ PlanFilter parse_filter(const char* text) {
         if (key == "ds") f.ds = v;
         if (key == "nbuf") f.nbuf = v;
         if (key == "waves") f.waves = v;
+        if (key == "parts") f.parts = v;
       }
     }
     pos = end + 1;
@@ -420,6 +423,10 @@ const PlanFilter& plan_filter(int mode) {
 // see convnd_types.h), when the real channel count per group is small enough to stage.
 constexpr int kSplit = 6;
 constexpr int kSplitMaxChannels = 64;
+// Wider layers (three-part layout only) from one full tile of output channels on (72 -> 16
+// channels, 3^4 taps, 4x4x4x8: 2809 -> 65 us; 96 -> 96 on 8^4, both directions: 25.2 -> 0.44 ms).
+// Narrower ones are pinned to the direct kernels by the plan test.
+constexpr int kSplitWideOut = 16;
 
 IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
                                const PlanFilter& filter);
@@ -440,19 +447,21 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   if ((!is_half(dt) && !split) || g.rank > kFastRank || !fits_int32(g)) return plan;
   const int R = g.rank;
   const int real_cin = static_cast<int>(mode == 0 ? g.cin_g : g.cout_g);
-  if (split && real_cin > kSplitMaxChannels) return plan;
-  const int gemm_cin = ((split ? kSplit : 1) * real_cin + 7) / 8 * 8;
+  // Channels per group along K (of the six copies: split precision, one part).
+  const int real_octs = (real_cin + 7) / 8;
+  const int gemm_cin = split ? (kSplit * real_cin + 7) / 8 * 8 : real_octs * 8;
   const int gemm_cout = static_cast<int>(mode == 0 ? g.cout_g : g.cin_g);
   // 16-bit channel counts that are no whole octets run here too, on an octet-major copy with
   // zero channels: at worst (one channel) seven eighths of the MFMA work is padding, which still
   // beats the direct kernels' one serial chain of loads per output (3 -> 32 channels, 3^4 taps,
   // 145,350 outputs: 3549 -> 34 us; 20 -> 36 channels on 9x13x11x14: 3637 -> 20 us).
   const bool padded = !split && gemm_cin != real_cin;
-  // The split copies and the zero channels of partial octets multiply the staged input; keep it
-  // int32-addressable.
-  if ((split || padded) && (int64_t)gemm_cin * g.groups * g.batch *
-                       (mode == 0 ? g.in_vol : g.out_vol) > kI32Safe / 2)
-    return plan;
+  const bool wide = split && real_cin > kSplitMaxChannels;
+  if (wide && gemm_cout < kSplitWideOut) return plan;
+  // The split copies and the zero channels of partial octets multiply the staged input; it is
+  // kept int32-addressable.
+  const int64_t in_positions = g.groups * g.batch * (mode == 0 ? g.in_vol : g.out_vol);
+  auto staged_fits = [&](int64_t channels) { return channels * in_positions <= kI32Safe / 2; };
   const int out_es = split ? 4 : 2;
   int nphase = 1;
   if (mode == 1) {
@@ -503,11 +512,11 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
       2.0 * 2.0 * double(g.batch) * (mode == 0 ? g.in_vol : g.out_vol) * gemm_cin * g.groups *
       (2.4e9 / 5.0e12);
 
-  // Channel chunk: 8, 16, 32 or 64 channels dividing gemm_cin (octet planes per chunk are
-  // a power of two).
-  std::vector<int> chunk_options;
-  for (int cc = 64; cc >= 8; cc /= 2)
-    if (cc <= gemm_cin && gemm_cin % cc == 0) chunk_options.push_back(cc);
+  // Operand layouts of split precision (IgemmArgs::parts): the parts once each, or the six
+  // copies as one K dimension, whose few channels fill whole octets better (3 channels: 24
+  // channels along K against 6 products x 8). Channel chunk: 1, 2, 3, 4, 6 or 8 octets dividing
+  // the channels along K.
+  const std::vector<int> part_options = split ? std::vector<int>{3, 1} : std::vector<int>{1};
 
   static const int kTiles[][3] = {{1, 2, 1}, {1, 4, 1}, {1, 8, 1}, {2, 2, 1}, {2, 4, 1},
                                   {2, 8, 1}, {4, 2, 1}, {4, 4, 1}, {4, 8, 1}, {1, 4, 2},
@@ -520,13 +529,22 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   std::map<std::vector<int>, PitchMemo> pitch_memo;
   double best = -1.0;
   for (const auto& staging : staging_options)
+  for (const int parts : part_options)
   for (const auto& tile : kTiles)
   for (const int waves : {4, 8}) {
     const bool direct = staging.first;
     const int nbuf = staging.second;
     const int mb = tile[0], nb = tile[1], wm = tile[2], wn = waves / wm;
     // Eight-wave workgroups (one per CU, two waves per SIMD) exist for direct staging.
-    if ((waves == 8 && !direct) || !igemm_tile_supported(mb, nb, wm, waves)) continue;
+    if ((waves == 8 && !direct) || !igemm_tile_supported(mb, nb, wm, waves, parts)) continue;
+    if (filter.parts && filter.parts != parts) continue;
+    const int kcin = parts == 3 ? real_octs * 8 : gemm_cin;  // channels along K
+    const int products = parts == 3 ? kSplit : 1;            // MFMAs per K32 step and fragment pair
+    const int staged_cin = parts == 3 ? 3 * kcin : gemm_cin; // staged channels per group
+    if ((split || padded) && !staged_fits(staged_cin)) continue;
+    // Six copies: few channels, up to the width that always used them.
+    if (parts == 1 && wide) continue;
+    if (parts == 3 && real_cin < 3) continue;
     if (filter.waves && filter.waves != waves) continue;
     // Cover the output channels without idle waves: the waves' M extent may exceed the
     // channel count by less than one wave's share.
@@ -537,11 +555,14 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     const int mgroups = (mtiles + wm * mb - 1) / (wm * mb);
     const int box_vol = wn * nb * 16;
     const int reg_waves = igemm_reg_waves(mb, nb);
-    for (int cc : chunk_options) {
-      if (filter.cc && filter.cc != cc) continue;
-      const int noct = cc / 8;
+    for (const int noct : {8, 6, 4, 3, 2, 1}) {
+      const int cc = noct * 8;
+      if (kcin % cc != 0 || (filter.cc && filter.cc != cc)) continue;
+      const int planes = parts * noct;  // octet planes of a chunk
       const int64_t kc = (ntaps_max * cc + 31) / 32;
-      const int64_t nchunk = gemm_cin / cc;
+      const int64_t nchunk = kcin / cc;
+      // The packing pass indexes weight elements with 32 bits.
+      if (nphase * g.groups * nchunk * kc * parts * mgroups * wm * mb * 512 > kI32Safe) continue;
       // Box coordinates are packed in 16-bit fields up to rank 4 and in 8-bit fields above
       // (extents at most 64 there).
       int limit[kFastRank];
@@ -565,7 +586,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           boxes *= (J[a] + b[a] - 1) / b[a];
           useful *= J[a];
         }
-        if (noct * hvol * 16 > kLdsBudget) return;
+        if (planes * hvol * 16 > kLdsBudget) return;
         // Direct staging moves whole runs of 8 last-axis elements per task and writes them
         // row by row; with halo rows shorter than two runs its tasks are mostly partial and
         // its LDS writes collide (measured about twice as costly as the octet copy there).
@@ -588,7 +609,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         const int64_t plane_pos = hit->second.plane_pos;
         const int64_t plane_bytes = align_up(plane_pos * 16);
         const int tap_row = static_cast<int>((kc + kTapPad + 3) / 4 * 4);
-        const int64_t lds = nbuf * noct * plane_bytes + align_up(rows * 8) +
+        const int64_t lds = nbuf * planes * plane_bytes + align_up(rows * 8) +
                             align_up(box_vol * 4) + align_up(16 * tap_row);
         if (rows > (int64_t{1} << 20)) return;
         // Epilogue stores: a lane writes 4 consecutive positions at once when they are
@@ -607,9 +628,9 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         // plane in a K32 step, which costs a second cycle), A-fragment reads through the
         // vector L1 (about 64 bytes per clock per CU).
         const int lds_factor = std::max(conflict, noct == 1 ? 2 : 1);
-        const double mfma = mb * nb * 16.0;
-        const double ldsc = 4.0 * nb * 4.0 * lds_factor;
-        const double l1 = 4.0 * mb * 1024.0 / 64.0;
+        const double mfma = products * mb * nb * 16.0;
+        const double ldsc = parts * 4.0 * nb * 4.0 * lds_factor;
+        const double l1 = parts * 4.0 * mb * 1024.0 / 64.0;
         const double step = std::max(mfma, std::max(ldsc, l1)) * (waves / 4);
         // Issue efficiency of the main loop: two waves per SIMD hide each other's load
         // latency; one wave per SIMD stalls on its own loads (measured on MI355X: the same
@@ -620,8 +641,8 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         // the previous chunk's MFMAs), each chunk still pays its LDS writes and a barrier.
         const double stage =
             short_rows *
-            (nbuf == 2 ? (noct * hvol * 16.0 / 64.0 + 1500.0) + double(nchunk) * (noct * hvol * 16.0 / 256.0 + 300.0)
-                       : double(nchunk) * (noct * hvol * 16.0 / 64.0 + 1500.0));
+            (nbuf == 2 ? (planes * hvol * 16.0 / 64.0 + 1500.0) + double(nchunk) * (planes * hvol * 16.0 / 256.0 + 300.0)
+                       : double(nchunk) * (planes * hvol * 16.0 / 64.0 + 1500.0));
         // Epilogue: one store per lane of `run` output values.
         const double out_bytes = double(wm) * mb * 16 * box_vol * out_es;
         const double epilogue = out_bytes / (4.0 * out_es * run) + 400.0;
@@ -654,15 +675,16 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         A.batch = static_cast<int>(g.batch);
         A.groups = static_cast<int>(g.groups);
         A.nphase = nphase;
-        A.cin_g = gemm_cin;
+        A.cin_g = staged_cin;
         A.cout_g = gemm_cout;
-        A.cin_total = static_cast<int>(gemm_cin * g.groups);
+        A.cin_total = static_cast<int>(A.cin_g * g.groups);
         A.cout_total = static_cast<int>(gemm_cout * g.groups);
         A.wk_cin_g = static_cast<int>(g.cin_g);
         A.wk_cout_g = static_cast<int>(g.cout_g);
         A.cc = cc;
         A.noct = noct;
-        A.log2_noct = noct == 8 ? 3 : noct == 4 ? 2 : noct == 2 ? 1 : 0;
+        A.parts = parts;
+        A.part_octs = A.cin_g / 8 / parts;
         A.rows = static_cast<int>(rows);
         A.hlast = hext[R - 1];
         A.nchunk = static_cast<int>(nchunk);
@@ -672,7 +694,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         A.mgroups = mgroups;
         A.mtiles_padded = mgroups * wm * mb;
         A.plane_bytes = static_cast<int>(plane_bytes);
-        A.halo_bytes = static_cast<int>(noct * plane_bytes);
+        A.halo_bytes = static_cast<int>(planes * plane_bytes);
         int ivol = 1, ovol = 1;
         for (int a = 0; a < R; ++a) {
           A.hpitch[a] = hpitch[a];
@@ -700,7 +722,8 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         A.packed_ok = run == 4 ? 1 : 0;
         A.coord_bits = R <= 4 ? 16 : 8;
         A.tap_row = tap_row;
-        A.div_mt = make_fast_div(static_cast<unsigned>(A.mtiles_padded));
+        A.div_mt = make_fast_div(static_cast<unsigned>(parts * A.mtiles_padded));
+        A.div_noct = make_fast_div(static_cast<unsigned>(noct));
         A.div_kc = make_fast_div(static_cast<unsigned>(A.kc_max));
         A.div_nchunk = make_fast_div(static_cast<unsigned>(A.nchunk));
         A.div_groups = make_fast_div(static_cast<unsigned>(A.groups));
@@ -715,13 +738,9 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   if (plan.ok) {
     IgemmArgs& A = plan.args;
     plan.padded = padded;
-    plan.wpk_elems = (size_t)A.nphase * A.groups * A.nchunk * A.kc_max * A.mtiles_padded * 64 * 8;
+    plan.or_direct = padded || wide || (split && !staged_fits(gemm_cin));
+    plan.wpk_elems = (size_t)A.nphase * A.groups * A.nchunk * A.kc_max * A.parts * A.mtiles_padded * 64 * 8;
     plan.staged_elems = (size_t)A.batch * A.in_vol * A.cin_total;
-    // The packing pass indexes weight elements with 32 bits.
-    if (padded && plan.wpk_elems > (size_t)kI32Safe) {
-      plan.ok = false;
-      return plan;
-    }
     // Byte offsets into the staged operand are 32-bit (buffer loads, an offset of 0xffffffe0
     // or more reads zero).
     if (plan.staged_elems * 2 > 0xffffffe0ull) {
@@ -760,6 +779,9 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     S.src_cg = real_cin;
     S.dst_cg = A.cin_g;
     S.split_c = split ? real_cin : 0;
+    S.split_pitch = A.parts == 3 ? real_octs * 8 : real_cin;
+    S.split_n = A.parts == 3 ? 3 : kSplit;
+    S.split_map = A.parts == 3 ? kSplitPartsMap : kSplitDataMap;
     S.split_batch = 0;
     for (int a = 0; a < R; ++a) {
       S.in[a] = A.in_size[a];
@@ -1493,10 +1515,10 @@ Setup cached_plan(PlanCache<Setup>& cache, const std::string& key, Make&& make) 
   return setup;
 }
 
-ForwardSetup make_forward(const Geom& g, convnd_hip_dtype dt) {
+// The workspace of an implicit-GEMM forward plan.
+ForwardSetup layout_forward(const IgemmPlan& ig) {
   ForwardSetup f;
-  if (tiny_preferred(g, dt)) f.tiny = plan_tiny(g, dt, 0);
-  if (!f.tiny.ok) f.ig = plan_igemm(g, dt, 0);
+  f.ig = ig;
   Layout L;
   if (f.ig.ok) {
     // Staged operands and packed weights are 16-bit (bf16 parts for split-precision fp32).
@@ -1505,6 +1527,15 @@ ForwardSetup make_forward(const Geom& g, convnd_hip_dtype dt) {
   }
   f.bytes = L.total;
   return f;
+}
+
+ForwardSetup make_forward(const Geom& g, convnd_hip_dtype dt) {
+  if (tiny_preferred(g, dt)) {
+    ForwardSetup f;
+    f.tiny = plan_tiny(g, dt, 0);
+    if (f.tiny.ok) return f;
+  }
+  return layout_forward(plan_igemm(g, dt, 0));
 }
 
 struct BackwardSetup {
@@ -1836,12 +1867,12 @@ int run_forward(const Geom& g, convnd_hip_dtype dtype, const ForwardSetup& f, co
 }
 
 // The forward plan's geometry tables (kept null for the plans without any). A first call under
-// stream capture has none: a padded plan then becomes the direct kernel's, any other fails.
+// stream capture has none: an or_direct plan then becomes the direct kernel's, any other fails.
 bool forward_tables(const Geom& g, convnd_hip_dtype dtype, ForwardSetup* f, hipStream_t stream,
                     TablesRef* tables) {
   if (!f->ig.ok) return true;
   *tables = igemm_device_tables(plan_key(g, dtype, 0), f->ig.args, stream);
-  if (*tables == nullptr && f->ig.padded) f->ig.ok = false;
+  if (*tables == nullptr && f->ig.or_direct) f->ig.ok = false;
   return *tables != nullptr || !f->ig.ok;
 }
 
@@ -1880,8 +1911,8 @@ struct ClBackward {
 ClBackward cl_backward_plan(const Geom& g, convnd_hip_dtype dt, const BackwardSetup& b, bool gi,
                             bool gw, bool gb) {
   ClBackward c;
-  // (A padded plan may become the direct kernel's, which writes channels-first only.)
-  const bool mfma_dx = gi && g.batch > 0 && b.dg.ok && !b.dg.padded;
+  // (An or_direct plan may become the direct kernel's, which writes channels-first only.)
+  const bool mfma_dx = gi && g.batch > 0 && b.dg.ok && !b.dg.or_direct;
   // The weight and bias gradients read a channels-first grad_output copy; the input gradient
   // then stages from it as well, and reads channels-last grad_output only when it is alone.
   c.dgrad_cl = mfma_dx && !gw && !gb && igemm_stages_cl(b.dg);
@@ -1943,8 +1974,8 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   bool mfma_dx = gi && b.dg.ok;
   if (mfma_dx) {
     dx_tables = igemm_device_tables(plan_key(g, dtype, 64), b.dg.args, stream);
-    if (dx_tables == nullptr && !b.dg.padded) return CONVND_HIP_LAUNCH_FAILED;
-    mfma_dx = dx_tables != nullptr;  // (a padded plan without tables: the direct kernel)
+    if (dx_tables == nullptr && !b.dg.or_direct) return CONVND_HIP_LAUNCH_FAILED;
+    mfma_dx = dx_tables != nullptr;  // (an or_direct plan without tables: the direct kernel)
   }
   const bool fused_bias = gb && !cm_bias && !tiny_bias && mfma_dx && is_half(dtype);
   if (gb && !fused_bias && !cm_bias && !tiny_bias) {
@@ -2261,11 +2292,23 @@ int convnd_hip_forward_noalloc(const convnd_hip_problem* problem, convnd_hip_dty
   if (g.batch == 0) return CONVND_HIP_SUCCESS;
   ForwardSetup f = setup_forward(g, dtype);
   // Scratch: [geometry tables | the workspace regions of convnd_hip_forward].
-  const size_t tab = f.ig.ok ? align_up(static_cast<size_t>(f.ig.args.tab_bytes)) : 0;
-  if (f.ig.ok && f.ig.padded && tab + f.bytes > kNoAllocScratchBytes) f.ig.ok = false;
+  size_t tab = f.ig.ok ? align_up(static_cast<size_t>(f.ig.args.tab_bytes)) : 0;
+  if (f.ig.ok && tab + f.bytes > kNoAllocScratchBytes) {
+    if (f.ig.or_direct) {
+      f.ig.ok = false;
+    } else if (f.ig.args.parts == 3) {
+      // Split precision whose three-part plan exceeds the scratch: six copies may still fit.
+      PlanFilter six;
+      six.parts = 1;
+      const IgemmPlan ig = plan_igemm_filtered(g, dtype, 0, six);
+      const ForwardSetup f6 = layout_forward(ig);
+      if (ig.ok && align_up(static_cast<size_t>(ig.args.tab_bytes)) + f6.bytes <= kNoAllocScratchBytes) f = f6;
+    }
+  }
   if (!f.ig.ok)  // the direct kernels use no scratch
     return run_forward(g, dtype, f, input, weight, bias, output, CONVND_HIP_ACT_NONE, nullptr,
                        nullptr, nullptr, false, stream);
+  tab = align_up(static_cast<size_t>(f.ig.args.tab_bytes));
   if (tab + f.bytes > kNoAllocScratchBytes)
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "convnd_hip_forward_noalloc: this problem needs " + std::to_string(tab + f.bytes) +
@@ -2452,6 +2495,7 @@ std::string check_igemm_tables(const IgemmArgs& A0, size_t lds_bytes, const char
   igemm_build_tables(A, tab.data());
   auto fail_at = [&](const std::string& m) { return std::string(what) + ": " + m; };
   const int positions_per_plane = A.plane_bytes / 16;
+  const int part_bytes = A.halo_bytes / A.parts;  // tap offsets address one part's planes
   const int nbuf = A.direct ? A.nbuf : 1;
   // LDS carve-up: halo buffers, row tables (2 ints per row), box output offsets, taps.
   const size_t lds_need = (size_t)nbuf * A.halo_bytes + (size_t)A.rows * 8 +
@@ -2475,10 +2519,10 @@ std::string check_igemm_tables(const IgemmArgs& A0, size_t lds_bytes, const char
     for (int lg = 0; lg < 4; ++lg) {
       const int* row = taps + (ph * 4 + lg) * A.tap_row;
       for (int k = 0; k < A.tap_row; ++k)
-        if (row[k] < 0 || max_pos + row[k] + 16 > A.halo_bytes)
+        if (row[k] < 0 || max_pos + row[k] + 16 > part_bytes)
           return fail_at("tap offset reads past the halo");
       const int t = tail[ph * 4 + lg];
-      if (t < -1 || (t >= 0 && max_pos + t + 16 > A.halo_bytes))
+      if (t < -1 || (t >= 0 && max_pos + t + 16 > part_bytes))
         return fail_at("tail tap offset reads past the halo");
       for (int k = 0; k < A.kc_max; ++k) {
         const int* e = pack + ((ph * A.kc_max + k) * 4 + lg) * 2;
@@ -2616,6 +2660,7 @@ int convnd_hip_plan_describe(const convnd_hip_problem* problem, convnd_hip_dtype
              ",\"conflict\":" + std::to_string(p.conflict) +
              ",\"boxes\":" + std::to_string(A.boxes) + ",\"phases\":" +
              std::to_string(A.nphase) + ",\"cc\":" + std::to_string(A.cc) +
+             ",\"parts\":" + std::to_string(A.parts) +
              ",\"nchunk\":" + std::to_string(A.nchunk) + ",\"kc_max\":" +
              std::to_string(A.kc_max) + ",\"mgroups\":" + std::to_string(A.mgroups) +
              ",\"lds\":" + std::to_string(p.lds) + ",\"direct\":" + std::to_string(A.direct) +

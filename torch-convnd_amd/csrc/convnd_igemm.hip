@@ -39,10 +39,36 @@ namespace {
 template <int MB, int NB>
 constexpr int igemm_waves = MB * NB >= 32 ? 1 : 2;
 
+// body(std::integral_constant<int, 0>) .. <N - 1>.
+template <int N, typename F, int I = 0>
+__device__ __forceinline__ void unrolled(F&& body) {
+  if constexpr (I < N) {
+    body(std::integral_constant<int, I>{});
+    unrolled<N, F, I + 1>(static_cast<F&&>(body));
+  }
+}
+
+// The six part products of one K32 step, smallest first: position parts b, weight parts a.
+template <typename M, int MB, int NB>
+__device__ __forceinline__ void part_products(const typename M::frag (*b)[NB],
+                                              const typename M::frag (*a)[MB],
+                                              f32x4 (&acc)[MB][NB]) {
+  constexpr int kData[6] = {1, 2, 0, 1, 0, 0};
+  constexpr int kOther[6] = {1, 0, 2, 0, 1, 0};
+#pragma unroll
+  for (int q = 0; q < 6; ++q)
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        acc[mb][nb] = M::run(b[kData[q]][nb], a[kOther[q]][mb], acc[mb][nb]);
+}
+
 // T: GEMM operand type; O: output and bias type (T, or float for split-precision fp32).
+// P: bf16 parts of split-precision fp32 staged and packed once each (3), else 1.
 // Every per-axis quantity comes from the geometry tables (IgemmArgs::tables), so the
 // kernel body is the same for every rank.
-template <typename T, typename O, int MB, int NB, int WM, bool DS, int W>
+template <typename T, typename O, int MB, int NB, int WM, bool DS, int W, int P = 1>
 __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(igemm_waves<MB, NB>, igemm_waves<MB, NB>)))
 void igemm_kernel(IgemmArgs A) {
@@ -131,7 +157,7 @@ void igemm_kernel(IgemmArgs A) {
   const int hlast = A.hlast;
   const int corg = box.corg;
   const int last_size = A.last_size;
-  const int onoct = A.noct - 1;
+  const int noct = A.noct;
   const T* in = static_cast<const T*>(A.in);
   const frag* wp = static_cast<const frag*>(A.wpk);
   f32x4 acc[MB][NB];
@@ -140,7 +166,8 @@ void igemm_kernel(IgemmArgs A) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const size_t wstep = (size_t)A.mtiles_padded * 64;  // fragments per K32 step
+  const size_t wpart = (size_t)A.mtiles_padded * 64;  // fragments per part of a K32 step
+  const size_t wstep = P * wpart;                     // fragments per K32 step
   constexpr unsigned kPast = 0xffffffe0u;  // past every staged tensor (planner: < kPast bytes)
   const __amdgpu_buffer_rsrc_t srsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(in), 0, A.in_bytes, 0x00020000);
@@ -152,6 +179,96 @@ void igemm_kernel(IgemmArgs A) {
     const frag* wck = wp +
                       ((size_t)((phase * A.groups + g) * A.nchunk + ck) * A.kc_max) * wstep +
                       (size_t)mt0 * 64 + lane;
+    if constexpr (P == 3) {
+      // Split-precision fp32, each K32 step from the three parts of both operands: 3 MB weight
+      // and 3 NB position fragments feed 6 MB NB MFMAs, half the operand traffic per MFMA of
+      // six copies along K (which a small tile is bound by: the weights through the vector L1
+      // at 64 B per clock, the positions through LDS). Weights kRing - 1 steps ahead (ring),
+      // position fragments one step ahead, tap offsets kUnroll at a time one iteration ahead.
+      // 48 -> 24 channels, 3^4 taps, [2,.,13,11,10,15] (input gradient): 111 -> 78 us.
+      constexpr int kRing = MB * NB <= 2 ? 8 : (MB == 1 ? 4 : 2);
+      constexpr int kUnroll = kRing < 4 ? 4 : kRing;
+      static_assert(kUnroll <= kTapPad && kUnroll % kRing == 0 && kUnroll % 4 == 0, "tap prefetch");
+      const int ppitch = noct * A.plane_bytes;  // LDS bytes from one part's planes to the next
+      if (KF > 0) {
+        const int last = KF - 1;
+        auto wstep_at = [&](int k) { return (size_t)(k < last ? k : last) * wstep; };
+        frag ar[kRing][3][MB], br[2][3][NB];
+        auto load_w = [&](frag (*a)[MB], int k) {
+          const size_t at = wstep_at(k);
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) a[p][mb] = wck[at + p * wpart + mb * 64];
+        };
+        auto load_b = [&](frag (*b)[NB], int tap) {
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+              b[p][nb] = *reinterpret_cast<const frag*>(hb + pbase[nb] + tap + p * ppitch);
+        };
+        int4 tq[kUnroll / 4];
+        auto tap_of = [](const int4* q, int j) {
+          const int4 v = q[j >> 2];
+          return (j & 3) == 0 ? v.x : (j & 3) == 1 ? v.y : (j & 3) == 2 ? v.z : v.w;
+        };
+#pragma unroll
+        for (int j = 0; j < kRing - 1; ++j) load_w(ar[j], j);
+#pragma unroll
+        for (int j = 0; j < kUnroll / 4; ++j) tq[j] = *reinterpret_cast<const int4*>(tp + 4 * j);
+        load_b(br[0], tap_of(tq, 0));
+        __builtin_amdgcn_sched_barrier(0);
+        issue();
+        // Step i of an iteration at kc; tb: tap offset of the step after it.
+        auto step = [&](auto ic, int kc, int tb) {
+          constexpr int i = decltype(ic)::value;
+          load_b(br[(i + 1) & 1], tb);
+          load_w(ar[(i + kRing - 1) % kRing], kc + i + kRing - 1);
+          __builtin_amdgcn_sched_barrier(0);
+          part_products<M, MB, NB>(br[i & 1], ar[i % kRing], acc);
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        int kc = 0;
+        for (; kc + kUnroll <= KF; kc += kUnroll) {
+          int4 tn[kUnroll / 4];
+#pragma unroll
+          for (int j = 0; j < kUnroll / 4; ++j)
+            tn[j] = *reinterpret_cast<const int4*>(tp + kc + kUnroll + 4 * j);
+          unrolled<kUnroll>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            step(ic, kc, i + 1 < kUnroll ? tap_of(tq, i + 1) : tap_of(tn, i + 1 - kUnroll));
+          });
+#pragma unroll
+          for (int j = 0; j < kUnroll / 4; ++j) tq[j] = tn[j];
+        }
+        const int left = KF - kc;  // 0 to kUnroll - 1 whole steps remain
+        unrolled<kUnroll - 1>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          if (i < left) step(ic, kc, tap_of(tq, i + 1));
+        });
+      } else {
+        issue();
+      }
+      if (KC > KF) {
+        // The partial last step: zero position fragments past the phase's last tap.
+        frag at[3][MB], bt[3][NB];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) at[p][mb] = wck[(size_t)KF * wstep + p * wpart + mb * 64];
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(hb + pbase[nb] + (tail_tap < 0 ? 0 : tail_tap) +
+                                                      p * ppitch);
+            if (tail_tap < 0) v = u32x4{0u, 0u, 0u, 0u};
+            bt[p][nb] = __builtin_bit_cast(frag, v);
+          }
+        }
+        part_products<M, MB, NB>(bt, at, acc);
+      }
+      return;
+    }
     if (KF > 0 && MB * NB <= 4 && std::is_same<O, float>::value) {
       // Small tiles (at most 4 MFMAs per K step) of split-precision fp32: their packed weights
       // (six part products per channel) mostly come from beyond L2, and a step's MFMAs take
@@ -359,8 +476,8 @@ void igemm_kernel(IgemmArgs A) {
     const unsigned cl_img = static_cast<unsigned>(n) * in_vol;
     const unsigned cl_stride = static_cast<unsigned>(A.cin_total);
     auto task_load = [&](int ck, int t, u32x4* v) {
-      const int o = t & onoct;
-      const int rt = t >> A.log2_noct;
+      const int rt = fast_div(t, A.div_noct);
+      const int o = t - rt * noct;
       const int r = rt / nrun;
       const int jj = rt - r * nrun;
       const int ro = (t < ntask && jj < nrun_box) ? rowin[r] : -1;
@@ -399,8 +516,8 @@ void igemm_kernel(IgemmArgs A) {
       }
     };
     auto task_store = [&](int t, const u32x4* v, unsigned char* buf) {
-      const int o = t & onoct;
-      const int rt = t >> A.log2_noct;
+      const int rt = fast_div(t, A.div_noct);
+      const int o = t - rt * noct;
       const int r = rt / nrun;
       const int jj = rt - r * nrun;
       if (t >= ntask || jj >= nrun_box) return;
@@ -486,10 +603,10 @@ void igemm_kernel(IgemmArgs A) {
       }
     }
   } else {
-    // Staging walk over the octet-major copy: item = ((row * noct) + octet) * hlast +
-    // column, 256 items apart per thread; the division happens once and every later item
+    // Staging walk over the octet-major copy: item = ((row * parts + part) * noct + octet) *
+    // hlast + column, 256 items apart per thread; the division happens once and every later item
     // updates incrementally.
-    const int items = A.rows * A.noct * hlast;
+    const int items = A.rows * P * noct * hlast;
     const int rp0 = tid / hlast, c0 = tid - (tid / hlast) * hlast;
     const int drp = kWT / hlast, dc = kWT - drp * hlast;
     // Halo staging in batches of items per thread: the loads of a batch (branch-free buffer
@@ -504,19 +621,27 @@ void igemm_kernel(IgemmArgs A) {
     const unsigned img_base =
         static_cast<unsigned>(((size_t)n * (A.cin_total >> 3) + (size_t)(g * (A.cin_g >> 3))) *
                               A.in_vol * 16);
+    // Row, octet and part of walk index rp = (row * parts + part) * noct + octet.
+    auto split_item = [&](int rp, int& r, int& o, int& part) {
+      const int q = fast_div(rp, A.div_noct);
+      o = rp - q * noct;
+      r = P == 3 ? static_cast<int>(static_cast<unsigned>(q) / 3u) : q;
+      part = P == 3 ? q - r * 3 : 0;
+    };
     u32x4 pre[kPreBatch];
     auto stage_load = [&](int ck, int it0, int rp, int c, u32x4* v, auto nbatch) {
       const unsigned cbase = img_base + static_cast<unsigned>(ck * A.noct) * A.in_vol * 16u;
 #pragma unroll
       for (int u = 0; u < decltype(nbatch)::value; ++u) {
         const int it = it0 + u * kWT;
-        const int r = rp >> A.log2_noct;
-        const int o = rp & onoct;
+        int r, o, part;
+        split_item(rp, r, o, part);
         const int ro = it < items ? rowin[r < A.rows ? r : 0] : -1;
         const int cl = corg + c;
         const bool ok = ro >= 0 && cl >= 0 && cl < last_size;
+        const unsigned plane = static_cast<unsigned>(part * A.part_octs + o);
         const unsigned off =
-            ok ? cbase + static_cast<unsigned>(o * A.in_vol + ro + cl) * 16u : kPast;
+            ok ? cbase + (plane * A.in_vol + static_cast<unsigned>(ro + cl)) * 16u : kPast;
         v[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(srsrc, off, 0, 0));
         c += dc;
         rp += drp;
@@ -531,9 +656,9 @@ void igemm_kernel(IgemmArgs A) {
       for (int u = 0; u < decltype(nbatch)::value; ++u) {
         const int it = it0 + u * kWT;
         if (it < items) {
-          const int r = rp >> A.log2_noct;
-          const int o = rp & onoct;
-          *reinterpret_cast<u32x4*>(lds + o * A.plane_bytes + (rowlds[r] + c) * 16) = v[u];
+          int r, o, part;
+          split_item(rp, r, o, part);
+          *reinterpret_cast<u32x4*>(lds + (part * noct + o) * A.plane_bytes + (rowlds[r] + c) * 16) = v[u];
         }
         c += dc;
         rp += drp;
@@ -712,6 +837,26 @@ void igemm_kernel(IgemmArgs A) {
 #define CONVND_IGEMM_TILES8(X) \
   X(4, 4, 1) X(2, 4, 1) X(4, 2, 1) X(2, 8, 1) X(1, 8, 1) X(1, 4, 1) X(1, 2, 1) X(2, 2, 1)
 
+// Split precision from three parts (two waves per SIMD, 256 registers each).
+#define CONVND_IGEMM_TILES_P3(X) \
+  X(1, 2, 1) X(1, 4, 1) X(2, 2, 1) X(2, 4, 1) X(1, 4, 2) X(2, 4, 2) X(2, 2, 2) X(1, 4, 4) X(4, 2, 1)
+
+hipError_t igemm_dispatch_p3(int mb, int nb, const IgemmArgs& a, size_t lds, hipStream_t s) {
+  const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * a.nphase);
+#define CONVND_IGEMM_CASE(MBV, NBV, WMV)                                                       \
+  if (mb == MBV && nb == NBV && a.wm == WMV && a.waves == 4) {                                 \
+    auto fn = igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3>;                         \
+    hipError_t err =                                                                           \
+        ensure_dynamic_lds<igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3>>(lds);      \
+    if (err != hipSuccess) return err;                                                         \
+    hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, a);                                        \
+    return hipGetLastError();                                                                  \
+  }
+  CONVND_IGEMM_TILES_P3(CONVND_IGEMM_CASE)
+#undef CONVND_IGEMM_CASE
+  return hipErrorInvalidValue;
+}
+
 template <typename T, typename O, bool DS>
 hipError_t igemm_dispatch(int mb, int nb, const IgemmArgs& a, size_t lds, hipStream_t s) {
   const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * a.nphase);
@@ -742,9 +887,15 @@ hipError_t igemm_dispatch(int mb, int nb, const IgemmArgs& a, size_t lds, hipStr
 
 }  // namespace
 
-bool igemm_tile_supported(int mb, int nb, int wm, int waves) {
+bool igemm_tile_supported(int mb, int nb, int wm, int waves, int parts) {
 #define CONVND_IGEMM_HAS(MBV, NBV, WMV) \
   if (mb == MBV && nb == NBV && wm == WMV) return true;
+  if (parts == 3) {
+    if (waves == 4) {
+      CONVND_IGEMM_TILES_P3(CONVND_IGEMM_HAS)
+    }
+    return false;
+  }
   if (waves == 4) {
     CONVND_IGEMM_TILES(CONVND_IGEMM_HAS)
   } else if (waves == 8) {
@@ -763,6 +914,8 @@ hipError_t launch_igemm(convnd_hip_dtype dtype, int mb, int nb, const IgemmArgs&
   if (dtype == CONVND_HIP_FLOAT16)
     return a.direct ? igemm_dispatch<_Float16, _Float16, true>(mb, nb, a, lds_bytes, stream)
                     : igemm_dispatch<_Float16, _Float16, false>(mb, nb, a, lds_bytes, stream);
+  if (dtype == CONVND_HIP_FLOAT32 && a.split_c > 0 && !a.direct && a.parts == 3)
+    return igemm_dispatch_p3(mb, nb, a, lds_bytes, stream);
   if (dtype == CONVND_HIP_FLOAT32 && a.split_c > 0 && !a.direct)
     return igemm_dispatch<__bf16, float, false>(mb, nb, a, lds_bytes, stream);
   return hipErrorInvalidValue;

@@ -115,12 +115,12 @@ struct IgemmArgs {
   int cin_g, cout_g;          // GEMM reduction channels / output channels per group
   int cin_total, cout_total;
   int wk_cin_g, wk_cout_g;    // channels per group of the original weight tensor
-  int cc, noct, log2_noct;    // channels and octets per LDS chunk (powers of two)
+  int cc, noct;               // channels and octets per LDS chunk
   int nchunk, kc_max;         // chunks, K32 steps per chunk (widest phase)
   int wm;                     // waves along M (output channels); 4 / wm along positions
   int mtiles, mgroups, mtiles_padded;
   int plane_bytes;            // LDS bytes of one octet plane (multiple of 256)
-  int halo_bytes;             // noct * plane_bytes
+  int halo_bytes;             // parts * noct * plane_bytes
   int rows, hlast;            // halo rows (all axes but the last) and last-axis extent
   int hext[kFastRank];        // halo extent per axis (<= 64 on all axes but the last)
   int hpitch[kFastRank];      // halo position pitch per axis (hpitch[rank-1] == 1)
@@ -131,6 +131,12 @@ struct IgemmArgs {
   int k[kFastRank], s[kFastRank], p[kFastRank], d[kFastRank];
   int k_vol;
   int split_c;     // split-precision fp32: real channels per group in the GEMM-input role
+  // Split-precision fp32 operand layout. parts 1: six copies of the channels (one per part
+  // product) as one K dimension. parts 3: the three bf16 parts of every channel once, cin_g =
+  // 3 * part_octs * 8 staged channels per group (part slowest) and three weight fragments per
+  // (step, M tile); every K32 step runs the six part products from registers. 16-bit data: 1.
+  int parts;
+  int part_octs;   // octets of one part's channels per group (all of them: cin_g / 8 / parts)
   int in_bytes;    // bytes of the staged operand (unsigned bit pattern, below 0xffffffe0)
   // Geometry tables in device memory, built once per plan by the host (convnd_geometry.h)
   // and read by the packing pass and the GEMM kernel, which then needs no per-axis code:
@@ -164,8 +170,9 @@ struct IgemmArgs {
   // run of 8 last-axis positions is eight 16-byte loads of one octet's channels, stored
   // without a transpose); out_cl, the output is [N][out_vol][cout_total]. 0: channels-first.
   int in_cl, out_cl;
-  // Divisions of the weight-packing unit index by mtiles_padded, kc_max, nchunk and groups.
-  FastDiv div_mt, div_kc, div_nchunk, div_groups;
+  // Divisions of the weight-packing unit index by parts * mtiles_padded, kc_max, nchunk and
+  // groups, and by the octets of a chunk.
+  FastDiv div_mt, div_kc, div_nchunk, div_groups, div_noct;
 };
 
 constexpr int kTapPad = 16;  // tap-table entries past the last step (prefetch distance)
@@ -398,14 +405,16 @@ hipError_t ensure_dynamic_lds(size_t bytes) {
 // dst[n][c/8][u_0]..[u_{R-1}][c%8] = src[n][c'][u - pad] (zero when u - pad lies outside the
 // input), u_a < pe[a], where destination channel c is channel cc = c % dst_cg of group
 // gi = c / dst_cg: source channel gi*src_cg + cc (zero past src_cg), or with split_c > 0 part
-// split_data_part(s) of source channel gi*split_c + c for cc = s*split_c + c (fp32 source,
-// split-precision GEMM input). With split_batch > 0 (fp32 source) destination image n holds
+// split_map_part(split_map, s) of source channel gi*split_c + c for cc = s*split_pitch + c
+// (fp32 source, split-precision GEMM input; zero for c >= split_c and past split_n copies). With split_batch > 0 (fp32 source) destination image n holds
 // part split_data_part(n / split_batch) of source image n % split_batch.
 struct PadArgs {
   int rank, channels;       // destination channels (groups x dst_cg)
   int src_channels;         // source channels per image
   int src_cg, dst_cg;       // channels per group: source, destination (multiple of 8, zero-filled)
   int split_c;              // split-precision channel copies (fp32 source), else 0
+  int split_pitch, split_n; // channels from one copy to the next, and how many copies
+  unsigned split_map;       // the part that each copy holds
   int split_batch;  // fp32 source: images per split part (destination batch = 6x), else 0
   int in[kFastRank], pe[kFastRank], pad[kFastRank];
   int in_vol, pvol;
@@ -495,9 +504,9 @@ hipError_t launch_grad_bias(convnd_hip_dtype dtype, int64_t batch, int64_t chann
 hipError_t launch_igemm(convnd_hip_dtype dtype, int mb, int nb, const IgemmArgs& a,
                         size_t lds_bytes, hipStream_t stream);
 // Whether launch_igemm has a compiled kernel for this wave tile (mb x nb fragments), wave
-// arrangement (wm waves along output channels) and workgroup size (waves: 4, or 8 with direct
-// staging).
-bool igemm_tile_supported(int mb, int nb, int wm, int waves);
+// arrangement (wm waves along output channels), workgroup size (waves: 4, or 8 with direct
+// staging) and operand layout (parts).
+bool igemm_tile_supported(int mb, int nb, int wm, int waves, int parts);
 // stg: staging slots per thread (8, 16 or 24); multi: the item's staging takes
 // several batches of 8 slots (only the first is prefetched).
 hipError_t launch_wgrad_mfma(convnd_hip_dtype dtype, int mb, int stg, bool multi,

@@ -13,11 +13,12 @@ namespace stage {
 
 // ---- weight packing --------------------------------------------------------------------
 
-// Packed weights: unit u = ((((phase*G + g)*nchunk + chunk)*kc_max + kc)*mtiles_padded
-// + mt)*64 + lane holds the 8 A-fragment elements W'[m][k], m = mt*16 + lane%16,
+// Packed weights: unit u = ((((phase*G + g)*nchunk + chunk)*kc_max + kc)*parts*mtiles_padded
+// + part*mtiles_padded + mt)*64 + lane holds the 8 A-fragment elements W'[m][k], m = mt*16 + lane%16,
 // k = kc*32 + (lane/16)*8 + i (i < 8), zero where m or k is padding.
 // S = float (split precision): GEMM channel ci is part split_other_part(ci / split_c) of
-// channel ci % split_c of the fp32 weight (zero past kSplitProducts copies).
+// channel ci % split_c of the fp32 weight (zero past kSplitProducts copies); with parts == 3
+// channel ci of part `part` (zero from split_c on).
 template <typename T, typename S>
 __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w, T* wpk,
                                                   int units, int block, int nblocks) {
@@ -31,7 +32,14 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
     int r = u >> 6;
     const int lane = u & 63;
     int q = fast_div(r, A.div_mt);
-    const int mt = r - q * A.mtiles_padded;
+    int mt = r - q * (A.parts * A.mtiles_padded);
+    int part = 0;
+    if constexpr (sizeof(S) == 4) {
+      if (A.parts == 3) {
+        part = (mt >= A.mtiles_padded ? 1 : 0) + (mt >= 2 * A.mtiles_padded ? 1 : 0);
+        mt -= part * A.mtiles_padded;
+      }
+    }
     r = q;
     q = fast_div(r, A.div_kc);
     const int kc = r - q * A.kc_max;
@@ -47,22 +55,26 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
     // the input gradient's phases read the plan's map.
     int tflat, chan;
     if (A.mode == 0) {
-      const int kk = kc * 32 + (lane >> 4) * 8;
-      tflat = kk >> (3 + A.log2_noct);  // cc = 8 << log2_noct
-      chan = kk - (tflat << (3 + A.log2_noct));
+      const int ko = kc * 4 + (lane >> 4);  // k-group: (tap, octet of the chunk)
+      tflat = fast_div(ko, A.div_noct);
+      chan = (ko - tflat * A.noct) * 8;
       if (tflat >= A.k_vol) tflat = -1;
     } else {
       const int* pe = pmap + ((phase * A.kc_max + kc) * 4 + (lane >> 4)) * 2;
       tflat = pe[0];
       chan = pe[1];
     }
-    int ci = ck * A.cc + chan + i, part = 0;
+    int ci = ck * A.cc + chan + i;
     bool live = m < A.cout_g && tflat >= 0;
     if constexpr (sizeof(S) == 4) {
-      const int sp = ci / A.split_c;
-      live = live && sp < kSplitProducts;
-      ci -= sp * A.split_c;
-      part = split_other_part(sp);
+      if (A.parts == 3) {
+        live = live && ci < A.split_c;
+      } else {
+        const int sp = ci / A.split_c;
+        live = live && sp < kSplitProducts;
+        ci -= sp * A.split_c;
+        part = split_other_part(sp);
+      }
     } else {
       // Zero channels that fill the last octet of the GEMM input.
       live = live && ci < (A.mode == 0 ? A.wk_cin_g : A.wk_cout_g);
@@ -100,8 +112,8 @@ struct OctetSmem {
 // coordinate u is input coordinate u - P.pad (zero outside the input). Channels, per group
 // of P.dst_cg destination channels:
 //   split_c == 0: channel cc < P.src_cg is source channel g*P.src_cg + cc, zero past it;
-//   split_c > 0 (fp32 source): cc = s*split_c + c holds part split_data_part(s) of source
-//                 channel g*split_c + c (zero past kSplitProducts copies);
+//   split_c > 0 (fp32 source): cc = s*split_pitch + c holds part split_map_part(split_map, s)
+//                 of source channel g*split_c + c (zero for c >= split_c, past split_n copies);
 //   split_batch > 0 (fp32 source): destination image n holds part
 //                 split_data_part(n / split_batch) of source image n % split_batch.
 // Block (position run bx of kOctRun, octet o, image n). Two paths:
@@ -148,10 +160,11 @@ __device__ __forceinline__ void octets16_block(const Src* src, unsigned short* d
     const int cc = c - gi * P.dst_cg;
     int sc = -1, part = ipart < 0 ? 0 : ipart;
     if (P.split_c > 0) {
-      const int sp = cc / P.split_c;
-      if (sp < kSplitProducts) {
-        sc = gi * P.split_c + (cc - sp * P.split_c);
-        part = split_data_part(sp);
+      const int sp = cc / P.split_pitch;
+      const int c1 = cc - sp * P.split_pitch;
+      if (sp < P.split_n && c1 < P.split_c) {
+        sc = gi * P.split_c + c1;
+        part = split_map_part(P.split_map, sp);
       }
     } else if (cc < P.src_cg) {
       sc = gi * P.src_cg + cc;
