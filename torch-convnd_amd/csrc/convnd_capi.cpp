@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdlib>
 #include <cstdint>
 #include <cstring>
@@ -248,9 +249,10 @@ struct IgemmPlan {
   bool padded = false;
   // Problems that calls without scratch or geometry tables (the allocation-free entry beyond
   // its scratch, a first call under stream capture) run on the direct kernels, which need
-  // neither, instead of being refused: padded ones, and wide or large split-precision ones.
+  // neither, instead of being refused: padded ones, wide or large split-precision ones, and
+  // halos that only fit LDS in odd boxes or with split taps.
   bool or_direct = false;
-  int conflict = 1;         // lanes per 16-byte bank slot in a B-fragment read (1 = none)
+  double conflict = 1;      // lanes per 16-byte bank slot in a B-fragment read (1 = none)
   double cost = 0.0;
 };
 
@@ -291,32 +293,123 @@ int occupancy(int64_t lds, int reg_waves = 2) {
 // Waves per SIMD the implicit-GEMM kernel is compiled for (igemm_waves in the kernel file).
 int igemm_reg_waves(int mb, int nb) { return mb * nb >= 32 ? 1 : 2; }
 
-// gfx950 serves a wave-wide 16-byte LDS read in four cycles of sixteen lanes; the lanes of
-// one 16-position block of a B fragment (one k-group) must hit distinct 16-byte slots of
-// the 256-byte bank row. Returns the worst number of lanes sharing a slot over the blocks.
-int block_conflict(int R, const int* box, const int* sigma, const int* hpitch, int box_vol) {
-  int worst = 1;
-  for (int b0 = 0; b0 < box_vol; b0 += 16) {
-    int count[16] = {0};
-    for (int nl = 0; nl < 16; ++nl) {
-      int q = b0 + nl, off = 0;
-      for (int a = R - 1; a >= 0; --a) {
-        const int qa = q % box[a];
-        q /= box[a];
-        off += qa * sigma[a] * hpitch[a];
-      }
-      worst = std::max(worst, ++count[off & 15]);
+// A box of output positions of the implicit GEMM and its halo.
+struct IgemmBoxShape {
+  int b[kFastRank], hext[kFastRank];
+  int64_t pos, hvol, rows, boxes;
+};
+
+// LDS layout of a box's halo: position pitches, positions per plane, and lanes per 16-byte bank
+// slot in a B-fragment read, averaged over the reads (1 = no conflict).
+struct IgemmPitches {
+  int hpitch[kFastRank];
+  int64_t plane_pos = 0;
+  double conflict = 1.0;
+};
+
+// Candidate boxes of at most box_vol positions for outputs of J positions per axis, with
+// `planes` halo planes in LDS: extents that are powers of two or split an axis evenly
+// (ceil(J / n)). Of all those that fill more than half the tile positions, the best few by padded
+// positions, by staged halo, and by an estimate of both (pos_weight: MFMA clocks of a padded
+// position over staging clocks of a halo position), separately for power-of-two boxes, whose LDS
+// reads conflict least, for those of which two workgroups fit a CU, and for long halo rows, which
+// direct staging moves best.
+std::vector<IgemmBoxShape> igemm_boxes(int R, const int* J, const int* sigma, const int* span,
+                                       int box_vol, int planes, double pos_weight) {
+  constexpr size_t kKeep = 6;
+  std::vector<int> ext[kFastRank];
+  int64_t most = 1;
+  for (int a = 0; a < R; ++a) {
+    // Box coordinates are packed in 16-bit fields up to rank 4 and in 8-bit fields above
+    // (extents at most 64 there).
+    const int cap = std::min(box_vol, R <= 4 ? box_vol : 64);
+    for (int l = 1;; l *= 2) {
+      if (l <= cap) ext[a].push_back(l);
+      if (l >= J[a] || l >= cap) break;
     }
+    for (int n = 1; n <= J[a]; ++n) {
+      const int e = (J[a] + n - 1) / n;
+      if (e <= cap) ext[a].push_back(e);
+    }
+    std::sort(ext[a].begin(), ext[a].end());
+    ext[a].erase(std::unique(ext[a].begin(), ext[a].end()), ext[a].end());
+    most = std::min<int64_t>(box_vol, most * ext[a].back());
   }
-  return worst;
+  std::vector<IgemmBoxShape> all[8];
+  IgemmBoxShape box;
+  auto visit = [&](auto&& self, int a, int64_t pos, int64_t hvol, int64_t boxes) -> void {
+    if (a == R) {
+      if (pos * 2 <= most) return;
+      box.pos = pos;
+      box.hvol = hvol;
+      box.boxes = boxes;
+      box.rows = hvol / box.hext[R - 1];
+      bool pow2 = true;
+      for (int i = 0; i < R; ++i) pow2 = pow2 && (box.b[i] & (box.b[i] - 1)) == 0;
+      const bool pair = planes * hvol * 16 * 2 <= 156 * 1024;
+      const bool long_rows = box.hext[R - 1] >= 16;
+      all[(pow2 ? 1 : 0) + (pair ? 2 : 0) + (long_rows ? 4 : 0)].push_back(box);
+      return;
+    }
+    for (int e : ext[a]) {
+      if (pos * e > box_vol) break;
+      const int64_t h = (int64_t)(e - 1) * sigma[a] + span[a] + 1;
+      // Row validity masks hold 64 halo coordinates per axis; coordinates are packed in bytes
+      // in the row table.
+      if (h > (a < R - 1 ? 64 : 255) || planes * hvol * h * 16 > kLdsBudget) break;
+      box.b[a] = e;
+      box.hext[a] = static_cast<int>(h);
+      self(self, a + 1, pos * e, hvol * h, boxes * ((J[a] + e - 1) / e));
+    }
+  };
+  visit(visit, 0, 1, 1, 1);
+  std::vector<IgemmBoxShape> out;
+  for (auto& set : all) {
+    auto keep = [&](auto&& score) {
+      const size_t n = std::min(kKeep, set.size());
+      std::partial_sort(set.begin(), set.begin() + n, set.end(),
+                        [&](const IgemmBoxShape& x, const IgemmBoxShape& y) {
+                          const double u = score(x), v = score(y);
+                          if (u != v) return u < v;
+                          return std::lexicographical_compare(x.b, x.b + R, y.b, y.b + R);
+                        });
+      for (size_t i = 0; i < n; ++i) {
+        bool seen = false;
+        for (const auto& o : out) seen = seen || std::equal(o.b, o.b + R, set[i].b);
+        if (!seen) out.push_back(set[i]);
+      }
+    };
+    keep([&](const IgemmBoxShape& x) { return double(x.boxes) * (pos_weight * box_vol + double(x.hvol)); });
+    keep([&](const IgemmBoxShape& x) { return double(x.boxes) * 1e9 + double(x.hvol); });
+    keep([&](const IgemmBoxShape& x) { return double(x.boxes) * double(x.hvol); });
+  }
+  return out;
+}
+
+// Whether some box of exactly box_vol positions with power-of-two extents has a halo (of one octet)
+// that fits LDS.
+bool pow2_box_fits(int R, const int* J, const int* sigma, const int* span, int box_vol) {
+  int limit[kFastRank];
+  for (int a = 0; a < R; ++a) {
+    limit[a] = 1;
+    while (limit[a] < J[a] && limit[a] < box_vol) limit[a] *= 2;
+  }
+  bool fits = false;
+  for_each_box(R, limit, box_vol, [&](const int* b) {
+    int64_t bytes = 16;
+    for (int a = 0; a < R; ++a) bytes *= (b[a] - 1) * sigma[a] + span[a] + 1;
+    fits = fits || bytes <= kLdsBudget;
+  });
+  return fits;
 }
 
 // Halo pitches: hpitch[R-1] = 1 and hpitch[a] = hpitch[a+1] * padded extent of axis a+1.
 // The two innermost padded extents are searched (0..15 extra positions each), smallest plane
-// first, for the first layout without bank conflicts (else the fewest). Returns the plane
-// size in positions.
-int64_t choose_pitches(int R, const int* box, const int* sigma, const int* hext, int box_vol,
-                       int* hpitch, int* conflict) {
+// first; returned are the smallest plane and every larger one with fewer bank conflicts than
+// those before it, up to one without any. gfx950 serves a
+// wave-wide 16-byte LDS read in four cycles of sixteen lanes: the lanes of one 16-position block
+// of a B fragment (one k-group) should hit distinct 16-byte slots of the 256-byte bank row.
+std::vector<IgemmPitches> choose_pitches(int R, const int* sigma, const IgemmBoxShape& box) {
   struct Candidate {
     int64_t size;
     int p1, p2;
@@ -327,12 +420,12 @@ int64_t choose_pitches(int R, const int* box, const int* sigma, const int* hext,
   auto pitches = [&](int p1, int p2, int* pitch) {
     pitch[R - 1] = 1;
     for (int a = R - 2; a >= 0; --a) {
-      int ext = hext[a + 1];
+      int ext = box.hext[a + 1];
       if (a + 1 == R - 1) ext += p1;
       if (a + 1 == R - 2) ext += p2;
       pitch[a] = pitch[a + 1] * ext;
     }
-    return (int64_t)pitch[0] * hext[0];
+    return (int64_t)pitch[0] * box.hext[0];
   };
   for (int p1 = 0; p1 <= pad_last_max; ++p1)
     for (int p2 = 0; p2 <= pad_mid_max; ++p2) {
@@ -341,21 +434,41 @@ int64_t choose_pitches(int R, const int* box, const int* sigma, const int* hext,
     }
   std::stable_sort(cands.begin(), cands.end(),
                    [](const Candidate& x, const Candidate& y) { return x.size < y.size; });
-  int best_conf = 1 << 30;
-  int64_t best_size = 0;
+  const int n = static_cast<int>(box.pos);
+  std::vector<int> coord((size_t)n * R);
+  for (int q = 0; q < n; ++q)
+    for (int a = R - 1, r = q; a >= 0; --a) {
+      coord[(size_t)q * R + a] = (r % box.b[a]) * sigma[a];
+      r /= box.b[a];
+    }
+  const int blocks = (n + 15) / 16;
+  std::vector<IgemmPitches> out;
+  int best = 1 << 30;
   for (const Candidate& c : cands) {
     int pitch[kFastRank];
     pitches(c.p1, c.p2, pitch);
-    const int conf = block_conflict(R, box, sigma, pitch, box_vol);
-    if (conf < best_conf) {
-      best_conf = conf;
-      best_size = c.size;
-      std::copy(pitch, pitch + R, hpitch);
-      if (conf == 1) break;
+    int total = 0;
+    for (int q0 = 0; q0 < n && total < best; q0 += 16) {
+      unsigned char count[16] = {0};
+      int worst = 1;
+      for (int q = q0; q < n && q < q0 + 16; ++q) {
+        int off = 0;
+        for (int a = 0; a < R; ++a) off += coord[(size_t)q * R + a] * pitch[a];
+        worst = std::max<int>(worst, ++count[off & 15]);
+      }
+      total += worst;
+    }
+    if (total < best) {
+      best = total;
+      IgemmPitches p;
+      p.plane_pos = c.size;
+      p.conflict = double(total) / blocks;
+      std::copy(pitch, pitch + R, p.hpitch);
+      out.push_back(p);
+      if (total == blocks) break;
     }
   }
-  *conflict = best_conf;
-  return best_size;
+  return out;
 }
 
 // Optional launch-plan override for tuning sweeps, read once per process from
@@ -365,7 +478,7 @@ int64_t choose_pitches(int R, const int* box, const int* sigma, const int* hext,
 // Any subset of the keys may be given; the planner then searches only plans matching it and
 // ignores the override when none does.
 struct PlanFilter {
-  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0;
+  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0, ts = -1;
   std::vector<int> box;
   bool active = false;
 };
@@ -403,6 +516,7 @@ PlanFilter parse_filter(const char* text) {
         if (key == "nbuf") f.nbuf = v;
         if (key == "waves") f.waves = v;
         if (key == "parts") f.parts = v;
+        if (key == "ts") f.ts = v;
       }
     }
     pos = end + 1;
@@ -462,7 +576,6 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   // kept int32-addressable.
   const int64_t in_positions = g.groups * g.batch * (mode == 0 ? g.in_vol : g.out_vol);
   auto staged_fits = [&](int64_t channels) { return channels * in_positions <= kI32Safe / 2; };
-  const int out_es = split ? 4 : 2;
   int nphase = 1;
   if (mode == 1) {
     for (int a = 0; a < R; ++a) nphase *= static_cast<int>(g.s[a]);
@@ -508,10 +621,6 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     if (filter.nbuf != 2) staging_options.push_back({true, 1});
   }
   if (filter.ds != 1 && filter.nbuf != 2) staging_options.push_back({false, 1});
-  const double copy_clk =
-      2.0 * 2.0 * double(g.batch) * (mode == 0 ? g.in_vol : g.out_vol) * gemm_cin * g.groups *
-      (2.4e9 / 5.0e12);
-
   // Operand layouts of split precision (IgemmArgs::parts): the parts once each, or the six
   // copies as one K dimension, whose few channels fill whole octets better (3 channels: 24
   // channels along K against 6 products x 8). Channel chunk: 1, 2, 3, 4, 6 or 8 octets dividing
@@ -521,12 +630,8 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   static const int kTiles[][3] = {{1, 2, 1}, {1, 4, 1}, {1, 8, 1}, {2, 2, 1}, {2, 4, 1},
                                   {2, 8, 1}, {4, 2, 1}, {4, 4, 1}, {4, 8, 1}, {1, 4, 2},
                                   {1, 8, 2}, {2, 4, 2}, {2, 8, 2}, {1, 4, 4}, {1, 8, 4}};
-  struct PitchMemo {
-    int hpitch[kFastRank];
-    int conflict;
-    int64_t plane_pos;
-  };
-  std::map<std::vector<int>, PitchMemo> pitch_memo;
+  std::map<std::array<int, 3>, std::vector<IgemmBoxShape>> box_memo;   // by (box_vol, planes, tsplit)
+  std::map<std::vector<int>, std::vector<IgemmPitches>> pitch_memo;    // by box and tsplit
   double best = -1.0;
   for (const auto& staging : staging_options)
   for (const int parts : part_options)
@@ -559,187 +664,198 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
       const int cc = noct * 8;
       if (kcin % cc != 0 || (filter.cc && filter.cc != cc)) continue;
       const int planes = parts * noct;  // octet planes of a chunk
-      const int64_t kc = (ntaps_max * cc + 31) / 32;
       const int64_t nchunk = kcin / cc;
-      // The packing pass indexes weight elements with 32 bits.
-      if (nphase * g.groups * nchunk * kc * parts * mgroups * wm * mb * 512 > kI32Safe) continue;
-      // Box coordinates are packed in 16-bit fields up to rank 4 and in 8-bit fields above
-      // (extents at most 64 there).
-      int limit[kFastRank];
-      for (int a = 0; a < R; ++a) {
-        int l = 1;
-        while (l < J[a] && l < box_vol && (R <= 4 || l < 64)) l *= 2;
-        limit[a] = l;
+      // Split taps (IgemmArgs::tsplit), with the octet-major copy: axes of several taps that
+      // every phase has.
+      int64_t tcount = 1;
+      for (int ts = 0; ts <= (direct ? 0 : std::min(2, R - 1)); ++ts) {
+      int span_ts[kFastRank];
+      for (int a = 0; a < R; ++a) span_ts[a] = a < ts ? 0 : span[a];
+      if (ts > 0) {
+        if (g.k[ts - 1] == 1 || (mode == 1 && g.s[ts - 1] != 1)) break;
+        tcount *= g.k[ts - 1];
       }
-      for_each_box(R, limit, box_vol, [&](const int* b) {
-        if (!filter.box.empty()) {
-          if (static_cast<int>(filter.box.size()) != R) return;
-          for (int a = 0; a < R; ++a)
-            if (filter.box[a] != b[a]) return;
-        }
-        int hext[kFastRank], hpitch[kFastRank];
-        int64_t hvol = 1, rows = 1, boxes = 1, useful = 1;
-        for (int a = 0; a < R; ++a) {
-          hext[a] = (b[a] - 1) * sigma[a] + span[a] + 1;
-          hvol *= hext[a];
-          if (a < R - 1) rows *= hext[a];
-          boxes *= (J[a] + b[a] - 1) / b[a];
-          useful *= J[a];
-        }
-        if (planes * hvol * 16 > kLdsBudget) return;
-        // Direct staging moves whole runs of 8 last-axis elements per task and writes them
-        // row by row; with halo rows shorter than two runs its tasks are mostly partial and
-        // its LDS writes collide (measured about twice as costly as the octet copy there).
-        const double short_rows = direct && hext[R - 1] < 16 ? 2.0 : 1.0;
-        // Row validity masks hold 64 halo coordinates per axis; coordinates are packed in
-        // bytes in the row table.
-        for (int a = 0; a < R; ++a)
-          if ((a < R - 1 && hext[a] > 64) || hext[a] > 255) return;
-        int conflict = 1;
-        // The pitches depend on the box alone (not on the tile or the chunk): memoised.
+      if (filter.ts >= 0 && filter.ts != ts) continue;
+      const int64_t kc = (ntaps_max / tcount * cc + 31) / 32;
+      // The packing pass indexes weight elements with 32 bits.
+      if (nphase * g.groups * tcount * nchunk * kc * parts * mgroups * wm * mb * 512 > kI32Safe) continue;
+      auto found = box_memo.find({box_vol, planes, ts});
+      if (found == box_memo.end()) {
+        // MFMA clocks of a CU per tile position over staging clocks per halo position and octet.
+        const double weight = std::max(1.0, double(mtiles) * ntaps_max * (split ? 6.0 : 1.0) / 4.0);
+        found = box_memo
+                    .emplace(std::array<int, 3>{box_vol, planes, ts},
+                             igemm_boxes(R, J, sigma, span_ts, box_vol, planes, weight))
+                    .first;
+      }
+      for (const IgemmBoxShape& shape : found->second) {
+        const int* b = shape.b;
+        if (!filter.box.empty() &&
+            (static_cast<int>(filter.box.size()) != R || !std::equal(b, b + R, filter.box.begin())))
+          continue;
+        const int* hext = shape.hext;
+        const int64_t hvol = shape.hvol, rows = shape.rows, boxes = shape.boxes;
+        // Epilogue stores: a lane writes 4 consecutive positions at once when they are adjacent
+        // in the output (box rows of whole runs of 4, unit output step on the last axis).
+        const bool unit_step = mode == 0 || g.s[R - 1] == 1;
+        const int run = unit_step && b[R - 1] % 4 == 0 ? 4 : 1;
+        const double short_rows = hext[R - 1] < 16 ? 1.7 : 1.0;
+        auto plane_align = [&](int64_t bytes) { return direct ? align_up(bytes) : (bytes + 1023) / 1024 * 1024; };
+        // Cost of this plan with the halo planes of plane_pos positions and `conflict` lanes per
+        // bank slot; negative when it cannot run.
+        auto evaluate = [&](int64_t plane_pos, double conflict, int64_t* lds_out, int* occ_out) {
+          const int64_t plane_bytes = plane_align(plane_pos * 16);
+          const int tap_row = static_cast<int>((kc + kTapPad + 3) / 4 * 4);
+          const int64_t lds = nbuf * planes * plane_bytes + align_up(rows * (direct ? 8 : 4)) +
+                              align_up(box_vol * 4) + align_up(16 * tap_row);
+          if (rows > (int64_t{1} << 20)) return -1.0;
+          const bool grid_ok = boxes <= (int64_t{1} << 30) && g.groups * mgroups <= 65535 &&
+                               g.batch * nphase <= 65535;
+          if (lds > kLdsBudget || !grid_ok) return -1.0;
+          // Resident workgroups per CU (an eight-wave one fills the register budget of two waves
+          // per SIMD by itself) and waves per SIMD on the CU.
+          const int occ = waves == 8 ? 1 : occupancy(lds, reg_waves);
+          const int simd_waves = occ * waves / 4;
+          // Clocks of a CU's resident workgroups, fitted to 7600 measured (problem, plan) pairs of 60
+          // forward and input-gradient problems over ranks 4-6, all dtypes and every compiled
+          // tile: the plan it picks is within 2.6 % of the best measured on average (the model it
+          // replaces, whose terms were set by hand: 9.5 %). One K32 step: MFMA issue, position
+          // fragments from LDS (one octet per step spreads its four taps over one plane, a third
+          // more; bank conflicts matter little), weight fragments through the vector L1, and the
+          // wave's own load-to-use latency, blended towards the largest.
+          const double lds_factor = std::max(1.0 + 0.145 * (conflict - 1.0), noct == 1 ? 1.34 : 1.0);
+          const double cu_waves = double(occ) * waves;
+          const double mfma = products * mb * nb * 16.0 * 1.03 * simd_waves;
+          const double ldsc = cu_waves * parts * nb * 1024.0 / 180.0 * lds_factor;
+          const double l1 = cu_waves * parts * mb * 1024.0 / 67.0;
+          const double latency = (simd_waves >= 2 ? 93.0 : 105.0) + 41.5 * parts * nb * lds_factor;
+          auto pow4 = [](double v) { return v * v * v * v; };
+          const double step =
+              std::sqrt(std::sqrt(pow4(mfma) + pow4(ldsc) + pow4(l1) + pow4(latency)));
+          const double core = double(tcount * nchunk) * kc * step;
+          // Staging of each chunk's halo: bytes and a round trip; direct staging moves whole runs
+          // of 8 last-axis elements per task, mostly partial ones on halo rows shorter than two
+          // runs. A second resident workgroup hides about half of it.
+          const double halo_bytes = planes * hvol * 16.0;
+          const double stage = double(tcount * nchunk) * (direct ? halo_bytes / 31.0 * short_rows + 2600.0
+                                                                 : halo_bytes / 18.4 + 6000.0);
+          const double exposed = (occ >= 2 ? 0.486 * occ : 1.3) * stage;
+          const double epilogue = double(wm) * mb * 16 * box_vol * 0.25;
+          const double per_round = core + exposed + occ * (epilogue + 10.0 * rows) + 2900.0;
+          // Work in padded boxes beyond the tensor is paid for as well (included via boxes). A
+          // partly filled last round of workgroups costs about two fifths of a whole one at least.
+          const int64_t wgs = boxes * g.groups * mgroups * g.batch * nphase;
+          const double share = double(wgs) / (256.0 * occ);
+          const double rounds = 0.41 * std::ceil(share) + 0.59 * std::max(share, 1.0);
+          *lds_out = lds;
+          *occ_out = occ;
+          // The octet-major copy reads the operand and writes the staged channels (3.5 TB/s).
+          const double copied =
+              direct ? 0.0 : double(in_positions) * (2.0 * staged_cin + (split ? 4.0 : 2.0) * real_cin);
+          return rounds * per_round + copied * (2400.0 / 3.5e6);
+        };
+        int64_t lds = 0;
+        int occ = 1;
+        // The pitches depend on the box alone (not on the tile or the chunk) and only cost more
+        // than dense conflict-free planes: chosen for boxes that could win.
         std::vector<int> key(b, b + R);
+        key.push_back(ts);
         auto hit = pitch_memo.find(key);
         if (hit == pitch_memo.end()) {
-          PitchMemo m;
-          m.plane_pos = choose_pitches(R, b, sigma, hext, box_vol, m.hpitch, &m.conflict);
-          hit = pitch_memo.emplace(key, m).first;
+          const double least = evaluate(hvol, 1.0, &lds, &occ);
+          if (least < 0 || (best >= 0 && least >= best)) continue;
+          hit = pitch_memo.emplace(key, choose_pitches(R, sigma, shape)).first;
         }
-        std::copy(hit->second.hpitch, hit->second.hpitch + R, hpitch);
-        conflict = hit->second.conflict;
-        const int64_t plane_pos = hit->second.plane_pos;
-        const int64_t plane_bytes = align_up(plane_pos * 16);
-        const int tap_row = static_cast<int>((kc + kTapPad + 3) / 4 * 4);
-        const int64_t lds = nbuf * planes * plane_bytes + align_up(rows * 8) +
-                            align_up(box_vol * 4) + align_up(16 * tap_row);
-        if (rows > (int64_t{1} << 20)) return;
-        // Epilogue stores: a lane writes 4 consecutive positions at once when they are
-        // adjacent in the output (box rows of at least 4, unit output step on the last axis).
-        const bool unit_step = mode == 0 || g.s[R - 1] == 1;
-        const int run = unit_step && b[R - 1] >= 4 ? 4 : 1;
-        const bool grid_ok = boxes <= (int64_t{1} << 30) && g.groups * mgroups <= 65535 &&
-                             g.batch * nphase <= 65535;
-        if (lds > kLdsBudget || !grid_ok) return;
-        // Resident workgroups per CU (an eight-wave one fills the register budget of two waves
-        // per SIMD by itself) and waves per SIMD on the CU.
-        const int occ = waves == 8 ? 1 : occupancy(lds, reg_waves);
-        const int simd_waves = occ * waves / 4;
-        // Clocks per K32 step of one workgroup: MFMA issue on each SIMD, B-fragment LDS
-        // reads (4 cycles per wave read when conflict-free; cc == 8 puts four taps of one
-        // plane in a K32 step, which costs a second cycle), A-fragment reads through the
-        // vector L1 (about 64 bytes per clock per CU).
-        const int lds_factor = std::max(conflict, noct == 1 ? 2 : 1);
-        const double mfma = products * mb * nb * 16.0;
-        const double ldsc = parts * 4.0 * nb * 4.0 * lds_factor;
-        const double l1 = parts * 4.0 * mb * 1024.0 / 64.0;
-        const double step = std::max(mfma, std::max(ldsc, l1)) * (waves / 4);
-        // Issue efficiency of the main loop: two waves per SIMD hide each other's load
-        // latency; one wave per SIMD stalls on its own loads (measured on MI355X: the same
-        // input-gradient problem ran 1.7x slower with one wave per SIMD).
-        const double eff = simd_waves >= 2 ? 0.75 : 0.35;
-        const double core = double(nchunk) * kc * step / eff;
-        // Direct staging: only the first chunk's halo is exposed (the rest is loaded during
-        // the previous chunk's MFMAs), each chunk still pays its LDS writes and a barrier.
-        const double stage =
-            short_rows *
-            (nbuf == 2 ? (planes * hvol * 16.0 / 64.0 + 1500.0) + double(nchunk) * (planes * hvol * 16.0 / 256.0 + 300.0)
-                       : double(nchunk) * (planes * hvol * 16.0 / 64.0 + 1500.0));
-        // Epilogue: one store per lane of `run` output values.
-        const double out_bytes = double(wm) * mb * 16 * box_vol * out_es;
-        const double epilogue = out_bytes / (4.0 * out_es * run) + 400.0;
-        // CU time of one round of resident workgroups: their MFMA work shares the SIMDs;
-        // a second resident workgroup hides most of the other's staging, but the two do not
-        // get even issue (measured on MI355X: the younger one finishes its main loop about a
-        // quarter later, alone); a lone workgroup (eight waves, or four at one wave per SIMD)
-        // exposes its staging.
-        const double exposed = occ >= 2 ? 0.25 * stage * occ : stage;
-        const double per_round = occ * core + exposed + occ * epilogue + (occ >= 2 ? 0.1 * core : 0.0);
-        const int64_t wgs = boxes * g.groups * mgroups * g.batch * nphase;
-        const int64_t slots = 256 * occ;
-        const double rounds = double((wgs + slots - 1) / slots);
-        // Work in padded boxes beyond the tensor is paid for as well (included via boxes).
-        const double cost = rounds * per_round + (direct ? 0.0 : copy_clk);
-        (void)useful;
-        if (best >= 0 && cost >= best) return;
-        best = cost;
-        plan.ok = true;
-        plan.mb = mb;
-        plan.nb = nb;
-        plan.waves = waves;
-        plan.occ = occ;
-        plan.cost = cost;
-        plan.conflict = conflict;
-        IgemmArgs& A = plan.args;
-        std::memset(&A, 0, sizeof(A));
-        A.rank = R;
-        A.mode = mode;
-        A.batch = static_cast<int>(g.batch);
-        A.groups = static_cast<int>(g.groups);
-        A.nphase = nphase;
-        A.cin_g = staged_cin;
-        A.cout_g = gemm_cout;
-        A.cin_total = static_cast<int>(A.cin_g * g.groups);
-        A.cout_total = static_cast<int>(gemm_cout * g.groups);
-        A.wk_cin_g = static_cast<int>(g.cin_g);
-        A.wk_cout_g = static_cast<int>(g.cout_g);
-        A.cc = cc;
-        A.noct = noct;
-        A.parts = parts;
-        A.part_octs = A.cin_g / 8 / parts;
-        A.rows = static_cast<int>(rows);
-        A.hlast = hext[R - 1];
-        A.nchunk = static_cast<int>(nchunk);
-        A.kc_max = static_cast<int>(kc);
-        A.wm = wm;
-        A.mtiles = mtiles;
-        A.mgroups = mgroups;
-        A.mtiles_padded = mgroups * wm * mb;
-        A.plane_bytes = static_cast<int>(plane_bytes);
-        A.halo_bytes = static_cast<int>(planes * plane_bytes);
-        int ivol = 1, ovol = 1;
-        for (int a = 0; a < R; ++a) {
-          A.hpitch[a] = hpitch[a];
-          A.hext[a] = hext[a];
-          A.box_shift[a] = 0;
-          while ((1 << A.box_shift[a]) < b[a]) ++A.box_shift[a];
-          A.in_size[a] = static_cast<int>(mode == 0 ? g.in[a] : g.out[a]);
-          A.out_size[a] = static_cast<int>(mode == 0 ? g.out[a] : g.in[a]);
-          ivol *= A.in_size[a];
-          ovol *= A.out_size[a];
-          A.box[a] = b[a];
-          A.nbox[a] = (J[a] + b[a] - 1) / b[a];
-          A.k[a] = static_cast<int>(g.k[a]);
-          A.s[a] = static_cast<int>(g.s[a]);
-          A.p[a] = static_cast<int>(g.p[a]);
-          A.d[a] = static_cast<int>(g.d[a]);
+        for (const IgemmPitches& pitches : hit->second) {
+          const double cost = evaluate(pitches.plane_pos, pitches.conflict, &lds, &occ);
+          if (cost < 0 || (best >= 0 && cost >= best)) continue;
+          const int* hpitch = pitches.hpitch;
+          const int64_t plane_bytes = plane_align(pitches.plane_pos * 16);
+          const int tap_row = static_cast<int>((kc + kTapPad + 3) / 4 * 4);
+          best = cost;
+          plan.ok = true;
+          plan.mb = mb;
+          plan.nb = nb;
+          plan.waves = waves;
+          plan.occ = occ;
+          plan.cost = cost;
+          plan.conflict = pitches.conflict;
+          IgemmArgs& A = plan.args;
+          std::memset(&A, 0, sizeof(A));
+          A.rank = R;
+          A.mode = mode;
+          A.batch = static_cast<int>(g.batch);
+          A.groups = static_cast<int>(g.groups);
+          A.nphase = nphase;
+          A.cin_g = staged_cin;
+          A.cout_g = gemm_cout;
+          A.cin_total = static_cast<int>(A.cin_g * g.groups);
+          A.cout_total = static_cast<int>(gemm_cout * g.groups);
+          A.wk_cin_g = static_cast<int>(g.cin_g);
+          A.wk_cout_g = static_cast<int>(g.cout_g);
+          A.cc = cc;
+          A.noct = noct;
+          A.parts = parts;
+          A.part_octs = A.cin_g / 8 / parts;
+          A.rows = static_cast<int>(rows);
+          A.hlast = hext[R - 1];
+          A.nchunk = static_cast<int>(nchunk);
+          A.tsplit = ts;
+          A.tcount = static_cast<int>(tcount);
+          A.kc_max = static_cast<int>(kc);
+          A.wm = wm;
+          A.mtiles = mtiles;
+          A.mgroups = mgroups;
+          A.mtiles_padded = mgroups * wm * mb;
+          A.plane_bytes = static_cast<int>(plane_bytes);
+          A.halo_bytes = static_cast<int>(planes * plane_bytes);
+          int ivol = 1, ovol = 1;
+          for (int a = 0; a < R; ++a) {
+            A.hpitch[a] = hpitch[a];
+            A.hext[a] = hext[a];
+            A.in_size[a] = static_cast<int>(mode == 0 ? g.in[a] : g.out[a]);
+            A.out_size[a] = static_cast<int>(mode == 0 ? g.out[a] : g.in[a]);
+            ivol *= A.in_size[a];
+            ovol *= A.out_size[a];
+            A.box[a] = b[a];
+            A.nbox[a] = (J[a] + b[a] - 1) / b[a];
+            A.k[a] = static_cast<int>(g.k[a]);
+            A.s[a] = static_cast<int>(g.s[a]);
+            A.p[a] = static_cast<int>(g.p[a]);
+            A.d[a] = static_cast<int>(g.d[a]);
+          }
+          A.in_vol = ivol;
+          A.out_vol = ovol;
+          A.box_pos = static_cast<int>(shape.pos);
+          A.box_vol = box_vol;
+          A.boxes = static_cast<int>(boxes);
+          A.k_vol = static_cast<int>(g.k_vol);
+          A.split_c = split ? real_cin : 0;
+          A.last_size = A.in_size[R - 1];
+          A.packed_ok = run == 4 ? 1 : 0;
+          A.coord_bits = R <= 4 ? 16 : 8;
+          A.tap_row = tap_row;
+          A.div_mt = make_fast_div(static_cast<unsigned>(parts * A.mtiles_padded));
+          A.div_noct = make_fast_div(static_cast<unsigned>(noct));
+          A.div_kc = make_fast_div(static_cast<unsigned>(A.kc_max));
+          A.div_nchunk = make_fast_div(static_cast<unsigned>(A.tcount * A.nchunk));
+          A.div_groups = make_fast_div(static_cast<unsigned>(A.groups));
+          A.direct = direct ? 1 : 0;
+          A.nbuf = nbuf;
+          A.waves = waves;
+          A.nrun = (hext[R - 1] + 14) / 8;  // bound; the exact count is set below
+          plan.lds = static_cast<size_t>(lds);
         }
-        A.in_vol = ivol;
-        A.out_vol = ovol;
-        A.box_vol = box_vol;
-        A.boxes = static_cast<int>(boxes);
-        A.k_vol = static_cast<int>(g.k_vol);
-        A.split_c = split ? real_cin : 0;
-        A.last_size = A.in_size[R - 1];
-        A.packed_ok = run == 4 ? 1 : 0;
-        A.coord_bits = R <= 4 ? 16 : 8;
-        A.tap_row = tap_row;
-        A.div_mt = make_fast_div(static_cast<unsigned>(parts * A.mtiles_padded));
-        A.div_noct = make_fast_div(static_cast<unsigned>(noct));
-        A.div_kc = make_fast_div(static_cast<unsigned>(A.kc_max));
-        A.div_nchunk = make_fast_div(static_cast<unsigned>(A.nchunk));
-        A.div_groups = make_fast_div(static_cast<unsigned>(A.groups));
-        A.direct = direct ? 1 : 0;
-        A.nbuf = nbuf;
-        A.waves = waves;
-        A.nrun = (hext[R - 1] + 14) / 8;  // bound; the exact count is set below
-        plan.lds = static_cast<size_t>(lds);
-      });
+      }
+      }
     }
   }
   if (plan.ok) {
     IgemmArgs& A = plan.args;
     plan.padded = padded;
-    plan.or_direct = padded || wide || (split && !staged_fits(gemm_cin));
-    plan.wpk_elems = (size_t)A.nphase * A.groups * A.nchunk * A.kc_max * A.parts * A.mtiles_padded * 64 * 8;
+    plan.or_direct = padded || wide || (split && !staged_fits(gemm_cin)) ||
+                     !pow2_box_fits(R, J, sigma, span, mtiles >= 4 ? 64 : 128);
+    plan.wpk_elems = (size_t)A.nphase * A.groups * A.tcount * A.nchunk * A.kc_max * A.parts * A.mtiles_padded * 64 * 8;
     plan.staged_elems = (size_t)A.batch * A.in_vol * A.cin_total;
     // Byte offsets into the staged operand are 32-bit (buffer loads, an offset of 0xffffffe0
     // or more reads zero).
@@ -2498,7 +2614,8 @@ std::string check_igemm_tables(const IgemmArgs& A0, size_t lds_bytes, const char
   const int part_bytes = A.halo_bytes / A.parts;  // tap offsets address one part's planes
   const int nbuf = A.direct ? A.nbuf : 1;
   // LDS carve-up: halo buffers, row tables (2 ints per row), box output offsets, taps.
-  const size_t lds_need = (size_t)nbuf * A.halo_bytes + (size_t)A.rows * 8 +
+  const size_t lds_need = (size_t)nbuf * A.halo_bytes +
+                          (size_t)((A.rows + 3) & ~3) * (A.direct ? 8 : 4) +
                           (size_t)((A.box_vol + 3) & ~3) * 4 + (size_t)4 * A.tap_row * 4;
   if (lds_need > lds_bytes) return fail_at("LDS layout exceeds the plan's LDS size");
   const int4* pos = reinterpret_cast<const int4*>(tab.data() + A.tab_pos);
@@ -2511,6 +2628,19 @@ std::string check_igemm_tables(const IgemmArgs& A0, size_t lds_bytes, const char
   for (int r = 0; r < A.rows; ++r)
     if (rows[r].x < 0 || rows[r].x + A.hlast > positions_per_plane)
       return fail_at("halo row past its LDS plane");
+  if (!A.direct) {
+    if (A.plane_bytes % 1024 != 0) return fail_at("plane not whole wave loads");
+    const int* slots = reinterpret_cast<const int*>(tab.data() + A.tab_slots);
+    int64_t live = 0;
+    for (int i = 0; i < positions_per_plane; ++i) {
+      if (slots[i] == -1) continue;
+      const int row = slots[i] >> 8, col = slots[i] & 0xff;
+      if (slots[i] < 0 || row >= A.rows || col >= A.hlast || rows[row].x + col != i)
+        return fail_at("staging slot is not its halo position");
+      ++live;
+    }
+    if (live != (int64_t)A.rows * A.hlast) return fail_at("halo positions without a staging slot");
+  }
   const int* taps = reinterpret_cast<const int*>(tab.data() + A.tab_taps);
   const int* tail = reinterpret_cast<const int*>(tab.data() + A.tab_tail);
   const int* pack = reinterpret_cast<const int*>(tab.data() + A.tab_pack);
@@ -2660,7 +2790,8 @@ int convnd_hip_plan_describe(const convnd_hip_problem* problem, convnd_hip_dtype
              ",\"conflict\":" + std::to_string(p.conflict) +
              ",\"boxes\":" + std::to_string(A.boxes) + ",\"phases\":" +
              std::to_string(A.nphase) + ",\"cc\":" + std::to_string(A.cc) +
-             ",\"parts\":" + std::to_string(A.parts) +
+             ",\"parts\":" + std::to_string(A.parts) + ",\"tsplit\":" + std::to_string(A.tsplit) +
+             ",\"tcount\":" + std::to_string(A.tcount) +
              ",\"nchunk\":" + std::to_string(A.nchunk) + ",\"kc_max\":" +
              std::to_string(A.kc_max) + ",\"mgroups\":" + std::to_string(A.mgroups) +
              ",\"lds\":" + std::to_string(p.lds) + ",\"direct\":" + std::to_string(A.direct) +

@@ -84,14 +84,15 @@ __host__ __device__ inline int axis_e(const IgemmArgs& A, int a, const AxisTaps&
   return A.mode == 0 ? tap * A.d[a] : (t.r + A.p[a] - tap * A.d[a]) / A.s[a];
 }
 
-// Axis information of every axis for one phase; returns the phase's tap count.
+// Axis information of every axis for one phase; returns the phase's tap count (per split tap:
+// the split axes' taps are chunks, not K steps).
 __host__ __device__ inline int phase_axes(const IgemmArgs& A, int phase, AxisTaps* ax) {
   int rr = phase, ntaps = 1;
   for (int a = A.rank - 1; a >= 0; --a) {
     const int radix = A.mode ? A.s[a] : 1;
     ax[a] = axis_taps(A, a, rr % radix);
     rr /= radix;
-    ntaps *= ax[a].ntap;
+    if (a >= A.tsplit) ntaps *= ax[a].ntap;
   }
   return ntaps;
 }
@@ -105,7 +106,7 @@ __host__ __device__ inline int igemm_tap_offset(const IgemmArgs& A, const AxisTa
   const int ci = kk - tau * A.cc;
   if (tau >= ntaps) return -1;
   int rem = tau, t = 0;
-  for (int a = A.rank - 1; a >= 0; --a) {
+  for (int a = A.rank - 1; a >= A.tsplit; --a) {
     const int i = rem % ax[a].ntap;
     rem /= ax[a].ntap;
     t += (axis_e(A, a, ax[a], i) - ax[a].emin) * A.hpitch[a];
@@ -113,7 +114,8 @@ __host__ __device__ inline int igemm_tap_offset(const IgemmArgs& A, const AxisTa
   return t * 16 + (ci >> 3) * A.plane_bytes;
 }
 
-// Flat weight tap index (row-major over the kernel extents) of tap tau of a phase, and the
+// Flat weight tap index (row-major over the kernel extents, split axes at tap 0) of tap tau of a
+// phase, and the
 // channel of k-group (step, lg) within its chunk: the weight-packing map {tflat, channel},
 // tflat = -1 past the phase's last tap.
 __host__ __device__ inline void igemm_pack_entry(const IgemmArgs& A, const AxisTaps* ax,
@@ -127,7 +129,7 @@ __host__ __device__ inline void igemm_pack_entry(const IgemmArgs& A, const AxisT
     return;
   }
   int rem = tau, tf = 0, kstr = 1;
-  for (int a = A.rank - 1; a >= 0; --a) {
+  for (int a = A.rank - 1; a >= A.tsplit; --a) {
     const int idx = rem % ax[a].ntap;
     rem /= ax[a].ntap;
     tf += (ax[a].first + idx * ax[a].step) * kstr;
@@ -148,7 +150,7 @@ __host__ __device__ inline IgemmBox igemm_box_entry(const IgemmArgs& A, int phas
   B.out_origin = 0;
   B.kc = (ntaps * A.cc + 31) / 32;
   B.kf = ntaps * A.cc / 32;
-  B.unused0 = B.unused1 = 0;
+  B.org[0] = B.org[1] = 0;
   B.unused2 = 0;
   bool outside = false, interior = true;
   unsigned long long lo = 0, hi = 0, lim = 0;
@@ -158,7 +160,10 @@ __host__ __device__ inline IgemmBox igemm_box_entry(const IgemmArgs& A, int phas
       const int j0 = (bb % A.nbox[a]) * A.box[a];
       bb /= A.nbox[a];
       outside = outside || j0 >= ax[a].J;
-      const int horg = j0 * ax[a].sigma + ax[a].cshift + ax[a].emin;
+      const int org = j0 * ax[a].sigma + ax[a].cshift;
+      const int horg = org + (a < A.tsplit ? 0 : ax[a].emin);
+      if (a == 0 && A.tsplit > 0) B.org[0] = org;
+      if (a == 1 && A.tsplit > 1) B.org[1] = org;
       int l = ax[a].J - j0;
       interior = interior && l >= A.box[a];
       l = l < 0 ? 0 : (l > A.box[a] ? A.box[a] : l);
@@ -182,7 +187,7 @@ __host__ __device__ inline IgemmBox igemm_box_entry(const IgemmArgs& A, int phas
     }
     if (a >= R - 1) hi |= 1ull << (a * 8);
   }
-  B.flags = (outside ? 1 : 0) | (interior ? 2 : 0);
+  B.flags = (outside ? 1 : 0) | (interior && A.box_pos == A.box_vol ? 2 : 0);
   B.lo = lo;
   B.hi = hi;
   B.lim = lim;
@@ -201,6 +206,8 @@ inline size_t igemm_table_layout(IgemmArgs& A) {
   A.tab_tail = take((size_t)A.nphase * 4 * 4);
   A.tab_pos = take((size_t)A.box_vol * 16);
   A.tab_rows = take((size_t)A.rows * 16);
+  A.tab_slots = take(A.direct ? 0 : (size_t)(A.plane_bytes / 16) * 4);
+  A.tab_split = take((size_t)A.tcount * 8);
   A.tab_box = take((size_t)A.nphase * A.boxes * sizeof(IgemmBox));
   A.tab_pack = take((size_t)A.nphase * A.kc_max * 4 * 8);
   A.tab_bytes = static_cast<int>(at);
@@ -212,9 +219,12 @@ inline size_t igemm_table_layout(IgemmArgs& A) {
 //   [0, nphase*4)            one (phase, lane group): its tap row, tail entry and packing map;
 //   [.., + nphase*boxes)     one IgemmBox record;
 //   [.., + box_vol)          one box-position record;
-//   [.., + rows)             one halo-row record.
+//   [.., + rows)             one halo-row record;
+//   [.., + plane positions)  one LDS slot of a plane (octet-major staging);
+//   [.., + tcount)           one split tap.
 __host__ __device__ inline long igemm_table_entries(const IgemmArgs& A) {
-  return (long)A.nphase * 4 + (long)A.nphase * A.boxes + A.box_vol + A.rows;
+  return (long)A.nphase * 4 + (long)A.nphase * A.boxes + A.box_vol + A.rows +
+         (A.direct ? 0 : A.plane_bytes / 16) + A.tcount;
 }
 
 __host__ __device__ inline void igemm_table_entry(const IgemmArgs& A, unsigned char* tab, long e) {
@@ -248,12 +258,17 @@ __host__ __device__ inline void igemm_table_entry(const IgemmArgs& A, unsigned c
     int qq = q, halo = 0, orel = 0, ostr = 1;
     unsigned long long c = 0;
     for (int a = R - 1; a >= 0; --a) {
-      const int qa = qq & (A.box[a] - 1);
-      qq >>= A.box_shift[a];
+      const int qa = qq % A.box[a];
+      qq /= A.box[a];
       halo += qa * (A.mode == 0 ? A.s[a] : 1) * A.hpitch[a];
       orel += qa * (A.mode == 0 ? 1 : A.s[a]) * ostr;
       ostr *= A.out_size[a];
       c |= static_cast<unsigned long long>(qa) << (a * cb);
+    }
+    if (q >= A.box_pos) {
+      // An idle lane: reads the box's first position, fails every bounds check.
+      halo = orel = 0;
+      c = static_cast<unsigned long long>(A.box[0]);
     }
     int* p = reinterpret_cast<int*>(tab + A.tab_pos) + q * 4;
     p[0] = halo * 16;
@@ -280,6 +295,40 @@ __host__ __device__ inline void igemm_table_entry(const IgemmArgs& A, unsigned c
     p[1] = irel;
     p[2] = static_cast<int>(h & 0xffffffffu);
     p[3] = static_cast<int>(h >> 32);
+    return;
+  }
+  e -= A.rows;
+  const int slots = A.direct ? 0 : A.plane_bytes / 16;
+  if (e < slots) {
+    // Halo coordinates from the outermost pitch inwards; a coordinate past its extent (the
+    // pitches' padding) or a position past the halo is padding.
+    int rem = static_cast<int>(e), row = 0, col = 0;
+    bool live = true;
+    for (int a = 0; a < R; ++a) {
+      const int h = rem / A.hpitch[a];
+      rem -= h * A.hpitch[a];
+      live = live && h < A.hext[a];
+      if (a < R - 1) {
+        row = row * A.hext[a] + h;
+      } else {
+        col = h;
+      }
+    }
+    reinterpret_cast<int*>(tab + A.tab_slots)[e] = live ? (row << 8) | col : -1;
+    return;
+  }
+  e -= slots;
+  if (e < A.tcount) {
+    // Shifts of split tap e (row-major over the split axes): mode 0 t*d, mode 1 (unit stride on
+    // the split axes) p - t*d.
+    int rem = static_cast<int>(e);
+    int* p = reinterpret_cast<int*>(tab + A.tab_split) + e * 2;
+    p[0] = p[1] = 0;
+    for (int a = A.tsplit - 1; a >= 0; --a) {
+      const int t = rem % A.k[a];
+      rem /= A.k[a];
+      p[a] = A.mode == 0 ? t * A.d[a] : A.p[a] - t * A.d[a];
+    }
   }
 }
 

@@ -1,8 +1,8 @@
 // Implicit GEMM (gfx950, 16x16x32 bf16/fp16 MFMA -> fp32) for the forward convolution and
 // for the stride phases of the input gradient.
 //
-//   * A workgroup owns a box of output positions (a power-of-two extent per axis) and a
-//     group of output channels. Its W waves (4 or 8) are arranged WM along the channels and
+//   * A workgroup owns a box of output positions (any extents whose product fits its tiles)
+//     and a group of output channels. Its W waves (4 or 8) are arranged WM along the channels and
 //     W/WM along the positions; each wave accumulates MB x NB fragments of 16 x 16.
 //   * The GEMM input is staged per call into octet-major planes (8 channels = 16 bytes per
 //     position). The region the box reads through every tap (the halo) is copied once per
@@ -38,6 +38,15 @@ namespace {
 // the host code) must match.
 template <int MB, int NB>
 constexpr int igemm_waves = MB * NB >= 32 ? 1 : 2;
+
+// 16 bytes per lane from the buffer straight into LDS: lane l writes dst + 16 l (dst the same
+// for every lane). Outside a lambda: the builtin's address-space cast inside one leaves the
+// kernel's host stub undefined.
+__device__ __forceinline__ void stage_lds16(__amdgpu_buffer_rsrc_t r, unsigned char* dst,
+                                            unsigned voff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      r, (__attribute__((address_space(3))) void*)(dst), 16, voff, 0, 0, 0);
+}
 
 // body(std::integral_constant<int, 0>) .. <N - 1>.
 template <int N, typename F, int I = 0>
@@ -105,12 +114,13 @@ void igemm_kernel(IgemmArgs A) {
   const int KF = box.kf;
 
   // LDS: [octet planes (DS: nbuf sets, alternating per channel chunk) | rows: input offset
-  // (-1 outside the input), LDS position offset | output offset of every box position (read
+  // (-1 outside the input), with DS also LDS position offset | output offset of every box position (read
   // by the epilogue; kept out of registers during the main loop) | the phase's tap offsets,
   // 4 lane groups x tap_row].
   int* rowin = reinterpret_cast<int*>(lds + (DS ? A.nbuf : 1) * A.halo_bytes);
-  int* rowlds = rowin + A.rows;
-  int* posout = rowlds + A.rows;
+  const int rows4 = (A.rows + 3) & ~3;
+  int* rowlds = rowin + rows4;  // (direct staging)
+  int* posout = DS ? rowlds + rows4 : rowlds;
   int* ltaps = posout + ((A.box_vol + 3) & ~3);
   const int4* pt = reinterpret_cast<const int4*>(tab + A.tab_pos);
   for (int q = tid; q < A.box_vol; q += kWT) posout[q] = pt[q].y;
@@ -118,19 +128,40 @@ void igemm_kernel(IgemmArgs A) {
     const int* gt = reinterpret_cast<const int*>(tab + A.tab_taps) + phase * 4 * A.tap_row;
     for (int i = tid; i < 4 * A.tap_row; i += kWT) ltaps[i] = gt[i];
   }
-  {
+  // Input offset of every halo row, for split tap tc: its shift moves the origin and the bounds
+  // along the split axes.
+  auto fill_rows = [&](int tc) {
     const int4* rt = reinterpret_cast<const int4*>(tab + A.tab_rows);
-    const unsigned long long lo = box.lo, hi = box.hi;
-    const int in_base = box.in_base;
+    unsigned long long lo = box.lo, hi = box.hi;
+    int in_base = box.in_base;
+    if (!DS && A.tsplit > 0) {
+      const int2 e = reinterpret_cast<const int2*>(tab + A.tab_split)[tc];
+      const int vol0 = A.in_vol / A.in_size[0];
+      in_base += e.x * vol0;
+      auto bound = [&](int a, int h) {
+        const int lo_a = h >= 0 ? 0 : (-h < A.hext[a] ? -h : A.hext[a]);
+        int hi_a = A.in_size[a] - h;
+        hi_a = hi_a < 0 ? 0 : (hi_a < A.hext[a] ? hi_a : A.hext[a]);
+        const unsigned long long keep = ~(0xffull << (8 * a));
+        lo = (lo & keep) | (static_cast<unsigned long long>(lo_a) << (8 * a));
+        hi = (hi & keep) | (static_cast<unsigned long long>(hi_a) << (8 * a));
+      };
+      bound(0, box.org[0] + e.x);
+      if (A.tsplit > 1) {
+        in_base += e.y * (vol0 / A.in_size[1]);
+        bound(1, box.org[1] + e.y);
+      }
+    }
     for (int r = tid; r < A.rows; r += kWT) {
       const int4 e = rt[r];
       const unsigned long long h =
           static_cast<unsigned>(e.z) | (static_cast<unsigned long long>(static_cast<unsigned>(e.w)) << 32);
       const bool ok = swar_all_ge(h, lo, kGuard8) && swar_all_less(h, hi, kGuard8, kOnes8);
       rowin[r] = ok ? in_base + e.y : -1;
-      rowlds[r] = e.x;
+      if constexpr (DS) rowlds[r] = e.x;
     }
-  }
+  };
+  fill_rows(0);
   // Per lane and position block: LDS byte offset of the lane's B-fragment position.
   int pbase[NB];
 #pragma unroll
@@ -172,12 +203,12 @@ void igemm_kernel(IgemmArgs A) {
   const __amdgpu_buffer_rsrc_t srsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(in), 0, A.in_bytes, 0x00020000);
 
-  // MFMAs of channel chunk ck over the halo planes at hb. `issue` runs once, after the first
+  // MFMAs of chunk ck (split tap, channel chunk) over the halo planes at hb. `issue` runs once, after the first
   // weight fragments and B fragments are requested and before the loop (the next chunk's
   // staging loads go there, behind this chunk's first weight loads in the load queue).
   auto mma_chunk = [&](int ck, const unsigned char* hb, auto&& issue) {
     const frag* wck = wp +
-                      ((size_t)((phase * A.groups + g) * A.nchunk + ck) * A.kc_max) * wstep +
+                      ((size_t)((phase * A.groups + g) * A.tcount * A.nchunk + ck) * A.kc_max) * wstep +
                       (size_t)mt0 * 64 + lane;
     if constexpr (P == 3) {
       // Split-precision fp32, each K32 step from the three parts of both operands: 3 MB weight
@@ -603,115 +634,81 @@ void igemm_kernel(IgemmArgs A) {
       }
     }
   } else {
-    // Staging walk over the octet-major copy: item = ((row * parts + part) * noct + octet) *
-    // hlast + column, 256 items apart per thread; the division happens once and every later item
-    // updates incrementally.
-    const int items = A.rows * P * noct * hlast;
-    const int rp0 = tid / hlast, c0 = tid - (tid / hlast) * hlast;
-    const int drp = kWT / hlast, dc = kWT - drp * hlast;
-    // Halo staging in batches of items per thread: the loads of a batch (branch-free buffer
-    // loads; entries outside the input read zero through an offset past the buffer) are all
-    // in flight before the first LDS store. The first kPreBatch items of the next chunk are
-    // loaded into registers before the current chunk's MFMA loop and stored after it, so
-    // their latency hides behind the MFMAs; the rest go in batches of kStageBatch.
-    constexpr int kPreBatch = 4;
-    constexpr int kStageBatch = 8;
+    // Halo staged straight to LDS from the octet-major copy, every load in flight at once: a
+    // wave's load writes 64 consecutive LDS positions of a plane (1 KB), each lane reading the
+    // position's source (slot table: halo row and column; zero past the staged tensor for
+    // padding and for positions outside the input), the same positions of all planes in turn.
+    // With split taps the halo is restaged per tap of the outer axes: at rank 6 (3^6 taps) it is
+    // what lets a box of 256 positions, or all three parts of fp32, fit LDS. [1,8,8^6] -> 16
+    // channels, forward / input gradient: fp32 696 / 1417 -> 266 / 503 us, bf16 154 / 274 ->
+    // 105 / 131 us.
+    const int plane_pos = A.plane_bytes >> 4;  // a multiple of 64
     // Octet planes of this image and group: [cin_total/8][in_vol][8], addressed in bytes from
     // the staged tensor's base.
     const unsigned img_base =
         static_cast<unsigned>(((size_t)n * (A.cin_total >> 3) + (size_t)(g * (A.cin_g >> 3))) *
                               A.in_vol * 16);
-    // Row, octet and part of walk index rp = (row * parts + part) * noct + octet.
-    auto split_item = [&](int rp, int& r, int& o, int& part) {
-      const int q = fast_div(rp, A.div_noct);
-      o = rp - q * noct;
-      r = P == 3 ? static_cast<int>(static_cast<unsigned>(q) / 3u) : q;
-      part = P == 3 ? q - r * 3 : 0;
-    };
-    u32x4 pre[kPreBatch];
-    auto stage_load = [&](int ck, int it0, int rp, int c, u32x4* v, auto nbatch) {
-      const unsigned cbase = img_base + static_cast<unsigned>(ck * A.noct) * A.in_vol * 16u;
-#pragma unroll
-      for (int u = 0; u < decltype(nbatch)::value; ++u) {
-        const int it = it0 + u * kWT;
-        int r, o, part;
-        split_item(rp, r, o, part);
-        const int ro = it < items ? rowin[r < A.rows ? r : 0] : -1;
-        const int cl = corg + c;
+    const int* slots = reinterpret_cast<const int*>(tab + A.tab_slots);
+    const unsigned plane_step = static_cast<unsigned>(A.in_vol) * 16u;
+    auto stage = [&](int ck) {
+      const unsigned cbase = img_base + static_cast<unsigned>(ck * noct) * plane_step;
+      for (int i0 = __builtin_amdgcn_readfirstlane(wave) * 64; i0 < plane_pos; i0 += kWT) {
+        const int e = slots[i0 + lane];
+        const int ro = e >= 0 ? rowin[e >> 8] : -1;
+        const int cl = corg + (e & 0xff);
         const bool ok = ro >= 0 && cl >= 0 && cl < last_size;
-        const unsigned plane = static_cast<unsigned>(part * A.part_octs + o);
-        const unsigned off =
-            ok ? cbase + (plane * A.in_vol + static_cast<unsigned>(ro + cl)) * 16u : kPast;
-        v[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(srsrc, off, 0, 0));
-        c += dc;
-        rp += drp;
-        if (c >= hlast) {
-          c -= hlast;
-          ++rp;
+        unsigned off = ok ? cbase + static_cast<unsigned>(ro + cl) * 16u : kPast;
+        unsigned char* dst = lds + i0 * 16;
+#pragma unroll 1
+        for (int p = 0; p < P; ++p) {
+          unsigned po = off;
+#pragma unroll 1
+          for (int o = 0; o < noct; ++o) {
+            stage_lds16(srsrc, dst, po);
+            dst += A.plane_bytes;
+            if (ok) po += plane_step;
+          }
+          if (ok) off += static_cast<unsigned>(A.part_octs) * plane_step;
         }
       }
     };
-    auto stage_store = [&](int it0, int rp, int c, const u32x4* v, auto nbatch) {
-#pragma unroll
-      for (int u = 0; u < decltype(nbatch)::value; ++u) {
-        const int it = it0 + u * kWT;
-        if (it < items) {
-          int r, o, part;
-          split_item(rp, r, o, part);
-          *reinterpret_cast<u32x4*>(lds + (part * noct + o) * A.plane_bytes + (rowlds[r] + c) * 16) = v[u];
-        }
-        c += dc;
-        rp += drp;
-        if (c >= hlast) {
-          c -= hlast;
-          ++rp;
-        }
+    for (int tc = 0; tc < A.tcount; ++tc) {
+      if (tc > 0) {
+        // Every wave is past the staging that read the rows (the last chunk's barrier).
+        fill_rows(tc);
       }
-    };
-    // Position of item it0 + n * kWT in the walk, from the position of it0.
-    auto advance = [&](int& rp, int& c, auto nbatch) {
-#pragma unroll
-      for (int u = 0; u < decltype(nbatch)::value; ++u) {
-        c += dc;
-        rp += drp;
-        if (c >= hlast) {
-          c -= hlast;
-          ++rp;
-        }
+      for (int ck = 0; ck < A.nchunk; ++ck) {
+        // Row table written, and every wave done reading the chunk before.
+        __syncthreads();
+        stage(ck);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads have landed in LDS
+        __syncthreads();
+        mma_chunk(tc * A.nchunk + ck, lds, []() {});
       }
-    };
-    using PreN = std::integral_constant<int, kPreBatch>;
-    using StageN = std::integral_constant<int, kStageBatch>;
-    __syncthreads();  // row tables in LDS
-    stage_load(0, tid, rp0, c0, pre, PreN{});
-    for (int ck = 0; ck < A.nchunk; ++ck) {
-      {
-        // Chunk ck: the first kPreBatch items are in `pre`; the rest is loaded and stored here.
-        stage_store(tid, rp0, c0, pre, PreN{});
-        int rp = rp0, c = c0;
-        advance(rp, c, PreN{});
-        for (int it0 = tid + kPreBatch * kWT; it0 < items; it0 += kStageBatch * kWT) {
-          u32x4 v[kStageBatch];
-          stage_load(ck, it0, rp, c, v, StageN{});
-          stage_store(it0, rp, c, v, StageN{});
-          advance(rp, c, StageN{});
-        }
-      }
-      __syncthreads();
-      if (ck + 1 < A.nchunk) stage_load(ck + 1, tid, rp0, c0, pre, PreN{});
-      mma_chunk(ck, lds, []() {});
-      if (ck + 1 < A.nchunk) __syncthreads();  // every wave is done reading this chunk's halo
     }
   }
 
   // Epilogue: straight from the accumulators. A lane's four values are box positions
-  // 4*lg .. 4*lg+3 of its position block. In a box inside the output whose rows have at
-  // least 4 positions on a unit output step they are adjacent: one 8-byte store for 16-bit
-  // O, 16 bytes for float. Otherwise every position has its own offset and bounds check.
+  // 4*lg .. 4*lg+3 of its position block. In a box inside the output whose rows have whole runs
+  // of 4 positions on a unit output step they are adjacent: one 8-byte store for 16-bit
+  // O, 16 bytes for float. Otherwise every position has its own offset and bounds check, and a
+  // lane whose four positions are all inside and adjacent still stores them at once.
   // The activation is a compile-time constant of each epilogue copy, dispatched once: every
   // copy's code is contiguous (a launch starts on a cold instruction cache, and per-element
   // branches over the activations' code would spread the executed instructions over many
   // more cache lines).
+  auto store4 = [](O* dst, const O* v) {
+    if constexpr (sizeof(O) == 2) {
+      uint2 w;
+      w.x = __builtin_bit_cast(unsigned short, v[0]) |
+            ((unsigned)__builtin_bit_cast(unsigned short, v[1]) << 16);
+      w.y = __builtin_bit_cast(unsigned short, v[2]) |
+            ((unsigned)__builtin_bit_cast(unsigned short, v[3]) << 16);
+      *reinterpret_cast<uint2*>(dst) = w;
+    } else {
+      *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+    }
+  };
   auto epilogue = [&](auto act_c) {
     constexpr int kAct = decltype(act_c)::value;
     O* out = static_cast<O*>(A.out);
@@ -769,17 +766,7 @@ void igemm_kernel(IgemmArgs A) {
           O v[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) v[i] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
-          O* dst = orow + posout[(wn * NB + nb) * 16 + 4 * lg];
-          if constexpr (sizeof(O) == 2) {
-            uint2 w;
-            w.x = __builtin_bit_cast(unsigned short, v[0]) |
-                  ((unsigned)__builtin_bit_cast(unsigned short, v[1]) << 16);
-            w.y = __builtin_bit_cast(unsigned short, v[2]) |
-                  ((unsigned)__builtin_bit_cast(unsigned short, v[3]) << 16);
-            *reinterpret_cast<uint2*>(dst) = w;
-          } else {
-            *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-          }
+          store4(orow + posout[(wn * NB + nb) * 16 + 4 * lg], v);
         }
       }
     } else {
@@ -804,10 +791,18 @@ void igemm_kernel(IgemmArgs A) {
         O* orow = obox + (chan0 + m) * A.out_vol;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
+          O v[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (off[nb][i] >= 0)
-              orow[off[nb][i]] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
+            v[i] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
+          const int o0 = off[nb][0];
+          if (o0 >= 0 && off[nb][1] == o0 + 1 && off[nb][2] == o0 + 2 && off[nb][3] == o0 + 3) {
+            store4(orow + o0, v);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (off[nb][i] >= 0) orow[off[nb][i]] = v[i];
+          }
         }
       }
     }

@@ -116,18 +116,25 @@ struct IgemmArgs {
   int cin_total, cout_total;
   int wk_cin_g, wk_cout_g;    // channels per group of the original weight tensor
   int cc, noct;               // channels and octets per LDS chunk
-  int nchunk, kc_max;         // chunks, K32 steps per chunk (widest phase)
+  int nchunk, kc_max;         // channel chunks, K32 steps per chunk (widest phase)
+  // Split taps (octet-major staging): each of the tcount taps of the outermost tsplit axes (0, 1
+  // or 2) is a chunk of its own, so that the halo in LDS does not extend along those axes. K runs
+  // over (split tap, channel chunk, remaining tap, channel).
+  int tsplit, tcount;
   int wm;                     // waves along M (output channels); 4 / wm along positions
   int mtiles, mgroups, mtiles_padded;
-  int plane_bytes;            // LDS bytes of one octet plane (multiple of 256)
+  int plane_bytes;            // LDS bytes of one octet plane (multiple of 256; of 1024, one load
+                              // of a wave straight to LDS, with octet-major staging)
   int halo_bytes;             // parts * noct * plane_bytes
   int rows, hlast;            // halo rows (all axes but the last) and last-axis extent
   int hext[kFastRank];        // halo extent per axis (<= 64 on all axes but the last)
   int hpitch[kFastRank];      // halo position pitch per axis (hpitch[rank-1] == 1)
   int in_size[kFastRank], out_size[kFastRank];
   int in_vol, out_vol;
-  int box[kFastRank], box_shift[kFastRank], nbox[kFastRank];
-  int box_vol, boxes;
+  // Box of output positions: any extents, box_pos = their product, at most the box_vol positions
+  // of the workgroup's tiles (the rest are idle lanes: halo offset 0, never stored).
+  int box[kFastRank], nbox[kFastRank];
+  int box_pos, box_vol, boxes;
   int k[kFastRank], s[kFastRank], p[kFastRank], d[kFastRank];
   int k_vol;
   int split_c;     // split-precision fp32: real channels per group in the GEMM-input role
@@ -146,13 +153,17 @@ struct IgemmArgs {
   //   tail  int  [nphase][4]: the same for the partial last step, -1 past the last tap;
   //   pos   int4 [box_vol]: {halo byte offset, output offset, box coordinates (2 x 32 bit)};
   //   rows  int4 [rows]: {halo position offset, input position offset, halo coordinates};
+  //   slots int  [plane_bytes / 16] (octet-major staging): halo row << 8 | column of every LDS
+  //              position of a plane, -1 for padding;
+  //   split int2 [tcount]: input shifts of a split tap along axes 0 and 1;
   //   boxes IgemmBox [nphase][boxes];
   //   pack  int2 [nphase][kc_max][4 lane groups]: weight tap index (-1 past the last tap)
   //              and channel within the chunk of each k-group.
   // Coordinates are packed one field per axis (axis a in field a) so that one subtraction
   // compares every axis against packed bounds (see swar_all_less / swar_all_ge).
   const void* tables;
-  int tab_taps, tab_tail, tab_pos, tab_rows, tab_box, tab_pack;  // byte offsets in `tables`
+  int tab_taps, tab_tail, tab_pos, tab_rows, tab_slots, tab_split, tab_box, tab_pack;  // byte
+                                                                           // offsets in `tables`
   int tab_bytes;
   int tap_row;       // entries per (phase, lane group): kc_max + kTapPad, rounded to 4
   int last_size;     // input extent of the last axis
@@ -182,9 +193,10 @@ struct IgemmBox {
   int in_base;     // input position offset of the halo origin over all axes but the last
   int corg;        // halo origin on the last axis (may be negative)
   int out_origin;  // output offset of the box origin
-  int flags;       // bit 0: the box lies past the phase's output; bit 1: fully inside it
+  int flags;       // bit 0: the box lies past the phase's output; bit 1: fully inside it and
+                   // box_pos == box_vol
   int kc, kf;      // K32 steps of the phase: all, and whole ones
-  int unused0, unused1;
+  int org[2];      // halo origin along the split axes, without the tap's shift
   unsigned long long lo, hi;  // halo rows inside the input: lo <= h < hi per axis (8 bits)
   unsigned long long lim;     // box positions inside the output: q < lim per axis
   unsigned long long unused2;

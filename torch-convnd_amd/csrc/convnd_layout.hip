@@ -444,7 +444,7 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     P.ig = a;
     P.w = p.w;
     P.wpk = p.wpk;
-    P.units = (int64_t)a.nphase * a.groups * a.nchunk * a.kc_max * a.parts * a.mtiles_padded * 64;
+    P.units = (int64_t)a.nphase * a.groups * a.tcount * a.nchunk * a.kc_max * a.parts * a.mtiles_padded * 64;
     if (P.units * 8 > 0x7fffffff) return hipErrorInvalidValue;  // 32-bit element indices
     const int64_t blocks = (P.units * 8 + kThreads - 1) / kThreads;
     P.b_blocks = static_cast<int>(blocks < 8192 ? blocks : 8192);

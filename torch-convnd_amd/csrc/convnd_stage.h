@@ -13,7 +13,7 @@ namespace stage {
 
 // ---- weight packing --------------------------------------------------------------------
 
-// Packed weights: unit u = ((((phase*G + g)*nchunk + chunk)*kc_max + kc)*parts*mtiles_padded
+// Packed weights: unit u = ((((phase*G + g)*tcount*nchunk + chunk)*kc_max + kc)*parts*mtiles_padded
 // + part*mtiles_padded + mt)*64 + lane holds the 8 A-fragment elements W'[m][k], m = mt*16 + lane%16,
 // k = kc*32 + (lane/16)*8 + i (i < 8), zero where m or k is padding.
 // S = float (split precision): GEMM channel ci is part split_other_part(ci / split_c) of
@@ -45,11 +45,17 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
     const int kc = r - q * A.kc_max;
     r = q;
     q = fast_div(r, A.div_nchunk);
-    const int ck = r - q * A.nchunk;
+    int ck = r - q * (A.tcount * A.nchunk);
     r = q;
     const int phase = fast_div(r, A.div_groups);
     const int g = r - phase * A.groups;
     const int m = mt * 16 + (lane & 15);
+    int tc = 0;  // split tap of the chunk
+    while (ck >= A.nchunk) {
+      ck -= A.nchunk;
+      ++tc;
+    }
+    const int tvol = A.tcount > 1 ? A.k_vol / A.tcount : A.k_vol;  // taps per split tap
     // Tap and channel of the lane's k-group: for the forward convolution (one phase, every
     // tap in row-major order) k-group kk / 8 of the chunk is tap kk / cc, channel kk % cc;
     // the input gradient's phases read the plan's map.
@@ -58,12 +64,13 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
       const int ko = kc * 4 + (lane >> 4);  // k-group: (tap, octet of the chunk)
       tflat = fast_div(ko, A.div_noct);
       chan = (ko - tflat * A.noct) * 8;
-      if (tflat >= A.k_vol) tflat = -1;
+      if (tflat >= tvol) tflat = -1;
     } else {
       const int* pe = pmap + ((phase * A.kc_max + kc) * 4 + (lane >> 4)) * 2;
       tflat = pe[0];
       chan = pe[1];
     }
+    if (tflat >= 0) tflat += tc * tvol;
     int ci = ck * A.cc + chan + i;
     bool live = m < A.cout_g && tflat >= 0;
     if constexpr (sizeof(S) == 4) {
