@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstdlib>
 #include <cstdint>
 #include <cstring>
@@ -478,7 +479,7 @@ std::vector<IgemmPitches> choose_pitches(int R, const int* sigma, const IgemmBox
 // Any subset of the keys may be given; the planner then searches only plans matching it and
 // ignores the override when none does.
 struct PlanFilter {
-  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0, ts = -1;
+  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0, ts = -1, parity = -1;
   std::vector<int> box;
   bool active = false;
 };
@@ -517,6 +518,7 @@ PlanFilter parse_filter(const char* text) {
         if (key == "waves") f.waves = v;
         if (key == "parts") f.parts = v;
         if (key == "ts") f.ts = v;
+        if (key == "parity") f.parity = v;
       }
     }
     pos = end + 1;
@@ -940,6 +942,7 @@ struct WgradPlan {
   // caller's input directly (no staged copy); `args` then only describes grad_output for
   // the padded copy (rank, extents, batch, channels).
   bool cm = false;
+  bool or_direct = false;  // as IgemmPlan::or_direct
   WgradCmArgs cm_args{};
   PlanarPadArgs ppad{};  // the zero-padded channels-first input it reads (staged_elems)
 };
@@ -959,10 +962,24 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
   const int64_t batch = split ? g.batch * kSplit : g.batch;
   const int64_t sbatch = split ? g.batch * 3 : g.batch;
   const int R = g.rank;
-  if (g.s[R - 1] != 1) return false;
+  const int ls = static_cast<int>(g.s[R - 1]);
+  if (ls > kMaxLastStride) return false;
   const int cin_g = static_cast<int>(g.cin_g), cout_g = static_cast<int>(g.cout_g);
   const int k_vol = static_cast<int>(g.k_vol);
   const int kl = static_cast<int>(g.k[R - 1]), dl = static_cast<int>(g.d[R - 1]);
+  // Copies of the padded input (WgradCmArgs::copy_id), with shifted ones or without.
+  auto copies_of = [&](bool parity, signed char* id, signed char* phase, signed char* shift) {
+    std::fill(id, id + 2 * kMaxLastStride, static_cast<signed char>(-1));
+    int n = 0;
+    for (int t = 0; t < kl; ++t) {
+      const int r = t * dl % ls, odd = parity ? t * dl / ls & 1 : 0;
+      if (id[2 * r + odd] >= 0) continue;
+      phase[n] = static_cast<signed char>(r);
+      shift[n] = static_cast<signed char>(odd);
+      id[2 * r + odd] = static_cast<signed char>(n++);
+    }
+    return n;
+  };
   const int mtiles = (cout_g + 15) / 16;
   const int mb = mtiles >= 4 ? 4 : (mtiles >= 2 ? 2 : 1);
   const int mgroups = (mtiles + mb - 1) / mb;
@@ -1005,7 +1022,7 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
           rows_h *= h;
           e = (int64_t)(nbox[a] - 1) * b[a] * g.s[a] + h;
         } else {
-          e = ((int64_t)nbox[a] * b[a] + (kl - 1) * dl + 7) / 8 * 8;
+          e = ((int64_t)nbox[a] * b[a] + (kl - 1) * dl / ls + 7) / 8 * 8;
         }
         if (e > kI32Safe) return;
         pe[a] = static_cast<int>(e);
@@ -1013,7 +1030,8 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         if (pvol > kI32Safe) return;
       }
       // The padded copy must stay int32-addressable and not dwarf the input.
-      if (pvol * sbatch * g.channels * 2 > kI32Safe || pvol > 8 * g.in_vol + (1 << 20)) return;
+      const int64_t copy_elems = pvol * sbatch * g.channels;
+      if (copy_elems * 2 > kI32Safe || pvol > 8 * g.in_vol + (1 << 20)) return;
       const int bl8 = bl / 8;
       const int nrho = kl * bl8;
       const int runpitch = nrho * 16;
@@ -1076,22 +1094,41 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         const int64_t lds = lds_items + ipc * 8;
         if (lds > dyn_budget) continue;
         if (npc * per_chunk_wgs > INT32_MAX) continue;
+        for (const bool parity : {false, true})
         for (const int waves : {8, 4}) {
         if (!wgrad_cm_supported(mb, nt, waves)) continue;
         if (filter.waves && filter.waves != waves) continue;
-        // Per item, clocks of one CU: MFMA issue of one wave (MB x NT per K32 step) and the
-        // LDS fragment reads of four waves (128 B/clock) against the item's loads straight
-        // into LDS (~64 B/clock/CU of L2 traffic), which overlap, plus barriers.
-        // Two waves per SIMD (eight-wave workgroups) issue MFMAs more evenly.
-        const double mfma = double(ksteps) * mb * nt * 16.0 / (waves == 8 ? 0.9 : 0.8);
-        const double ldsr = double(ksteps) * (mb + nt) * 32.0;
-        const double stage = (double(xi) * 1024 + double(dyt_bytes)) / 64.0;
-        const double per_item = std::max(std::max(mfma, ldsr), stage) + 800.0;
-        const double per_wg = double(ipc) * per_item + 4000.0;
+        if (filter.parity >= 0 && filter.parity != (parity ? 1 : 0)) continue;
+        signed char copy_id[2 * kMaxLastStride], phase[kMaxCopies] = {}, shift[kMaxCopies] = {};
+        const int ncopy = copies_of(parity, copy_id, phase, shift);
+        if (ncopy * copy_elems * 2 > kI32Safe) continue;
+        // Taps whose runs start at odd elements: one lane per clock (see WgradCmArgs::ls).
+        int odd = 0;
+        for (int t = 0; t < kl && !parity; ++t) odd += t * dl / ls & 1;
+        const double odd_share = double(odd) / kl;
+        // Per item, clocks of one CU: MFMA issue (two waves per SIMD issue more evenly), LDS
+        // fragment reads of four waves, the lanes of the item's loads straight into LDS (odd
+        // elements at a third of the rate) and their bytes, partly overlapping. Fitted to 1200
+        // measured (problem, plan) pairs of 41 layers over ranks 4-6 and all dtypes: plans within
+        // 5 % of the best measured on average, 7 % before. Shifted copies cost their write in
+        // the prologue (2 TB/s): they pay where the loads bound the item (rank 6, 8 -> 16
+        // channels: kernel 157 -> 122 us, fp32 836 -> 665) and not where the MFMAs do (32 -> 64
+        // channels: 57.5 -> 55.8 us for 13 us of copy).
+        const double mfma = double(ksteps) * mb * nt * 16.0 * (waves == 8 ? 1.28 : 1.7);
+        const double ldsr = double(ksteps) * (mb + nt) * 4096.0 / 260.0;
+        const double lanes = double(xi) * 64.0 * ((1.0 - odd_share) / 2.35 + odd_share / 0.816) +
+                             double(dyt_bytes) / 16.0 / 2.35;
+        const double bytes = (double(xi) * 1024.0 + double(dyt_bytes)) / 41.0;
+        const double per_item = std::pow(std::pow(mfma, 1.6) + std::pow(ldsr, 1.6) +
+                                             std::pow(lanes, 1.6) + std::pow(bytes, 1.6),
+                                         1.0 / 1.6) +
+                                590.0;
+        const double per_wg = double(ipc) * per_item + 27000.0;
         const int64_t wgs = npc * per_chunk_wgs;
         const double rounds = double((wgs + 255) / 256);
-        const double partial_clk = double(wgs) * 4 * mb * nt * 64 * 16 * 2 / 3000.0;
-        const double cost = rounds * per_wg + partial_clk;
+        const double partial_clk = double(wgs) * 4 * mb * nt * 64 * 16 * 2 / 1470.0;
+        const double copy_clk = double(ncopy) * copy_elems * 2.0 * (2400.0 / 2.0e6);
+        const double cost = rounds * per_wg + partial_clk + copy_clk;
         if (best >= 0 && cost >= best) continue;
         best = cost;
         plan = WgradPlan{};
@@ -1102,7 +1139,7 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         plan.lds = static_cast<size_t>(lds);
         // Split precision always reads grad_output's padded part copy.
         plan.exact = dvol == g.out_vol && !split;
-        plan.staged_elems = (size_t)sbatch * g.channels * pvol;
+        plan.staged_elems = (size_t)ncopy * copy_elems;
         WgradCmArgs& C = plan.cm_args;
         std::memset(&C, 0, sizeof(C));
         C.x_bytes = static_cast<unsigned>(plan.staged_elems * 2);
@@ -1125,6 +1162,11 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         C.runpitch = runpitch;
         C.chpitch = static_cast<int>(chpitch);
         C.dl = dl;
+        C.ls = ls;
+        C.ncopy = ncopy;
+        C.copy_elems = static_cast<int>(copy_elems);
+        C.parity = parity ? 1 : 0;
+        std::copy(copy_id, copy_id + 2 * kMaxLastStride, C.copy_id);
         C.dyt_bytes = static_cast<int>(dyt_bytes);
         C.xi = static_cast<int>(xi);
         C.di = static_cast<int>(dyt_bytes / 1024);
@@ -1143,6 +1185,10 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         std::memset(&P, 0, sizeof(P));
         P.rank = R;
         P.channels = static_cast<int>(g.channels);
+        P.copies = ncopy;
+        P.last_stride = ls;
+        std::copy(phase, phase + ncopy, P.phase);
+        std::copy(shift, shift + ncopy, P.shift);
         P.in_vol = static_cast<int>(g.in_vol);
         P.pvol = static_cast<int>(pvol);
         P.src_bytes = static_cast<unsigned>(g.batch * g.channels * g.in_vol * element_size(dt));
@@ -1197,13 +1243,25 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
 
 WgradPlan plan_wgrad_octets(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter);
 
-// The channel-major kernel where it applies (CONVND_HIP_WGRAD_PLAN=cm=0 forces the
-// octet-major one), else the octet-major kernel; an override that no plan of this problem
+// The channel-major kernel where it applies (CONVND_HIP_WGRAD_PLAN=cm=0 forces the octet-major
+// one), but the octet-major one first for a strided last axis, else the octet-major kernel; an override that no plan of this problem
 // matches is ignored.
 WgradPlan plan_wgrad(const Geom& g, convnd_hip_dtype dt) {
   auto search = [&](const PlanFilter& filter) {
+    // A strided last axis: the octet-major kernel reads its one padded copy as it is, while the
+    // channel-major one needs a copy per stride phase, gathered element by element (32 -> 64
+    // channels, 20^4, stride 2: 85 us against 108 with their copies); it takes the halos that
+    // only fit LDS one channel at a time (16 -> 32 channels, 11^5, stride 2: 0.04 ms; 4.0 ms on
+    // the direct kernel).
+    if (g.s[g.rank - 1] != 1 && filter.cm != 1) {
+      const WgradPlan oct = plan_wgrad_octets(g, dt, filter);
+      if (oct.ok) return oct;
+    }
     WgradPlan cm;
-    if (filter.cm != 0 && plan_wgrad_cm(g, dt, filter, &cm)) return cm;
+    if (filter.cm != 0 && plan_wgrad_cm(g, dt, filter, &cm)) {
+      cm.or_direct = g.s[g.rank - 1] != 1;
+      return cm;
+    }
     return plan_wgrad_octets(g, dt, filter);
   };
   const PlanFilter& filter = plan_filter(2);
@@ -2085,8 +2143,15 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   // input gradient runs on MFMA (its octet-major grad_output copy, or, with direct staging, a
   // sums part of the same launch); otherwise grad_output is reduced on its own.
   const bool tiny_bias = gb && gw && b.tdw.ok;
-  const bool cm_bias = gb && gw && b.wg.ok && b.wg.cm && is_half(dtype);
   TablesRef dx_tables, dw_tables;  // held until the kernels that read them are enqueued
+  bool mfma_dw = gw && b.wg.ok;
+  if (mfma_dw) {
+    dw_tables = b.wg.cm ? wgrad_cm_device_tables(plan_key(g, dtype, 66), b.wg.cm_args, stream)
+                        : wgrad_device_tables(plan_key(g, dtype, 65), b.wg.args, stream);
+    if (dw_tables == nullptr && !b.wg.or_direct) return CONVND_HIP_LAUNCH_FAILED;
+    mfma_dw = dw_tables != nullptr;
+  }
+  const bool cm_bias = gb && mfma_dw && b.wg.cm && is_half(dtype);
   bool mfma_dx = gi && b.dg.ok;
   if (mfma_dx) {
     dx_tables = igemm_device_tables(plan_key(g, dtype, 64), b.dg.args, stream);
@@ -2104,7 +2169,6 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   // Staging passes of both MFMA gradients (grad_output channels-last copy with the bias
   // sums, input-gradient weight packing, octet-major input, padded grad_output) in one
   // launch.
-  const bool mfma_dw = gw && b.wg.ok;
   IgemmArgs DA{};
   WgradArgs WA{};
   WgradCmArgs CA{};
@@ -2144,8 +2208,6 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   if (mfma_dw && b.wg.cm) {
     WA = b.wg.args;
     CA = b.wg.cm_args;
-    dw_tables = wgrad_cm_device_tables(plan_key(g, dtype, 66), CA, stream);
-    if (dw_tables == nullptr) return CONVND_HIP_LAUNCH_FAILED;
     CA.tables = dw_tables->dev;
     CA.x = ws + b.off_x_stage;
     CA.dy = grad_output;
@@ -2175,8 +2237,6 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
     }
   } else if (mfma_dw) {
     WA = b.wg.args;
-    dw_tables = wgrad_device_tables(plan_key(g, dtype, 65), WA, stream);
-    if (dw_tables == nullptr) return CONVND_HIP_LAUNCH_FAILED;
     WA.tables = dw_tables->dev;
     WA.x = ws + b.off_x_stage;
     WA.dy = grad_output;
@@ -2713,9 +2773,18 @@ std::string check_wgrad_cm_tables(const WgradCmArgs& C0) {
     if (col[i] < 0 || col[i] + max_run + 16 > C.xi * 1024)
       return what + ": column read past the staged input runs";
   }
+  // Every run of a copy's row stays inside the row, wherever the box lies on the last axis.
+  for (int tl = 0; tl < C.kl; ++tl) {
+    int copy, off;
+    wgrad_cm_tap_copy(C, tl, &copy, &off);
+    if (copy < 0 || copy >= C.ncopy || off < 0 || (C.parity && off % 2 != 0) ||
+        C.nbox[C.rank - 1] * C.box[C.rank - 1] + off > C.pe[C.rank - 1])
+      return what + ": last-axis tap outside its copy";
+  }
   const int* xsrc = reinterpret_cast<const int*>(tab.data() + C.tab_xsrc);
   for (size_t i = 0; i < (size_t)C.ncq * C.xi * 64; ++i)
-    if (xsrc[i] < -1 || xsrc[i] >= C.cin_g * C.pvol) return what + ": input run source out of range";
+    if (xsrc[i] < -1 || xsrc[i] >= (int64_t)(C.ncopy - 1) * C.copy_elems + (int64_t)C.cin_g * C.pvol)
+      return what + ": input run source out of range";
   return "";
 }
 
@@ -2813,7 +2882,7 @@ int convnd_hip_plan_describe(const convnd_hip_problem* problem, convnd_hip_dtype
              ",\"items\":" + std::to_string(C.items) + ",\"npc\":" + std::to_string(C.npc) +
              ",\"items_per_pc\":" + std::to_string(C.items_per_pc) +
              ",\"ncq\":" + std::to_string(C.ncq) + ",\"mgroups\":" +
-             std::to_string(C.mgroups) + ",\"xi\":" + std::to_string(C.xi) +
+             std::to_string(C.mgroups) + ",\"copies\":" + std::to_string(C.ncopy) + ",\"xi\":" + std::to_string(C.xi) +
              ",\"di\":" + std::to_string(C.di) + ",\"lds\":" + std::to_string(p.lds) +
              ",\"exact\":" + std::to_string(p.exact ? 1 : 0) + ",\"workgroups\":" +
              std::to_string((int64_t)C.npc * C.ncq * C.groups * C.mgroups) + "}";

@@ -568,6 +568,14 @@ inline void wgrad_cm_chunk_channels(const WgradCmArgs& A, int cq, int* first, in
   *count = t0 < t1 ? (c_end - 1) / A.kvp - *first + 1 : 0;
 }
 
+// Copy of the padded input that last-axis tap tl reads, and its element offset there.
+inline void wgrad_cm_tap_copy(const WgradCmArgs& A, int tl, int* copy, int* offset) {
+  const int r = tl * A.dl % A.ls, q = tl * A.dl / A.ls;
+  const int odd = A.parity ? q & 1 : 0;
+  *copy = A.copy_id[2 * r + odd];
+  *offset = q - odd;
+}
+
 // Halo-row pitch (in rows) of each axis but the last.
 inline void wgrad_cm_row_pitch(const WgradCmArgs& A, int* hpitch) {
   int hp = 1;
@@ -684,7 +692,7 @@ inline void wgrad_cm_build_tables(const WgradCmArgs& A, unsigned char* tab) {
   }
   // Input run slots: slot = (channel c, halo row hr, run rho = tl * bl8 + sr) in LDS order;
   // its first element in the padded input: channel c, halo row hr (padded coordinates from
-  // the box origin), last-axis offset tl * dl + 8 * sr from the box origin.
+  // the box origin), last-axis offset of tap tl in its copy + 8 * sr from the box origin.
   const int nrho = A.kl * A.bl8;
   int* xsrc = reinterpret_cast<int*>(tab + A.tab_xsrc);
   for (int cq = 0; cq < A.ncq; ++cq) {
@@ -703,7 +711,9 @@ inline void wgrad_cm_build_tables(const WgradCmArgs& A, unsigned char* tab) {
           rem /= A.hext[a];
         }
         const int tl = rho / A.bl8, sr = rho % A.bl8;
-        v = c * A.pvol + roff + tl * A.dl + 8 * sr;
+        int copy, off;
+        wgrad_cm_tap_copy(A, tl, &copy, &off);
+        v = copy * A.copy_elems + c * A.pvol + roff + off + 8 * sr;
       }
       xsrc[(size_t)cq * A.xi * 64 + sl] = v;
     }
@@ -735,7 +745,7 @@ inline void wgrad_cm_build_tables(const WgradCmArgs& A, unsigned char* tab) {
     for (int a = R - 1; a >= 0; --a) {
       const int j0 = (bb % A.nbox[a]) * A.box[a];
       bb /= A.nbox[a];
-      xbase += (long long)j0 * A.s[a] * pstride[a];
+      xbase += (long long)j0 * (a == R - 1 ? 1 : A.s[a]) * pstride[a];
       dbase += (long long)j0 * dstride[a];
     }
     item[2 * it] = static_cast<int>(xbase);

@@ -270,6 +270,9 @@ struct WgradArgs {
 // Byte offset past every buffer the weight-gradient kernel reads: such a load returns zero.
 constexpr unsigned kWgradOob = 0x80000000u;
 
+constexpr int kMaxLastStride = 4;  // last-axis strides of the channel-major weight gradient
+constexpr int kMaxCopies = 2 * kMaxLastStride;
+
 // Arguments of the channel-major MFMA weight gradient (convnd_wgrad_cm.hip): the GEMM
 // M = output channels, N = columns (input channel, tap) in the weight layout's order (16 per
 // MFMA tile), K = output positions. Per box of positions the workgroup keeps in LDS, for
@@ -290,6 +293,14 @@ struct WgradCmArgs {
   int runpitch;         // LDS bytes per halo row: kl * bl8 runs of 16 bytes
   int chpitch;          // LDS bytes per staged channel (rows_h * runpitch)
   int dl;               // last-axis tap step (dilation)
+  // Copies of the padded input along the last axis (stride ls): a tap's step t*dl = q*ls + r reads
+  // phase r at offset q, from the copy of that phase shifted by one element when q is odd, so
+  // that every run starts on a 4-byte boundary: 16-byte loads at odd multiples of 2 bytes run at
+  // one lane per clock and CU, at 4-byte ones at 3.7. copy_id[2 r + (q & 1)] is the copy (-1:
+  // none), copy_elems the elements of one; parity 0: no shifted copies (one fits 32-bit
+  // offsets, two do not).
+  int ls, ncopy, copy_elems, parity;
+  signed char copy_id[2 * kMaxLastStride];
   int dyt_bytes;        // LDS bytes of the grad_output tile (MB * 16 rows of box_vol * 2)
   int xi, di;           // 64-run load instructions per item: input runs, grad_output runs
   int mgroups, ncq, nt; // output-channel groups of 16 * MB, column chunks, tiles per wave
@@ -375,8 +386,12 @@ struct PartialRescaleArgs {
 // Zero-padded channels-first copy of the input for the channel-major weight gradient:
 // dst[n][c][u] = src[n][c][u - pad] (zero outside the input), u_a < pe[a] (pe[rank-1] a
 // multiple of 8).
+// With copies > 1 or last_stride > 1 the destination is [copies][n][c][pe...], copy m holding
+// src at last-axis coordinate (u + shift[m]) * last_stride + phase[m] - last_pad.
 struct PlanarPadArgs {
   int rank, channels;
+  int copies, last_stride;
+  signed char phase[kMaxCopies], shift[kMaxCopies];
   // Outer axes a < rank - 1: input extent, padded extent, leading padding; entries from
   // rank - 1 on are identities (1, 1, 0) so the kernels walk all of them without a rank test.
   int in[kFastRank], pe[kFastRank], pad[kFastRank];

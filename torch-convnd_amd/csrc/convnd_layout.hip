@@ -65,6 +65,7 @@ struct DevPrologue {
   int e_blocks;
   int e_split_nc;  // split precision: source (image, channel) rows of each part block
   unsigned e_part_map;  // and the part each block holds
+  int e_nc_copy;        // (image, channel) rows of one copy
   // Channel partial sums of a channels-first 16-bit tensor (bias gradient): block (image,
   // channel, run of kSumRun positions) -> f_sums[c * (batch * f_nrun) + n * f_nrun + run].
   const void* f_src;
@@ -169,10 +170,11 @@ void prologue_kernel(DevPrologue P) {
     if constexpr (SPLIT) {
       stage::pad_planar_split_blocks(static_cast<const float*>(P.xpp_src),
                                      static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total,
-                                     P.e_split_nc, P.e_part_map, b);
+                                     P.e_split_nc, P.e_part_map, P.e_nc_copy, b);
     } else {
       stage::pad_planar16_blocks(static_cast<const unsigned short*>(P.xpp_src),
-                                 static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total, b);
+                                 static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total,
+                                 P.e_nc_copy, b);
     }
   }
 }
@@ -495,7 +497,10 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     P.ppa = *p.pp;
     P.xpp_src = p.x;
     P.x_pp = p.x_pp;
-    P.e_total = p.pp_batch * p.pp->channels * (p.pp->pvol / 8);
+    if (p.pp->copies < 1 || p.pp->copies > kMaxCopies || p.pp->last_stride < 1)
+      return hipErrorInvalidValue;
+    P.e_nc_copy = static_cast<int>(p.pp_batch * p.pp->channels);
+    P.e_total = p.pp->copies * p.pp_batch * p.pp->channels * (p.pp->pvol / 8);
     if (P.e_total > 0x7fffffff) return hipErrorInvalidValue;  // 32-bit run indices
     const int64_t per = (int64_t)stage::kPlanarRuns * kThreads;
     P.e_blocks = static_cast<int>((P.e_total + per - 1) / per);

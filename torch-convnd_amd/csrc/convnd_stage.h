@@ -408,11 +408,20 @@ struct PlanarRunSrc {
   int lo, hi;
 };
 
-__device__ __forceinline__ PlanarRunSrc planar_run_src(const PlanarPadArgs& P, int t) {
-  const int row = fast_div(t, P.div_chunks);  // (image, channel, padded row)
-  const int u0 = (t - row * (P.last_pe >> 3)) * 8 - P.last_pad;
-  const int nc = fast_div(row, P.div_rows);
+// nc_copy: (image, channel) rows of one copy; the copy is returned in *copy.
+__device__ __forceinline__ PlanarRunSrc planar_run_src(const PlanarPadArgs& P, int t, int nc_copy,
+                                                       int* copy) {
+  const int row = fast_div(t, P.div_chunks);  // (copy, image, channel, padded row)
+  int u0 = (t - row * (P.last_pe >> 3)) * 8 - P.last_pad;
+  int nc = fast_div(row, P.div_rows);
   int rem = row - nc * P.rows_per_img;
+  int m = 0;
+  while (nc >= nc_copy && m + 1 < P.copies) {
+    nc -= nc_copy;
+    ++m;
+  }
+  *copy = m;
+  u0 += P.shift[m];
   int srow = 0, istr = P.last_in;
   bool ok = true;
 #pragma unroll
@@ -430,6 +439,61 @@ __device__ __forceinline__ PlanarRunSrc planar_run_src(const PlanarPadArgs& P, i
   r.lo = -u0 < 0 ? 0 : (-u0 > 8 ? 8 : -u0);
   r.hi = ok ? (P.last_in - u0 < 0 ? 0 : (P.last_in - u0 > 8 ? 8 : P.last_in - u0)) : 0;
   return r;
+}
+
+// Copies of a strided last axis: the eight elements of a run lie last_stride apart in the source,
+// one load each (split_nc > 0: an fp32 source's bf16 part images, as below).
+template <typename Src>
+__device__ __forceinline__ void pad_planar_strided_blocks(const Src* src, unsigned short* dst,
+                                                          const PlanarPadArgs& P, int ntotal,
+                                                          int nc_copy, int split_nc,
+                                                          unsigned part_map, int block) {
+#pragma unroll
+  for (int q = 0; q < kPlanarRuns; ++q) {
+    const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
+    if (t >= ntotal) continue;
+    const int row = fast_div(t, P.div_chunks);
+    int nc = fast_div(row, P.div_rows);
+    int rem = row - nc * P.rows_per_img;
+    int m = 0;
+    while (nc >= nc_copy && m + 1 < P.copies) {
+      nc -= nc_copy;
+      ++m;
+    }
+    int part = 0;
+    if constexpr (sizeof(Src) == 4) {
+      const int s = nc / split_nc;
+      nc -= s * split_nc;
+      part = split_map_part(part_map, s);
+    }
+    int srow = 0, istr = P.last_in;
+    bool ok = true;
+#pragma unroll
+    for (int a = kFastRank - 2; a >= 0; --a) {
+      const int qa = fast_div(rem, P.div_pe[a]);
+      const int u = rem - qa * P.pe[a] - P.pad[a];
+      rem = qa;
+      ok = ok && u >= 0 && u < P.in[a];
+      srow += u * istr;
+      istr *= P.in[a];
+    }
+    const Src* s = src + (int64_t)nc * P.in_vol + srow;
+    const int u0 = (t - row * (P.last_pe >> 3)) * 8 + P.shift[m];
+    const int c0 = u0 * P.last_stride + P.phase[m] - P.last_pad;
+    unsigned h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int c = c0 + e * P.last_stride;
+      const bool in = ok && c >= 0 && c < P.last_in;
+      if constexpr (sizeof(Src) == 4) {
+        h[e] = in ? bf16_part_bits(s[c], part) : 0u;
+      } else {
+        h[e] = in ? s[c] : 0u;
+      }
+    }
+    *reinterpret_cast<u32x4*>(dst + (size_t)t * 8) =
+        u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+  }
 }
 
 // 16-byte chunk c of a buffer of nbytes (offset 0xfffffff0, past every buffer, for a chunk
@@ -458,13 +522,17 @@ __device__ __forceinline__ u32x4 planar_chunk16_tail(__amdgpu_buffer_rsrc_t sr, 
 __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
                                                     unsigned short* dst,
                                                     const PlanarPadArgs& P, int64_t total,
-                                                    int block) {
+                                                    int nc_copy, int block) {
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<unsigned short*>(src), static_cast<short>(0), static_cast<int>(P.src_bytes),
       0x00020000);
   const int64_t nbytes = static_cast<int64_t>(P.src_bytes);
   // 32-bit run indices: the planner keeps the copy and the source below 2^31 elements.
   const int ntotal = static_cast<int>(total);
+  if (P.last_stride > 1) {
+    pad_planar_strided_blocks<unsigned short>(src, dst, P, ntotal, nc_copy, 0, 0u, block);
+    return;
+  }
   // The two aligned 16-byte chunks that cover each run's 8 source elements (starting at
   // element o of the first).
   u32x4 c0[kPlanarRuns], c1[kPlanarRuns];
@@ -472,7 +540,8 @@ __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
-    const PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0);
+    int copy;
+    const PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy, &copy);
     const bool live = t < ntotal && r.lo < r.hi;
     const int64_t chunk = r.first >= 0 ? r.first >> 3 : -((7 - r.first) >> 3);  // floor(/8)
     o[q] = static_cast<int>(r.first - chunk * 8);
@@ -522,17 +591,22 @@ __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
 __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsigned short* dst,
                                                         const PlanarPadArgs& P, int64_t total,
                                                         int split_nc, unsigned part_map,
-                                                        int block) {
+                                                        int nc_copy, int block) {
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(src), static_cast<short>(0), static_cast<int>(P.src_bytes), 0x00020000);
   const int64_t nbytes = static_cast<int64_t>(P.src_bytes);
   const int ntotal = static_cast<int>(total);
+  if (P.last_stride > 1) {
+    pad_planar_strided_blocks<float>(src, dst, P, ntotal, nc_copy, split_nc, part_map, block);
+    return;
+  }
   u32x4 c0[kPlanarRuns], c1[kPlanarRuns], c2[kPlanarRuns];
   int o[kPlanarRuns], lo[kPlanarRuns], hi[kPlanarRuns], part[kPlanarRuns];
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
-    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0);
+    int copy;
+    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy, &copy);
     // Destination row block s reads source row nc - s * split_nc.
     const int s = r.nc / split_nc;
     r.first -= (int64_t)s * split_nc * P.in_vol;
