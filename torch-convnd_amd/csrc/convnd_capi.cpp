@@ -479,7 +479,7 @@ std::vector<IgemmPitches> choose_pitches(int R, const int* sigma, const IgemmBox
 // Any subset of the keys may be given; the planner then searches only plans matching it and
 // ignores the override when none does.
 struct PlanFilter {
-  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0, ts = -1, parity = -1;
+  int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0, ts = -1, parity = -1, plen = 0;
   std::vector<int> box;
   bool active = false;
 };
@@ -518,6 +518,7 @@ PlanFilter parse_filter(const char* text) {
         if (key == "waves") f.waves = v;
         if (key == "parts") f.parts = v;
         if (key == "ts") f.ts = v;
+        if (key == "plen") f.plen = v;
         if (key == "parity") f.parity = v;
       }
     }
@@ -586,24 +587,36 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   // Per axis: j extent, input step sigma, and the widest tap span over the phases.
   int J[kFastRank], sigma[kFastRank], span[kFastRank];
   int64_t ntaps_max = 1;
+  // Per axis over all phases (mode 1): smallest shift, and the span of every phase's taps; taps
+  // of the phases together.
+  int emin_all[kFastRank] = {}, span_all[kFastRank] = {};
+  double ntaps_mean = 1.0;
   for (int a = 0; a < R; ++a) {
     if (mode == 0) {
       J[a] = static_cast<int>(g.out[a]);
       sigma[a] = static_cast<int>(g.s[a]);
       span[a] = static_cast<int>((g.k[a] - 1) * g.d[a]);
+      span_all[a] = span[a];
       ntaps_max *= g.k[a];
     } else {
       J[a] = 0;
       sigma[a] = 1;
       span[a] = 0;
-      int nt = 0;
+      int nt = 0, lo = INT32_MAX, hi = INT32_MIN;
       for (int r = 0; r < g.s[a]; ++r) {
         const AxisPhaseHost t = grad_axis(g, a, r);
         J[a] = std::max(J[a], t.J);
         span[a] = std::max(span[a], t.emax - t.emin);
         nt = std::max(nt, t.ntap);
+        if (t.ntap > 0) {
+          lo = std::min(lo, t.emin);
+          hi = std::max(hi, t.emax);
+        }
       }
+      emin_all[a] = lo <= hi ? lo : 0;
+      span_all[a] = lo <= hi ? hi - lo : 0;
       ntaps_max *= nt;
+      ntaps_mean *= double(g.k[a]) / double(g.s[a]);
     }
   }
   const int mtiles = (gemm_cout + 15) / 16;
@@ -625,15 +638,16 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   if (filter.ds != 1 && filter.nbuf != 2) staging_options.push_back({false, 1});
   // Operand layouts of split precision (IgemmArgs::parts): the parts once each, or the six
   // copies as one K dimension, whose few channels fill whole octets better (3 channels: 24
-  // channels along K against 6 products x 8). Channel chunk: 1, 2, 3, 4, 6 or 8 octets dividing
+  // channels along K against 6 products x 8). Channel chunk: 1, 2, 3, 4, 6, 8, 12 or 16 octets dividing
   // the channels along K.
   const std::vector<int> part_options = split ? std::vector<int>{3, 1} : std::vector<int>{1};
 
   static const int kTiles[][3] = {{1, 2, 1}, {1, 4, 1}, {1, 8, 1}, {2, 2, 1}, {2, 4, 1},
                                   {2, 8, 1}, {4, 2, 1}, {4, 4, 1}, {4, 8, 1}, {1, 4, 2},
                                   {1, 8, 2}, {2, 4, 2}, {2, 8, 2}, {1, 4, 4}, {1, 8, 4}};
-  std::map<std::array<int, 3>, std::vector<IgemmBoxShape>> box_memo;   // by (box_vol, planes, tsplit)
-  std::map<std::vector<int>, std::vector<IgemmPitches>> pitch_memo;    // by box and tsplit
+  // Boxes by (box_vol, planes, tsplit, phases share a halo), their pitches by box and the last two.
+  std::map<std::array<int, 4>, std::vector<IgemmBoxShape>> box_memo;
+  std::map<std::vector<int>, std::vector<IgemmPitches>> pitch_memo;
   double best = -1.0;
   for (const auto& staging : staging_options)
   for (const int parts : part_options)
@@ -662,7 +676,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     const int mgroups = (mtiles + wm * mb - 1) / (wm * mb);
     const int box_vol = wn * nb * 16;
     const int reg_waves = igemm_reg_waves(mb, nb);
-    for (const int noct : {8, 6, 4, 3, 2, 1}) {
+    for (const int noct : {16, 12, 8, 6, 4, 3, 2, 1}) {
       const int cc = noct * 8;
       if (kcin % cc != 0 || (filter.cc && filter.cc != cc)) continue;
       const int planes = parts * noct;  // octet planes of a chunk
@@ -671,22 +685,33 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
       // every phase has.
       int64_t tcount = 1;
       for (int ts = 0; ts <= (direct ? 0 : std::min(2, R - 1)); ++ts) {
-      int span_ts[kFastRank];
-      for (int a = 0; a < R; ++a) span_ts[a] = a < ts ? 0 : span[a];
       if (ts > 0) {
         if (g.k[ts - 1] == 1 || (mode == 1 && g.s[ts - 1] != 1)) break;
         tcount *= g.k[ts - 1];
       }
       if (filter.ts >= 0 && filter.ts != ts) continue;
       const int64_t kc = (ntaps_max / tcount * cc + 31) / 32;
+      // Stride phases per workgroup: products of trailing strides, with the halo of one chunk.
+      for (int pa = R, plen = 1; pa >= 0; --pa) {
+      if (pa < R) {
+        if (mode == 0 || g.s[pa] == 1) continue;
+        plen *= static_cast<int>(g.s[pa]);
+        if (direct || tcount * nchunk != 1) break;
+      }
+      if (filter.plen && filter.plen != plen) continue;
+      const bool shared = plen > 1;
+      int span_ts[kFastRank];
+      for (int a = 0; a < R; ++a) span_ts[a] = a < ts ? 0 : (shared ? span_all[a] : span[a]);
+      // K32 steps of all phases of a workgroup.
+      const double ksteps = nphase == 1 ? double(kc) : plen * std::max(1.0, ntaps_mean / tcount * cc / 32.0);
       // The packing pass indexes weight elements with 32 bits.
       if (nphase * g.groups * tcount * nchunk * kc * parts * mgroups * wm * mb * 512 > kI32Safe) continue;
-      auto found = box_memo.find({box_vol, planes, ts});
+      auto found = box_memo.find({box_vol, planes, ts, shared});
       if (found == box_memo.end()) {
         // MFMA clocks of a CU per tile position over staging clocks per halo position and octet.
         const double weight = std::max(1.0, double(mtiles) * ntaps_max * (split ? 6.0 : 1.0) / 4.0);
         found = box_memo
-                    .emplace(std::array<int, 3>{box_vol, planes, ts},
+                    .emplace(std::array<int, 4>{box_vol, planes, ts, shared},
                              igemm_boxes(R, J, sigma, span_ts, box_vol, planes, weight))
                     .first;
       }
@@ -709,7 +734,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           const int64_t plane_bytes = plane_align(plane_pos * 16);
           const int tap_row = static_cast<int>((kc + kTapPad + 3) / 4 * 4);
           const int64_t lds = nbuf * planes * plane_bytes + align_up(rows * (direct ? 8 : 4)) +
-                              align_up(box_vol * 4) + align_up(16 * tap_row);
+                              align_up(box_vol * 4) + align_up(16 * tap_row * plen);
           if (rows > (int64_t{1} << 20)) return -1.0;
           const bool grid_ok = boxes <= (int64_t{1} << 30) && g.groups * mgroups <= 65535 &&
                                g.batch * nphase <= 65535;
@@ -734,21 +759,28 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           auto pow4 = [](double v) { return v * v * v * v; };
           const double step =
               std::sqrt(std::sqrt(pow4(mfma) + pow4(ldsc) + pow4(l1) + pow4(latency)));
-          const double core = double(tcount * nchunk) * kc * step;
+          const double core = double(tcount * nchunk) * ksteps * step + (plen - 1) * 1800.0;
           // Staging of each chunk's halo: bytes and a round trip; direct staging moves whole runs
           // of 8 last-axis elements per task, mostly partial ones on halo rows shorter than two
           // runs. A second resident workgroup hides about half of it.
           const double halo_bytes = planes * hvol * 16.0;
           const double stage = double(tcount * nchunk) * (direct ? halo_bytes / 31.0 * short_rows + 2600.0
-                                                                 : halo_bytes / 18.4 + 6000.0);
+                                                                 : nphase > 1 ? halo_bytes / 10.0 + 8000.0
+                                                                              : halo_bytes / 18.4 + 6000.0);
           const double exposed = (occ >= 2 ? 0.486 * occ : 1.3) * stage;
-          const double epilogue = double(wm) * mb * 16 * box_vol * 0.25;
+          // Phases of a strided last axis store single elements, a cache line per box row.
+          const double per_value =
+              nphase == 1 ? 0.25 : 0.36 + (g.s[R - 1] > 1 ? 1.48 / std::min(b[R - 1], 16) : 0.0);
+          const double epilogue = double(wm) * mb * 16 * box_vol * per_value * plen;
           const double per_round = core + exposed + occ * (epilogue + 10.0 * rows) + 2900.0;
           // Work in padded boxes beyond the tensor is paid for as well (included via boxes). A
-          // partly filled last round of workgroups costs about two fifths of a whole one at least.
-          const int64_t wgs = boxes * g.groups * mgroups * g.batch * nphase;
+          // partly filled last round of workgroups costs about two fifths of a whole one at least,
+          // a whole one where the workgroups are the longer ones of several phases. (Terms of
+          // strided input gradients fitted to 1100 measured plans of 14 more problems.)
+          const int64_t wgs = boxes * g.groups * mgroups * g.batch * (nphase / plen);
           const double share = double(wgs) / (256.0 * occ);
-          const double rounds = 0.41 * std::ceil(share) + 0.59 * std::max(share, 1.0);
+          const double whole = shared ? 1.0 : 0.41;
+          const double rounds = whole * std::ceil(share) + (1.0 - whole) * std::max(share, 1.0);
           *lds_out = lds;
           *occ_out = occ;
           // The octet-major copy reads the operand and writes the staged channels (3.5 TB/s).
@@ -761,7 +793,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
         // The pitches depend on the box alone (not on the tile or the chunk) and only cost more
         // than dense conflict-free planes: chosen for boxes that could win.
         std::vector<int> key(b, b + R);
-        key.push_back(ts);
+        key.push_back(2 * ts + (shared ? 1 : 0));
         auto hit = pitch_memo.find(key);
         if (hit == pitch_memo.end()) {
           const double least = evaluate(hvol, 1.0, &lds, &occ);
@@ -804,6 +836,8 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           A.nchunk = static_cast<int>(nchunk);
           A.tsplit = ts;
           A.tcount = static_cast<int>(tcount);
+          A.plen = plen;
+          std::copy(emin_all, emin_all + kFastRank, A.emin_all);
           A.kc_max = static_cast<int>(kc);
           A.wm = wm;
           A.mtiles = mtiles;
@@ -848,6 +882,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           A.nrun = (hext[R - 1] + 14) / 8;  // bound; the exact count is set below
           plan.lds = static_cast<size_t>(lds);
         }
+      }
       }
       }
     }
@@ -2676,7 +2711,7 @@ std::string check_igemm_tables(const IgemmArgs& A0, size_t lds_bytes, const char
   // LDS carve-up: halo buffers, row tables (2 ints per row), box output offsets, taps.
   const size_t lds_need = (size_t)nbuf * A.halo_bytes +
                           (size_t)((A.rows + 3) & ~3) * (A.direct ? 8 : 4) +
-                          (size_t)((A.box_vol + 3) & ~3) * 4 + (size_t)4 * A.tap_row * 4;
+                          (size_t)((A.box_vol + 3) & ~3) * 4 + (size_t)A.plen * 4 * A.tap_row * 4;
   if (lds_need > lds_bytes) return fail_at("LDS layout exceeds the plan's LDS size");
   const int4* pos = reinterpret_cast<const int4*>(tab.data() + A.tab_pos);
   const int4* rows = reinterpret_cast<const int4*>(tab.data() + A.tab_rows);
@@ -2725,6 +2760,9 @@ std::string check_igemm_tables(const IgemmArgs& A0, size_t lds_bytes, const char
     for (int bx = 0; bx < A.boxes; ++bx) {
       const IgemmBox& B = boxes[ph * A.boxes + bx];
       if (B.flags & 1) continue;
+      const IgemmBox& F = boxes[ph / A.plen * A.plen * A.boxes + bx];
+      if ((F.flags & 1) || F.in_base != B.in_base || F.corg != B.corg || F.lo != B.lo || F.hi != B.hi)
+        return fail_at("phases of a group do not share their halo");
       if (B.kc > A.kc_max || B.kf > B.kc || B.kf < 0)
         return fail_at("box K steps exceed the plan");
       if (B.kf + 4 > A.tap_row) return fail_at("tap prefetch reads past the tap row");
@@ -2860,7 +2898,7 @@ int convnd_hip_plan_describe(const convnd_hip_problem* problem, convnd_hip_dtype
              ",\"boxes\":" + std::to_string(A.boxes) + ",\"phases\":" +
              std::to_string(A.nphase) + ",\"cc\":" + std::to_string(A.cc) +
              ",\"parts\":" + std::to_string(A.parts) + ",\"tsplit\":" + std::to_string(A.tsplit) +
-             ",\"tcount\":" + std::to_string(A.tcount) +
+             ",\"tcount\":" + std::to_string(A.tcount) + ",\"plen\":" + std::to_string(A.plen) +
              ",\"nchunk\":" + std::to_string(A.nchunk) + ",\"kc_max\":" +
              std::to_string(A.kc_max) + ",\"mgroups\":" + std::to_string(A.mgroups) +
              ",\"lds\":" + std::to_string(p.lds) + ",\"direct\":" + std::to_string(A.direct) +
@@ -2868,7 +2906,7 @@ int convnd_hip_plan_describe(const convnd_hip_problem* problem, convnd_hip_dtype
              ",\"occupancy\":" +
              std::to_string(p.occ) + ",\"waves\":" + std::to_string(p.waves) +
              ",\"workgroups\":" +
-             std::to_string((int64_t)A.boxes * A.groups * A.mgroups * A.batch * A.nphase) + "}";
+             std::to_string((int64_t)A.boxes * A.groups * A.mgroups * A.batch * (A.nphase / A.plen)) + "}";
     }
   } else if (which == 2) {
     const WgradPlan p = plan_wgrad(g, dtype);

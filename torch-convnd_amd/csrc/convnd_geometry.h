@@ -91,6 +91,7 @@ __host__ __device__ inline int phase_axes(const IgemmArgs& A, int phase, AxisTap
   for (int a = A.rank - 1; a >= 0; --a) {
     const int radix = A.mode ? A.s[a] : 1;
     ax[a] = axis_taps(A, a, rr % radix);
+    if (A.plen > 1) ax[a].emin = A.emin_all[a];
     rr /= radix;
     if (a >= A.tsplit) ntaps *= ax[a].ntap;
   }

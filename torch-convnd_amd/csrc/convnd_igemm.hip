@@ -91,8 +91,11 @@ void igemm_kernel(IgemmArgs A) {
   const int wm = wave % WM;
   const int wn = wave / WM;
   const int lg = lane >> 4;
-  const int n = blockIdx.z / A.nphase;
-  const int phase = blockIdx.z % A.nphase;
+  // Phases phase .. phase + plen - 1 (plen 1 unless the octet-major halo is shared by several).
+  const int plen = DS ? 1 : A.plen;
+  const int phase_groups = DS ? A.nphase : A.nphase / plen;
+  const int n = blockIdx.z / phase_groups;
+  int phase = (blockIdx.z % phase_groups) * plen;
   const int g = blockIdx.y / A.mgroups;
   const int mg = blockIdx.y % A.mgroups;
 
@@ -107,16 +110,18 @@ void igemm_kernel(IgemmArgs A) {
     }
   }
   const char* tab = static_cast<const char*>(A.tables);
-  const IgemmBox& box = reinterpret_cast<const IgemmBox*>(tab + A.tab_box)[phase * A.boxes + bx];
-  const int flags = box.flags;
-  if (flags & 1) return;  // uniform over the workgroup (phase with a shorter j extent)
-  const int KC = box.kc;
-  const int KF = box.kf;
+  const IgemmBox* boxp = reinterpret_cast<const IgemmBox*>(tab + A.tab_box) + phase * A.boxes + bx;
+  // Uniform over the workgroup (phase with a shorter j extent; the first of a group has the
+  // longest).
+  if (boxp->flags & 1) return;
+  const IgemmBox& box = *boxp;  // the halo: the same for every phase of the group
+  int KC = box.kc;
+  int KF = box.kf;
 
   // LDS: [octet planes (DS: nbuf sets, alternating per channel chunk) | rows: input offset
   // (-1 outside the input), with DS also LDS position offset | output offset of every box position (read
-  // by the epilogue; kept out of registers during the main loop) | the phase's tap offsets,
-  // 4 lane groups x tap_row].
+  // by the epilogue; kept out of registers during the main loop) | the phases' tap offsets,
+  // 4 lane groups x tap_row each].
   int* rowin = reinterpret_cast<int*>(lds + (DS ? A.nbuf : 1) * A.halo_bytes);
   const int rows4 = (A.rows + 3) & ~3;
   int* rowlds = rowin + rows4;  // (direct staging)
@@ -126,7 +131,7 @@ void igemm_kernel(IgemmArgs A) {
   for (int q = tid; q < A.box_vol; q += kWT) posout[q] = pt[q].y;
   {
     const int* gt = reinterpret_cast<const int*>(tab + A.tab_taps) + phase * 4 * A.tap_row;
-    for (int i = tid; i < 4 * A.tap_row; i += kWT) ltaps[i] = gt[i];
+    for (int i = tid; i < plen * 4 * A.tap_row; i += kWT) ltaps[i] = gt[i];
   }
   // Input offset of every halo row, for split tap tc: its shift moves the origin and the bounds
   // along the split axes.
@@ -169,7 +174,7 @@ void igemm_kernel(IgemmArgs A) {
   // Tap offsets of this lane group (LDS, read in pairs of steps ahead of use); the partial
   // last step separately.
   const int* tp = ltaps + lg * A.tap_row;
-  const int tail_tap = reinterpret_cast<const int*>(tab + A.tab_tail)[phase * 4 + lg];
+  int tail_tap = reinterpret_cast<const int*>(tab + A.tab_tail)[phase * 4 + lg];
   // Bias of this wave's output channels, loaded now so its latency hides behind the loop.
   const int mt0 = (mg * WM + wm) * MB;  // first m-tile of this wave
   // The MFMAs run with the positions as the A operand, so D = (W X)^T: lane l holds output
@@ -206,7 +211,7 @@ void igemm_kernel(IgemmArgs A) {
   // MFMAs of chunk ck (split tap, channel chunk) over the halo planes at hb. `issue` runs once, after the first
   // weight fragments and B fragments are requested and before the loop (the next chunk's
   // staging loads go there, behind this chunk's first weight loads in the load queue).
-  auto mma_chunk = [&](int ck, const unsigned char* hb, auto&& issue) {
+  auto mma_chunk = [&](int ck, const unsigned char* hb, auto&& issue) __attribute__((always_inline)) {
     const frag* wck = wp +
                       ((size_t)((phase * A.groups + g) * A.tcount * A.nchunk + ck) * A.kc_max) * wstep +
                       (size_t)mt0 * 64 + lane;
@@ -481,6 +486,143 @@ void igemm_kernel(IgemmArgs A) {
     }
   };
 
+  // Epilogue: straight from the accumulators. A lane's four values are box positions
+  // 4*lg .. 4*lg+3 of its position block. In a box inside the output whose rows have whole runs
+  // of 4 positions on a unit output step they are adjacent: one 8-byte store for 16-bit
+  // O, 16 bytes for float. Otherwise every position has its own offset and bounds check, and a
+  // lane whose four positions are all inside and adjacent still stores them at once.
+  // The activation is a compile-time constant of each epilogue copy, dispatched once: every
+  // copy's code is contiguous (a launch starts on a cold instruction cache, and per-element
+  // branches over the activations' code would spread the executed instructions over many
+  // more cache lines).
+  auto store4 = [](O* dst, const O* v) {
+    if constexpr (sizeof(O) == 2) {
+      uint2 w;
+      w.x = __builtin_bit_cast(unsigned short, v[0]) |
+            ((unsigned)__builtin_bit_cast(unsigned short, v[1]) << 16);
+      w.y = __builtin_bit_cast(unsigned short, v[2]) |
+            ((unsigned)__builtin_bit_cast(unsigned short, v[3]) << 16);
+      *reinterpret_cast<uint2*>(dst) = w;
+    } else {
+      *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+    }
+  };
+  // (Inlined by force: left out of line for the largest tile, it put the accumulators in scratch.)
+  auto epilogue = [&](auto act_c) __attribute__((always_inline)) {
+    constexpr int kAct = decltype(act_c)::value;
+    const int flags = boxp->flags;
+    O* out = static_cast<O*>(A.out);
+    const size_t chan0 = (size_t)n * A.cout_total + (size_t)g * A.cout_g;
+    O* obox = out + boxp->out_origin;
+    if (A.out_cl) {
+      // Channels-last output: output channel m of position q at
+      // ((n*out_vol + q)*cout_total + g*cout_g + m); sixteen lanes write one position's 16
+      // consecutive channels.
+      const size_t ostride = static_cast<size_t>(A.cout_total);
+      O* ocl = out + ((size_t)n * A.out_vol + boxp->out_origin) * ostride + (size_t)g * A.cout_g;
+      const bool inside = A.packed_ok && (flags & 2);
+      int off[NB][4];
+      {
+        const unsigned long long lim = boxp->lim;
+        const unsigned long long guard = A.coord_bits == 16 ? kGuard16 : kGuard8;
+        const unsigned long long ones = A.coord_bits == 16 ? kOnes16 : kOnes8;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int q = (wn * NB + nb) * 16 + 4 * lg + i;
+            if (inside) {
+              off[nb][i] = posout[q];
+            } else {
+              const int4 e = pt[q];
+              const unsigned long long c = static_cast<unsigned>(e.z) |
+                                           (static_cast<unsigned long long>(static_cast<unsigned>(e.w)) << 32);
+              off[nb][i] = swar_all_less(c, lim, guard, ones) ? e.y : -1;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const int m = (mt0 + mb) * 16 + (lane & 15);
+        if (m >= A.cout_g) continue;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (off[nb][i] >= 0)
+              ocl[(size_t)off[nb][i] * ostride + m] =
+                  static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
+        }
+      }
+    } else if (A.packed_ok && (flags & 2)) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const int m = (mt0 + mb) * 16 + (lane & 15);
+        if (m >= A.cout_g) continue;
+        O* orow = obox + (chan0 + m) * A.out_vol;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          O v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
+          store4(orow + posout[(wn * NB + nb) * 16 + 4 * lg], v);
+        }
+      }
+    } else {
+      const unsigned long long lim = boxp->lim;
+      const unsigned long long guard = A.coord_bits == 16 ? kGuard16 : kGuard8;
+      const unsigned long long ones = A.coord_bits == 16 ? kOnes16 : kOnes8;
+      int off[NB][4];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int4 e = pt[(wn * NB + nb) * 16 + 4 * lg + i];
+          const unsigned long long c =
+              static_cast<unsigned>(e.z) | (static_cast<unsigned long long>(static_cast<unsigned>(e.w)) << 32);
+          off[nb][i] = swar_all_less(c, lim, guard, ones) ? e.y : -1;
+        }
+      }
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const int m = (mt0 + mb) * 16 + (lane & 15);
+        if (m >= A.cout_g) continue;
+        O* orow = obox + (chan0 + m) * A.out_vol;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          O v[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            v[i] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
+          const int o0 = off[nb][0];
+          if (o0 >= 0 && off[nb][1] == o0 + 1 && off[nb][2] == o0 + 2 && off[nb][3] == o0 + 3) {
+            store4(orow + o0, v);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (off[nb][i] >= 0) orow[off[nb][i]] = v[i];
+          }
+        }
+      }
+    }
+  };
+  auto store_outputs = [&]() __attribute__((always_inline)) {
+    switch (A.act) {
+      case CONVND_HIP_ACT_RELU:
+        epilogue(std::integral_constant<int, CONVND_HIP_ACT_RELU>{});
+        break;
+      case CONVND_HIP_ACT_GELU:
+        epilogue(std::integral_constant<int, CONVND_HIP_ACT_GELU>{});
+        break;
+      case CONVND_HIP_ACT_GELU_TANH:
+        epilogue(std::integral_constant<int, CONVND_HIP_ACT_GELU_TANH>{});
+        break;
+      default:
+        epilogue(std::integral_constant<int, CONVND_HIP_ACT_NONE>{});
+    }
+  };
+
   if constexpr (DS) {
     // Halo staged straight from the channels-first operand [N][cin_total][in_vol]. A task
     // (halo row r, run jj, octet o; octet fastest) loads the run of 8 consecutive last-axis
@@ -633,6 +775,7 @@ void igemm_kernel(IgemmArgs A) {
         __syncthreads();  // next chunk's halo written
       }
     }
+    store_outputs();
   } else {
     // Halo staged straight to LDS from the octet-major copy, every load in flight at once: a
     // wave's load writes 64 consecutive LDS positions of a plane (1 KB), each lane reading the
@@ -672,153 +815,40 @@ void igemm_kernel(IgemmArgs A) {
         }
       }
     };
-    for (int tc = 0; tc < A.tcount; ++tc) {
-      if (tc > 0) {
+    // The phases of the group (one, unless plen > 1) from one halo: with several there is one
+    // chunk, staged for the first. Half of a strided input gradient's workgroup was staging the
+    // halo that its phases share: 128 <- 64 channels in 4 groups, stride 2 on three axes, 24^3 x 12,
+    // 103 -> 79 us.
+    for (int q = 0;;) {
+      for (int tc = 0; tc < A.tcount; ++tc) {
         // Every wave is past the staging that read the rows (the last chunk's barrier).
-        fill_rows(tc);
-      }
-      for (int ck = 0; ck < A.nchunk; ++ck) {
-        // Row table written, and every wave done reading the chunk before.
-        __syncthreads();
-        stage(ck);
-        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads have landed in LDS
-        __syncthreads();
-        mma_chunk(tc * A.nchunk + ck, lds, []() {});
-      }
-    }
-  }
-
-  // Epilogue: straight from the accumulators. A lane's four values are box positions
-  // 4*lg .. 4*lg+3 of its position block. In a box inside the output whose rows have whole runs
-  // of 4 positions on a unit output step they are adjacent: one 8-byte store for 16-bit
-  // O, 16 bytes for float. Otherwise every position has its own offset and bounds check, and a
-  // lane whose four positions are all inside and adjacent still stores them at once.
-  // The activation is a compile-time constant of each epilogue copy, dispatched once: every
-  // copy's code is contiguous (a launch starts on a cold instruction cache, and per-element
-  // branches over the activations' code would spread the executed instructions over many
-  // more cache lines).
-  auto store4 = [](O* dst, const O* v) {
-    if constexpr (sizeof(O) == 2) {
-      uint2 w;
-      w.x = __builtin_bit_cast(unsigned short, v[0]) |
-            ((unsigned)__builtin_bit_cast(unsigned short, v[1]) << 16);
-      w.y = __builtin_bit_cast(unsigned short, v[2]) |
-            ((unsigned)__builtin_bit_cast(unsigned short, v[3]) << 16);
-      *reinterpret_cast<uint2*>(dst) = w;
-    } else {
-      *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-    }
-  };
-  auto epilogue = [&](auto act_c) {
-    constexpr int kAct = decltype(act_c)::value;
-    O* out = static_cast<O*>(A.out);
-    const size_t chan0 = (size_t)n * A.cout_total + (size_t)g * A.cout_g;
-    O* obox = out + box.out_origin;
-    if (A.out_cl) {
-      // Channels-last output: output channel m of position q at
-      // ((n*out_vol + q)*cout_total + g*cout_g + m); sixteen lanes write one position's 16
-      // consecutive channels.
-      const size_t ostride = static_cast<size_t>(A.cout_total);
-      O* ocl = out + ((size_t)n * A.out_vol + box.out_origin) * ostride + (size_t)g * A.cout_g;
-      const bool inside = A.packed_ok && (flags & 2);
-      int off[NB][4];
-      {
-        const unsigned long long lim = box.lim;
-        const unsigned long long guard = A.coord_bits == 16 ? kGuard16 : kGuard8;
-        const unsigned long long ones = A.coord_bits == 16 ? kOnes16 : kOnes8;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int q = (wn * NB + nb) * 16 + 4 * lg + i;
-            if (inside) {
-              off[nb][i] = posout[q];
-            } else {
-              const int4 e = pt[q];
-              const unsigned long long c = static_cast<unsigned>(e.z) |
-                                           (static_cast<unsigned long long>(static_cast<unsigned>(e.w)) << 32);
-              off[nb][i] = swar_all_less(c, lim, guard, ones) ? e.y : -1;
-            }
+        if (tc > 0) fill_rows(tc);
+        for (int ck = 0; ck < A.nchunk; ++ck) {
+          if (q == 0) {
+            // Row table written, and every wave done reading the chunk before.
+            __syncthreads();
+            stage(ck);
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads have landed in LDS
+            __syncthreads();
           }
+          mma_chunk(tc * A.nchunk + ck, lds, []() {});
         }
       }
+      store_outputs();
+      do {
+        if (++q == plen) return;
+        ++phase;
+        boxp += A.boxes;
+      } while (boxp->flags & 1);
+      KC = boxp->kc;
+      KF = boxp->kf;
+      tp = ltaps + (q * 4 + lg) * A.tap_row;
+      tail_tap = reinterpret_cast<const int*>(tab + A.tab_tail)[phase * 4 + lg];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const int m = (mt0 + mb) * 16 + (lane & 15);
-        if (m >= A.cout_g) continue;
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (off[nb][i] >= 0)
-              ocl[(size_t)off[nb][i] * ostride + m] =
-                  static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
-        }
-      }
-    } else if (A.packed_ok && (flags & 2)) {
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const int m = (mt0 + mb) * 16 + (lane & 15);
-        if (m >= A.cout_g) continue;
-        O* orow = obox + (chan0 + m) * A.out_vol;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          O v[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
-          store4(orow + posout[(wn * NB + nb) * 16 + 4 * lg], v);
-        }
-      }
-    } else {
-      const unsigned long long lim = box.lim;
-      const unsigned long long guard = A.coord_bits == 16 ? kGuard16 : kGuard8;
-      const unsigned long long ones = A.coord_bits == 16 ? kOnes16 : kOnes8;
-      int off[NB][4];
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int4 e = pt[(wn * NB + nb) * 16 + 4 * lg + i];
-          const unsigned long long c =
-              static_cast<unsigned>(e.z) | (static_cast<unsigned long long>(static_cast<unsigned>(e.w)) << 32);
-          off[nb][i] = swar_all_less(c, lim, guard, ones) ? e.y : -1;
-        }
-      }
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const int m = (mt0 + mb) * 16 + (lane & 15);
-        if (m >= A.cout_g) continue;
-        O* orow = obox + (chan0 + m) * A.out_vol;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          O v[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            v[i] = static_cast<O>(epilogue_act(acc[mb][nb][i] + bias_v[mb], kAct));
-          const int o0 = off[nb][0];
-          if (o0 >= 0 && off[nb][1] == o0 + 1 && off[nb][2] == o0 + 2 && off[nb][3] == o0 + 3) {
-            store4(orow + o0, v);
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (off[nb][i] >= 0) orow[off[nb][i]] = v[i];
-          }
-        }
-      }
+        for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-  };
-  switch (A.act) {
-    case CONVND_HIP_ACT_RELU:
-      epilogue(std::integral_constant<int, CONVND_HIP_ACT_RELU>{});
-      break;
-    case CONVND_HIP_ACT_GELU:
-      epilogue(std::integral_constant<int, CONVND_HIP_ACT_GELU>{});
-      break;
-    case CONVND_HIP_ACT_GELU_TANH:
-      epilogue(std::integral_constant<int, CONVND_HIP_ACT_GELU_TANH>{});
-      break;
-    default:
-      epilogue(std::integral_constant<int, CONVND_HIP_ACT_NONE>{});
   }
 }
 
@@ -837,7 +867,7 @@ void igemm_kernel(IgemmArgs A) {
   X(1, 2, 1) X(1, 4, 1) X(2, 2, 1) X(2, 4, 1) X(1, 4, 2) X(2, 4, 2) X(2, 2, 2) X(1, 4, 4) X(4, 2, 1)
 
 hipError_t igemm_dispatch_p3(int mb, int nb, const IgemmArgs& a, size_t lds, hipStream_t s) {
-  const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * a.nphase);
+  const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * (a.nphase / a.plen));
 #define CONVND_IGEMM_CASE(MBV, NBV, WMV)                                                       \
   if (mb == MBV && nb == NBV && a.wm == WMV && a.waves == 4) {                                 \
     auto fn = igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3>;                         \
@@ -854,7 +884,7 @@ hipError_t igemm_dispatch_p3(int mb, int nb, const IgemmArgs& a, size_t lds, hip
 
 template <typename T, typename O, bool DS>
 hipError_t igemm_dispatch(int mb, int nb, const IgemmArgs& a, size_t lds, hipStream_t s) {
-  const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * a.nphase);
+  const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * (a.nphase / a.plen));
 #define CONVND_IGEMM_CASE(MBV, NBV, WMV)                                                 \
   if (mb == MBV && nb == NBV && a.wm == WMV && a.waves == 4) {                           \
     auto fn = igemm_kernel<T, O, MBV, NBV, WMV, DS, 4>;                                  \

@@ -121,6 +121,12 @@ struct IgemmArgs {
   // or 2) is a chunk of its own, so that the halo in LDS does not extend along those axes. K runs
   // over (split tap, channel chunk, remaining tap, channel).
   int tsplit, tcount;
+  // Stride phases of one workgroup (input gradient, octet-major staging, one chunk): plen
+  // consecutive phases read one halo, staged once, whose origin is the smallest shift of any
+  // phase per axis (emin_all). plen is a product of trailing strides; 1: a phase per workgroup,
+  // with a halo of its own.
+  int plen;
+  int emin_all[kFastRank];
   int wm;                     // waves along M (output channels); 4 / wm along positions
   int mtiles, mgroups, mtiles_padded;
   int plane_bytes;            // LDS bytes of one octet plane (multiple of 256; of 1024, one load

@@ -499,6 +499,10 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     P.x_pp = p.x_pp;
     if (p.pp->copies < 1 || p.pp->copies > kMaxCopies || p.pp->last_stride < 1)
       return hipErrorInvalidValue;
+    // Unit last stride: the copy, and at most one shifted by an element (planar_run_src).
+    if (p.pp->last_stride == 1 && (p.pp->copies > 2 || p.pp->shift[0] != 0 ||
+                                   (p.pp->copies == 2 && p.pp->shift[1] != 1)))
+      return hipErrorInvalidValue;
     P.e_nc_copy = static_cast<int>(p.pp_batch * p.pp->channels);
     P.e_total = p.pp->copies * p.pp_batch * p.pp->channels * (p.pp->pvol / 8);
     if (P.e_total > 0x7fffffff) return hipErrorInvalidValue;  // 32-bit run indices

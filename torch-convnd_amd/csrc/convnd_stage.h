@@ -408,20 +408,17 @@ struct PlanarRunSrc {
   int lo, hi;
 };
 
-// nc_copy: (image, channel) rows of one copy; the copy is returned in *copy.
-__device__ __forceinline__ PlanarRunSrc planar_run_src(const PlanarPadArgs& P, int t, int nc_copy,
-                                                       int* copy) {
+// A unit last stride has one copy, or a second one shifted by one element; nc_copy: (image,
+// channel) rows of a copy.
+__device__ __forceinline__ PlanarRunSrc planar_run_src(const PlanarPadArgs& P, int t, int nc_copy) {
   const int row = fast_div(t, P.div_chunks);  // (copy, image, channel, padded row)
   int u0 = (t - row * (P.last_pe >> 3)) * 8 - P.last_pad;
   int nc = fast_div(row, P.div_rows);
   int rem = row - nc * P.rows_per_img;
-  int m = 0;
-  while (nc >= nc_copy && m + 1 < P.copies) {
+  if (P.copies > 1 && nc >= nc_copy) {  // (uniform where there is one copy)
     nc -= nc_copy;
-    ++m;
+    u0 += 1;
   }
-  *copy = m;
-  u0 += P.shift[m];
   int srow = 0, istr = P.last_in;
   bool ok = true;
 #pragma unroll
@@ -540,8 +537,7 @@ __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
-    int copy;
-    const PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy, &copy);
+    const PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy);
     const bool live = t < ntotal && r.lo < r.hi;
     const int64_t chunk = r.first >= 0 ? r.first >> 3 : -((7 - r.first) >> 3);  // floor(/8)
     o[q] = static_cast<int>(r.first - chunk * 8);
@@ -605,8 +601,7 @@ __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsign
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
-    int copy;
-    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy, &copy);
+    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy);
     // Destination row block s reads source row nc - s * split_nc.
     const int s = r.nc / split_nc;
     r.first -= (int64_t)s * split_nc * P.in_vol;
