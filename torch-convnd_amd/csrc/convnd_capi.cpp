@@ -836,6 +836,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           A.nchunk = static_cast<int>(nchunk);
           A.tsplit = ts;
           A.tcount = static_cast<int>(tcount);
+          A.tvol = static_cast<int>(g.k_vol / tcount);
           A.plen = plen;
           std::copy(emin_all, emin_all + kFastRank, A.emin_all);
           A.kc_max = static_cast<int>(kc);

@@ -121,6 +121,7 @@ struct IgemmArgs {
   // or 2) is a chunk of its own, so that the halo in LDS does not extend along those axes. K runs
   // over (split tap, channel chunk, remaining tap, channel).
   int tsplit, tcount;
+  int tvol;  // taps per split tap: k_vol / tcount
   // Stride phases of one workgroup (input gradient, octet-major staging, one chunk): plen
   // consecutive phases read one halo, staged once, whose origin is the smallest shift of any
   // phase per axis (emin_all). plen is a product of trailing strides; 1: a phase per workgroup,

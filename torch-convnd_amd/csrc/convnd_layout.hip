@@ -66,6 +66,8 @@ struct DevPrologue {
   int e_split_nc;  // split precision: source (image, channel) rows of each part block
   unsigned e_part_map;  // and the part each block holds
   int e_nc_copy;        // (image, channel) rows of one copy
+  // The three parts of an fp32 source from one read of it, for each of the copies.
+  bool a_all_parts, d_all_parts, e_all_parts;
   // Channel partial sums of a channels-first 16-bit tensor (bias gradient): block (image,
   // channel, run of kSumRun positions) -> f_sums[c * (batch * f_nrun) + n * f_nrun + run].
   const void* f_src;
@@ -147,6 +149,13 @@ void prologue_kernel(DevPrologue P) {
   b -= P.b_blocks;
   if (b < P.a_blocks) {
     const int bx = b % P.a_nbx, r = b / P.a_nbx, o = r % P.a_octs, n = r / P.a_octs;
+    if constexpr (SPLIT) {
+      if (P.a_all_parts) {
+        stage::octet_parts_block(static_cast<const float*>(P.src),
+                                 static_cast<unsigned short*>(P.staged), P.sa, bx, o, n);
+        return;
+      }
+    }
     stage::octets16_block<S>(static_cast<const S*>(P.src), static_cast<unsigned short*>(P.staged),
                              P.sa, P.a_vec, bx, o, n, P.a_nbx, P.sums,
                              P.a_nbx * (P.a_blocks / (P.a_nbx * P.a_octs)), P.is_bf16, &smem);
@@ -162,7 +171,8 @@ void prologue_kernel(DevPrologue P) {
   b -= P.c_blocks;
   if (b < P.d_blocks) {
     stage::pad_dy16_blocks<S>(static_cast<const S*>(P.dy), static_cast<unsigned short*>(P.dy_pad),
-                              P.wg, P.split_batch, P.dy_part_map, P.runs, b, P.d_blocks);
+                              P.wg, P.split_batch, P.dy_part_map, P.d_all_parts, P.runs, b,
+                              P.d_blocks);
     return;
   }
   b -= P.d_blocks;
@@ -170,7 +180,7 @@ void prologue_kernel(DevPrologue P) {
     if constexpr (SPLIT) {
       stage::pad_planar_split_blocks(static_cast<const float*>(P.xpp_src),
                                      static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total,
-                                     P.e_split_nc, P.e_part_map, P.e_nc_copy, b);
+                                     P.e_split_nc, P.e_part_map, P.e_nc_copy, P.e_all_parts, b);
     } else {
       stage::pad_planar16_blocks(static_cast<const unsigned short*>(P.xpp_src),
                                  static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total,
@@ -460,7 +470,16 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     P.staged = p.staged;
     P.sums = p.sums;
     P.a_vec = octet_vec(P.sa, p.src);
-    P.a_blocks = static_cast<int>(octet_grid(P.sa, p.batch, &P.a_nbx, &P.a_octs));
+    int64_t a_blocks = octet_grid(P.sa, p.batch, &P.a_nbx, &P.a_octs);
+    // One read of an fp32 source for its three parts (octet_parts_block).
+    P.a_all_parts = split && P.sa.split_c > 0 && P.sa.split_n == 3 && P.sa.split_map == kSplitPartsMap &&
+                    P.sa.split_batch == 0 && P.sa.split_pitch % 8 == 0 &&
+                    P.sa.dst_cg == 3 * P.sa.split_pitch && P.sa.pvol == P.sa.in_vol;
+    if (P.a_all_parts) {
+      P.a_octs /= 3;
+      a_blocks /= 3;
+    }
+    P.a_blocks = static_cast<int>(a_blocks);
     total += P.a_blocks;
   }
   if (p.x_oct != nullptr && p.pad != nullptr && p.oct_batch > 0 && p.pad->pvol > 0) {
@@ -482,7 +501,9 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     int dlast = 8;
     for (int i = 0; i < a.rank; ++i)
       if (i == a.rank - 1) dlast = a.dext[i];
-    P.runs = (int64_t)a.batch * a.cout_total * (a.dvol / dlast) * (dlast / 8);
+    P.d_all_parts = split && p.dy_part_map == kSplitPartsMap && a.batch == 3 * p.split_batch;
+    P.runs = (int64_t)(P.d_all_parts ? p.split_batch : a.batch) * a.cout_total * (a.dvol / dlast) *
+             (dlast / 8);
     const int64_t blocks = (P.runs + kThreads - 1) / kThreads;
     P.d_blocks = static_cast<int>(blocks < 2048 ? blocks : 2048);
     total += P.d_blocks;
@@ -504,7 +525,10 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
                                    (p.pp->copies == 2 && p.pp->shift[1] != 1)))
       return hipErrorInvalidValue;
     P.e_nc_copy = static_cast<int>(p.pp_batch * p.pp->channels);
-    P.e_total = p.pp->copies * p.pp_batch * p.pp->channels * (p.pp->pvol / 8);
+    P.e_all_parts = split && p.pp->last_stride == 1 && p.pp_blocks == 3 &&
+                    p.pp_part_map == kSplitPartsMap;
+    P.e_total = p.pp->copies * (P.e_all_parts ? p.split_batch : p.pp_batch) * p.pp->channels *
+                (p.pp->pvol / 8);
     if (P.e_total > 0x7fffffff) return hipErrorInvalidValue;  // 32-bit run indices
     const int64_t per = (int64_t)stage::kPlanarRuns * kThreads;
     P.e_blocks = static_cast<int>((P.e_total + per - 1) / per);

@@ -55,7 +55,6 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
       ck -= A.nchunk;
       ++tc;
     }
-    const int tvol = A.tcount > 1 ? A.k_vol / A.tcount : A.k_vol;  // taps per split tap
     // Tap and channel of the lane's k-group: for the forward convolution (one phase, every
     // tap in row-major order) k-group kk / 8 of the chunk is tap kk / cc, channel kk % cc;
     // the input gradient's phases read the plan's map.
@@ -64,13 +63,13 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
       const int ko = kc * 4 + (lane >> 4);  // k-group: (tap, octet of the chunk)
       tflat = fast_div(ko, A.div_noct);
       chan = (ko - tflat * A.noct) * 8;
-      if (tflat >= tvol) tflat = -1;
+      if (tflat >= A.tvol) tflat = -1;
     } else {
       const int* pe = pmap + ((phase * A.kc_max + kc) * 4 + (lane >> 4)) * 2;
       tflat = pe[0];
       chan = pe[1];
     }
-    if (tflat >= 0) tflat += tc * tvol;
+    if (tflat >= 0) tflat += tc * A.tvol;
     int ci = ck * A.cc + chan + i;
     bool live = m < A.cout_g && tflat >= 0;
     if constexpr (sizeof(S) == 4) {
@@ -329,15 +328,64 @@ __device__ __forceinline__ void octets16_block(const Src* src, unsigned short* d
   }
 }
 
+// The three bf16 parts of 8 fp32 elements as 16-byte units. The split copies are bound by their
+// loads (4-byte ones where rows are short): one read for all three parts instead of one per
+// part took the forward and backward prologues of fp32 [2,24,13,11,10,15] -> 48 channels from
+// 24.5 + 37 to 9.9 + 25 us, of [1,8,8^6] -> 16 from 21 + 103 to 9 + 50 us.
+__device__ __forceinline__ void split_parts8(const float (&v)[8], u32x4 (&w)[3]) {
+#pragma unroll
+  for (int part = 0; part < 3; ++part) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      w[part][k] = bf16_part_bits(v[2 * k], part) |
+                   (static_cast<unsigned>(bf16_part_bits(v[2 * k + 1], part)) << 16);
+  }
+}
+
+// Octet-major copy of an fp32 tensor's three bf16 parts, unpadded (PadArgs of split_n 3: the
+// parts of a group's channels one after the other): block (position run bx, octet o of the
+// channels, image n) reads its eight channels once and writes all three parts.
+__device__ __forceinline__ void octet_parts_block(const float* src, unsigned short* dst,
+                                                  const PadArgs& P, int bx, int o, int n) {
+  const int po = P.split_pitch >> 3;  // octets of one part
+  const int gi = o / po;
+  const int o1 = o - gi * po;
+  const int live = P.split_c - o1 * 8;  // channels from this octet on
+  const float* s = src + ((size_t)n * P.src_channels + gi * P.split_c + o1 * 8) * P.in_vol;
+  unsigned short* d =
+      dst + ((size_t)n * (P.channels >> 3) + gi * (P.dst_cg >> 3) + o1) * P.in_vol * 8;
+  const size_t part_step = (size_t)po * P.in_vol * 8;
+  constexpr int kPer = kOctRun / kThreads;
+  float v[kPer][8];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int p = bx * kOctRun + j * kThreads + static_cast<int>(threadIdx.x);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      v[j][k] = p < P.in_vol && k < live ? s[(size_t)k * P.in_vol + p] : 0.f;
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int p = bx * kOctRun + j * kThreads + static_cast<int>(threadIdx.x);
+    if (p >= P.in_vol) break;
+    u32x4 w[3];
+    split_parts8(v[j], w);
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+      *reinterpret_cast<u32x4*>(d + part * part_step + (size_t)p * 8) = w[part];
+  }
+}
+
 // Zero-padded copy of grad_output: dst[nc][u...] = src[nc][u...] for u inside the output
 // extents, else zero; each thread writes 8 consecutive elements of the last axis (whose
 // padded extent is a multiple of 8). Src = float (split precision): destination image n of
 // A.batch = blocks x split_batch holds part split_map_part(part_map, n / split_batch) of
-// source image n % split_batch.
+// source image n % split_batch; with all_parts (three blocks, parts 0, 1, 2) the runs are
+// those of the source's images, each read once and written to its three part images.
 template <typename Src>
 __device__ __forceinline__ void pad_dy16_blocks(const Src* src, unsigned short* dst,
                                                 const WgradArgs& A, int split_batch,
-                                                unsigned part_map,
+                                                unsigned part_map, bool all_parts,
                                                 int64_t total_runs, int block, int nblocks) {
   const int R = A.rank;
   int dlast = 8, olast = 1;
@@ -359,9 +407,11 @@ __device__ __forceinline__ void pad_dy16_blocks(const Src* src, unsigned short* 
     int64_t snc = nc;
     int part = 0;
     if constexpr (sizeof(Src) == 4) {
-      const int64_t n = nc / A.cout_total, c = nc - n * A.cout_total;
-      snc = (n % split_batch) * A.cout_total + c;
-      part = split_map_part(part_map, static_cast<int>(n / split_batch));
+      if (!all_parts) {
+        const int64_t n = nc / A.cout_total, c = nc - n * A.cout_total;
+        snc = (n % split_batch) * A.cout_total + c;
+        part = split_map_part(part_map, static_cast<int>(n / split_batch));
+      }
     }
     int srow = 0, istr = olast;
     bool ok = true;
@@ -376,6 +426,20 @@ __device__ __forceinline__ void pad_dy16_blocks(const Src* src, unsigned short* 
       }
     }
     const Src* s = src + snc * A.out_vol + srow;
+    if constexpr (sizeof(Src) == 4) {
+      if (all_parts) {
+        float f[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) f[k] = ok && u0 + k < olast ? s[u0 + k] : 0.f;
+        u32x4 w[3];
+        split_parts8(f, w);
+        const int64_t part_step = (int64_t)split_batch * A.cout_total * A.dvol;
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          *reinterpret_cast<u32x4*>(dst + p * part_step + rowd * dlast + u0) = w[p];
+        continue;
+      }
+    }
     auto bits = [&](int e) -> unsigned {
       if (!ok || e >= olast) return 0u;
       if constexpr (sizeof(Src) == 4) {
@@ -583,11 +647,13 @@ __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
 // split_map_part(part_map, s) of every source element. A run's 8 fp32 elements start at
 // element o of
 // the first of three aligned 16-byte chunks (the buffer's per-dword range check reads zero
-// past the source's end).
+// past the source's end). With all_parts (three blocks, parts 0, 1, 2; unit last stride) the
+// runs are those of one block per copy, each read once and written to all three.
 __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsigned short* dst,
                                                         const PlanarPadArgs& P, int64_t total,
                                                         int split_nc, unsigned part_map,
-                                                        int nc_copy, int block) {
+                                                        int nc_copy, bool all_parts,
+                                                        int block) {
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(src), static_cast<short>(0), static_cast<int>(P.src_bytes), 0x00020000);
   const int64_t nbytes = static_cast<int64_t>(P.src_bytes);
@@ -601,11 +667,14 @@ __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsign
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
-    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, nc_copy);
-    // Destination row block s reads source row nc - s * split_nc.
-    const int s = r.nc / split_nc;
-    r.first -= (int64_t)s * split_nc * P.in_vol;
-    part[q] = split_map_part(part_map, s);
+    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, all_parts ? split_nc : nc_copy);
+    part[q] = 0;
+    if (!all_parts) {
+      // Destination row block s reads source row nc - s * split_nc.
+      const int s = r.nc / split_nc;
+      r.first -= (int64_t)s * split_nc * P.in_vol;
+      part[q] = split_map_part(part_map, s);
+    }
     const bool live = t < ntotal && r.lo < r.hi;
     const int64_t chunk = r.first >= 0 ? r.first >> 2 : -((3 - r.first) >> 2);  // floor(/4)
     o[q] = static_cast<int>(r.first - chunk * 4);
@@ -621,15 +690,29 @@ __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsign
     if (t >= ntotal) continue;
     const unsigned d[12] = {c0[q][0], c0[q][1], c0[q][2], c0[q][3], c1[q][0], c1[q][1],
                             c1[q][2], c1[q][3], c2[q][0], c2[q][1], c2[q][2], c2[q][3]};
-    unsigned h[8];
+    float f[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       unsigned x = d[e];
 #pragma unroll
       for (int k = 1; k < 4; ++k)
         if (o[q] == k) x = d[e + k];
-      h[e] = e >= lo[q] && e < hi[q] ? bf16_part_bits(__builtin_bit_cast(float, x), part[q]) : 0u;
+      f[e] = e >= lo[q] && e < hi[q] ? __builtin_bit_cast(float, x) : 0.f;
     }
+    if (all_parts) {
+      // Run t of one block's runs per copy: its three part images lie a block apart.
+      const int64_t block_runs = ntotal / P.copies;
+      const int64_t copy = t / block_runs;
+      unsigned short* dt = dst + (copy * 2 * block_runs + t) * 8;
+      u32x4 w[3];
+      split_parts8(f, w);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dt + p * block_runs * 8) = w[p];
+      continue;
+    }
+    unsigned h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = bf16_part_bits(f[e], part[q]);
     *reinterpret_cast<u32x4*>(dst + (size_t)t * 8) =
         u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
   }
