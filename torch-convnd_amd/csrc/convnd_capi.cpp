@@ -1763,6 +1763,12 @@ ForwardSetup setup_forward(const Geom& g, convnd_hip_dtype dt) {
   return cached_plan(cache, plan_key(g, dt, 0), [&] { return make_forward(g, dt); });
 }
 
+// The input gradient's staging pass can add grad_output's channel sums: 16-bit data, and fp32
+// read once for its three parts.
+bool staging_sums(const IgemmPlan& dg, convnd_hip_dtype dt) {
+  return is_half(dt) || (dt == CONVND_HIP_FLOAT32 && dg.args.parts == 3);
+}
+
 BackwardSetup make_backward(const Geom& g, convnd_hip_dtype dt, bool gi, bool gw, bool gb) {
   BackwardSetup b;
   const int64_t es = element_size(dt);
@@ -1797,7 +1803,7 @@ BackwardSetup make_backward(const Geom& g, convnd_hip_dtype dt, bool gi, bool gw
   if (gb) {
     // Partial sums of the bias gradient: per channel, kBiasChunks doubles on the standalone
     // path or one float per 64-position tile when they come with the channels-last copy.
-    const size_t fused = (gi && b.dg.ok && is_half(dt))
+    const size_t fused = (gi && b.dg.ok && staging_sums(b.dg, dt))
                              ? (size_t)octet_sum_blocks(g.batch, g.out_vol) * sizeof(float)
                              : 0;
     // Or one float per position chunk of the channel-major weight gradient, which adds them.
@@ -2194,7 +2200,7 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
     if (dx_tables == nullptr && !b.dg.or_direct) return CONVND_HIP_LAUNCH_FAILED;
     mfma_dx = dx_tables != nullptr;  // (an or_direct plan without tables: the direct kernel)
   }
-  const bool fused_bias = gb && !cm_bias && !tiny_bias && mfma_dx && is_half(dtype);
+  const bool fused_bias = gb && !cm_bias && !tiny_bias && mfma_dx && staging_sums(b.dg, dtype);
   if (gb && !fused_bias && !cm_bias && !tiny_bias) {
     st = hip_check(launch_grad_bias(dtype, g.batch, g.out_channels, g.out_vol, grad_output,
                                     grad_bias, reinterpret_cast<float*>(ws + b.off_bias),
@@ -2212,7 +2218,7 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
   PrologueParts pp;
   // Channel sums from the octet-major copy's blocks, or from a part of their own where the GEMM
   // stages grad_output itself or the copy holds zero channels besides grad_output's.
-  const bool own_sums = mfma_dx && (b.dg.args.direct != 0 || b.dg.padded);
+  const bool own_sums = mfma_dx && is_half(dtype) && (b.dg.args.direct != 0 || b.dg.padded);
   if (mfma_dx) {
     DA = b.dg.args;
     DA.tables = dx_tables->dev;

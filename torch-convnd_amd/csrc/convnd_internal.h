@@ -465,7 +465,7 @@ int64_t prologue_sum_blocks(int64_t batch, int64_t volume);
 // (null pointers skip it) and runs on its own range of workgroups:
 //   weights:    packing for the implicit GEMM (reads ig->tables);
 //   GEMM input: octet-major copy of src with geometry and channel map sa (no padding),
-//               with optional channel sums (16-bit source);
+//               with optional channel sums (16-bit source, or fp32 in three parts);
 //   octets:     zero-padded octet-major input for the weight gradient (pad);
 //   dy_pad:     grad_output padded to whole boxes for the weight gradient (wg);
 //   planar pad: zero-padded channels-first input for the channel-major weight gradient

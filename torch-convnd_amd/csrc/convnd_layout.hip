@@ -152,7 +152,8 @@ void prologue_kernel(DevPrologue P) {
     if constexpr (SPLIT) {
       if (P.a_all_parts) {
         stage::octet_parts_block(static_cast<const float*>(P.src),
-                                 static_cast<unsigned short*>(P.staged), P.sa, bx, o, n);
+                                 static_cast<unsigned short*>(P.staged), P.sa, bx, o, n, P.a_nbx,
+                                 P.sums, P.a_nbx * (P.a_blocks / (P.a_nbx * P.a_octs)), &smem);
         return;
       }
     }
@@ -464,7 +465,7 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
   }
   if (p.staged != nullptr && p.sa != nullptr && p.batch > 0 && p.sa->pvol > 0) {
     if (!octet_ok(*p.sa, p.batch)) return hipErrorInvalidValue;
-    if (p.sums != nullptr && (split || p.sa->pvol != p.sa->in_vol)) return hipErrorInvalidValue;
+    if (p.sums != nullptr && p.sa->pvol != p.sa->in_vol) return hipErrorInvalidValue;
     P.sa = *p.sa;
     P.src = p.src;
     P.staged = p.staged;
@@ -475,6 +476,7 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     P.a_all_parts = split && P.sa.split_c > 0 && P.sa.split_n == 3 && P.sa.split_map == kSplitPartsMap &&
                     P.sa.split_batch == 0 && P.sa.split_pitch % 8 == 0 &&
                     P.sa.dst_cg == 3 * P.sa.split_pitch && P.sa.pvol == P.sa.in_vol;
+    if (p.sums != nullptr && split && !P.a_all_parts) return hipErrorInvalidValue;
     if (P.a_all_parts) {
       P.a_octs /= 3;
       a_blocks /= 3;

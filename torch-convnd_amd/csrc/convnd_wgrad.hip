@@ -398,7 +398,7 @@ hipError_t launch_wgrad_reduce(convnd_hip_dtype dtype, int mb, const WgradArgs& 
   const int64_t rblocks = (nslots + kThreads - 1) / kThreads;
   BiasSums bs{bias_sums, db, static_cast<int>(nsum), static_cast<int>(channels)};
   const int64_t bblocks = bias_sums != nullptr ? channels : 0;
-  if (bias_sums != nullptr && (dtype == CONVND_HIP_FLOAT32 || nsum > INT32_MAX)) return hipErrorInvalidValue;
+  if (bias_sums != nullptr && nsum > INT32_MAX) return hipErrorInvalidValue;
   if (rblocks + bblocks == 0) return hipSuccess;
   if (rblocks + bblocks > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid(static_cast<unsigned>(rblocks + bblocks));
