@@ -288,7 +288,7 @@ constexpr int kMaxCopies = 2 * kMaxLastStride;
 // read from a zero-padded channels-first copy of the input: every B fragment is one aligned
 // LDS read, the last-axis tap shift applied once when the run is loaded.
 struct WgradCmArgs {
-  const void* x;        // zero-padded input [N][cin_total][pe...] (pe: WgradCmArgs::pe)
+  const void* x;        // zero-padded input copies [copy][N][cin_total][pe...] (pe: WgradCmArgs::pe)
   const void* dy;       // grad_output [N][cout_total][dvol] (the output, or padded to boxes)
   float* partial;       // per-lane accumulator vectors, see wgrad_cm_partial_slots
   unsigned x_bytes, dy_bytes;  // buffer sizes (offsets at or past them read zero)
@@ -440,8 +440,9 @@ hipError_t ensure_dynamic_lds(size_t bytes) {
 // input), u_a < pe[a], where destination channel c is channel cc = c % dst_cg of group
 // gi = c / dst_cg: source channel gi*src_cg + cc (zero past src_cg), or with split_c > 0 part
 // split_map_part(split_map, s) of source channel gi*split_c + c for cc = s*split_pitch + c
-// (fp32 source, split-precision GEMM input; zero for c >= split_c and past split_n copies). With split_batch > 0 (fp32 source) destination image n holds
-// part split_data_part(n / split_batch) of source image n % split_batch.
+// (fp32 source, split-precision GEMM input; zero for c >= split_c and past split_n copies).
+// With split_batch > 0 (fp32 source) destination image n holds part
+// split_data_part(n / split_batch) of source image n % split_batch.
 struct PadArgs {
   int rank, channels;       // destination channels (groups x dst_cg)
   int src_channels;         // source channels per image

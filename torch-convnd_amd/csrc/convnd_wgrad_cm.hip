@@ -1,5 +1,5 @@
 // Channel-major MFMA weight gradient (gfx950, 16x16x32 bf16/fp16 -> fp32) of the N-d
-// convolution, for a unit stride along the last axis.
+// convolution.
 //
 // dW[co][ci][t] = sum over images n and output positions o of dY[n][co][o] * X[n][ci][o*s - p
 // + t*d]: a GEMM with M = output channels, N = columns (input channel, tap) in the weight
@@ -11,8 +11,11 @@
 //     out in the weight layout's order, so only the last tile of the last chunk is partial.
 //   * Per box of positions (an "item") the workgroup stages, for each input channel of its
 //     chunk and each halo row (all axes but the last), the 16-byte runs of 8 consecutive
-//     positions that the last-axis taps read, each one 16-byte load (at a 2-byte-aligned
-//     offset) from a zero-padded channels-first copy of the input. A lane's column (channel,
+//     positions that the last-axis taps read, each one 16-byte load from a zero-padded
+//     channels-first copy of the input. Direct-to-LDS loads at a 2-byte offset move one lane
+//     per clock, at a 4-byte offset 3.7, so taps of odd offset read a second copy shifted by one
+//     element, and a strided last axis has a copy per stride phase ([1,8,8^6] -> 16 channels
+//     bf16: 157 -> 123 us; fp32: 836 -> 665 us). A lane's column (channel,
 //     tap) is then a fixed LDS offset and a K32 step (four runs of 8 positions) adds a
 //     per-run offset: no transposes.
 //   * grad_output runs [channel][box positions], from grad_output itself when the boxes tile
@@ -21,9 +24,9 @@
 //   * Loads go straight to LDS (no registers, no stores): two item buffers in LDS alternate,
 //     the MFMAs of one item running while the next item's loads land in the other buffer.
 //     One workgroup per CU: four waves (one per SIMD), or eight (two per SIMD) that split
-//     each item's K steps between the two waves of a column set. Each workgroup writes fp32 partial sums of
-//     its range of items; a second pass adds them in a fixed order into the weight layout
-//     (deterministic, no atomics).
+//     each item's K steps between the two waves of a column set. Each workgroup writes fp32
+//     partial sums of its range of items; a second pass adds them in a fixed order into the
+//     weight layout (deterministic, no atomics).
 
 #include "convnd_internal.h"
 #include "convnd_stage.h"
