@@ -1,0 +1,79 @@
+"""Calls whose plan cannot have its geometry tables (without a GPU: every call), on the host.
+
+Without a device the tables of a plan cannot be uploaded, as they cannot on the first call of a
+geometry under stream capture: a plan that may run on the direct kernels instead goes on to
+them, and its call then fails at the first launch, which the message names. Nothing runs, so the
+buffers are addresses that are never read. Skipped where a GPU is present.
+"""
+
+import ctypes
+import math
+import random
+
+import pytest
+import torch
+
+from torch_convnd import _capi
+from torch_convnd._toolchain import HIP_LIBRARY
+
+pytestmark = pytest.mark.skipif(torch.cuda.is_available(), reason="the calls would run on the GPU")
+
+NOWHERE = ctypes.c_void_p(0x10000)
+
+
+@pytest.fixture(scope="module")
+def lib():
+    if not HIP_LIBRARY.exists():
+        pytest.skip("native libraries not built (python __graft_entry__.py)")
+    return _capi.bind(ctypes.CDLL(str(HIP_LIBRARY)))
+
+
+def out_shape(lib, problem, x_shape, w_shape):
+    sizes = (ctypes.c_int64 * _capi.MAX_RANK)()
+    assert lib.convnd_hip_validate(ctypes.byref(problem), 2, 1 << 62, sizes) == _capi.SUCCESS
+    return (x_shape[0], w_shape[0], *sizes[: len(x_shape) - 2])
+
+
+def small_problems(count, seed):
+    """16-bit layers of few output positions, or of halos near the size of LDS."""
+    rng = random.Random(seed)
+    for _ in range(count):
+        rank = rng.randint(1, 6)
+        top = {1: 60, 2: 20, 3: 16, 4: 11, 5: 11, 6: 6}[rank]
+        kernel = [rng.randint(2, 4 if rank < 5 else 3) for _ in range(rank)]
+        stride = [rng.choice((1, 1, 2, 3))] * rank
+        size = [max(k, rng.randint(2, top)) for k in kernel]
+        cin, cout = rng.choice((8, 16, 32, 5)), rng.choice((8, 16, 64, 3))
+        yield (rng.choice((1, 2)), cin, *size), (cout, cin, *kernel), tuple(stride), (1,) * rank, (1,) * rank, 1
+
+
+CHANNELS_LAST_CASES = [
+    # Fewer output positions than a tile, and a halo that no box of 128 positions fits.
+    ((1, 32, 2, 3, 2, 4), (32, 32, 3, 3, 3, 3), (1,) * 4, (1,) * 4, (1,) * 4, 1),
+    ((1, 8, 4, 8, 3, 7, 7, 4), (8, 8, 3, 5, 2, 4, 3, 3), (3, 1, 3, 2, 1, 1), (1, 2, 1, 2, 1, 1), (1,) * 6, 1),
+    ((1, 16, 13, 10, 11, 11, 8), (8, 16, 3, 3, 3, 3, 3), (2,) * 5, (1,) * 5, (1,) * 5, 1),
+    *small_problems(150, 3),
+]
+
+
+def test_channels_last_forward_stays_inside_its_workspace(lib):
+    """A call that goes on to its channels-first copies writes them behind the plan's own
+    workspace: the size that it asks for has to hold them."""
+    copied = staged = 0
+    for args in CHANNELS_LAST_CASES:
+        problem = _capi.Problem.make(*args)
+        ref = ctypes.byref(problem)
+        x_bytes = 2 * math.prod(args[0])
+        y_bytes = 2 * math.prod(out_shape(lib, problem, *args[:2]))
+        plan = lib.convnd_hip_forward_workspace_size(ref, _capi.BFLOAT16)
+        for layout, copies in ((_capi.CHANNELS_LAST, x_bytes + y_bytes), (_capi.CHANNELS_LAST_INPUT, x_bytes)):
+            need = lib.convnd_hip_forward_workspace_size_layout(ref, _capi.BFLOAT16, layout)
+            status = lib.convnd_hip_forward_layout(ref, _capi.BFLOAT16, layout, 0, NOWHERE, NOWHERE, None, NOWHERE,
+                                                   NOWHERE, need, None)
+            assert status == _capi.LAUNCH_FAILED
+            if "channels-last input copy" in lib.convnd_hip_last_error().decode():
+                assert need >= plan + copies, (args, layout)
+                copied += 1
+            else:
+                staged += 1
+    assert copied > 50 and staged > 0, (copied, staged)

@@ -2106,12 +2106,17 @@ bool igemm_stages_cl(const IgemmPlan& p) {
 
 bool forward_reads_cl(const ForwardSetup& f) { return igemm_stages_cl(f.ig); }
 
+// Whether a channels-last forward may run on channels-first copies: always, unless its GEMM reads
+// channels-last input and cannot become the direct kernel's (or_direct plans do without tables;
+// the copies' room is part of the workspace either way).
+bool forward_may_copy(const ForwardSetup& f) { return !forward_reads_cl(f) || f.ig.or_direct; }
+
 size_t tensor_bytes(int64_t batch, int64_t channels, int64_t volume, convnd_hip_dtype dt) {
   return align_up(static_cast<size_t>(batch * channels * volume * element_size(dt)));
 }
 
 size_t cl_forward_extra(const Geom& g, convnd_hip_dtype dt, const ForwardSetup& f) {
-  if (forward_reads_cl(f)) return 0;
+  if (!forward_may_copy(f)) return 0;
   return tensor_bytes(g.batch, g.channels, g.in_vol, dt) +
          tensor_bytes(g.batch, g.out_channels, g.out_vol, dt);
 }
@@ -2563,7 +2568,7 @@ size_t convnd_hip_forward_workspace_size_layout(const convnd_hip_problem* proble
   const ForwardSetup f = setup_forward(g, dtype);
   if (layout == CONVND_HIP_CHANNELS_LAST)
     return align_up(f.bytes) + cl_forward_extra(g, dtype, f);
-  if (layout == CONVND_HIP_CHANNELS_LAST_INPUT && !forward_reads_cl(f))
+  if (layout == CONVND_HIP_CHANNELS_LAST_INPUT && forward_may_copy(f))
     return align_up(f.bytes) + tensor_bytes(g.batch, g.channels, g.in_vol, dtype);
   return f.bytes;
 }
