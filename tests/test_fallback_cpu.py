@@ -77,3 +77,48 @@ def test_channels_last_forward_stays_inside_its_workspace(lib):
             else:
                 staged += 1
     assert copied > 50 and staged > 0, (copied, staged)
+
+
+# dtype, pass (0 forward, 1 input gradient), shapes: the halo of one octet in power-of-two boxes of
+# 128 positions (64 from four output-channel tiles on) just does not fit LDS with its tables and pitches,
+# reaches past 64 rows or 255 columns, or there are too few positions.
+NO_PLAIN_PLAN = [
+    ("bf16", 0, ((1, 16, 11, 11, 11, 11, 11), (32, 16, 3, 3, 3, 3, 3), (2,) * 5, (1,) * 5, (1,) * 5, 1)),
+    ("bf16", 0, ((1, 8, 9, 9, 9, 9, 9), (16, 8, 3, 3, 3, 3, 3), (2,) * 5, (1,) * 5, (1,) * 5, 1)),
+    ("bf16", 0, ((3, 48, 8, 7, 4, 8, 13), (24, 48, 3, 3, 3, 3, 3), (2,) * 5, (1,) * 5, (1,) * 5, 1)),
+    ("bf16", 0, ((1, 32, 2, 3, 2, 4), (32, 32, 3, 3, 3, 3), (1,) * 4, (1,) * 4, (1,) * 4, 1)),
+    ("fp32", 0, ((1, 20, 18, 12, 18, 16), (8, 5, 4, 4, 5, 3), (1, 2, 3, 1), (1, 3, 6, 1), (1, 2, 3, 1), 4)),
+    ("fp32", 0, ((2, 64, 4, 9, 10, 11, 5), (1, 64, 3, 3, 3, 3, 3), (1,) * 5, (1, 2, 0, 1, 4), (2, 1, 1, 3, 3), 1)),
+    ("fp32", 0, ((1, 192, 200), (64, 48, 3), (2,), (0,), (1,), 4)),
+    ("fp32", 1, ((1, 2, 2, 2, 2, 2, 3, 2, 3), (16, 2, 3, 3, 2, 3, 3, 2, 3), (1,) * 7, (1, 1, 0, 1, 0, 1, 0), (1,) * 7, 1)),
+]
+# Just inside the same line.
+PLAIN_PLAN = [
+    ("bf16", 1, ((1, 2, 5, 5, 5, 5, 5, 5), (32, 2, 3, 3, 3, 3, 3, 3), (1,) * 6, (1,) * 6, (1,) * 6, 1)),
+    ("bf16", 1, ((1, 96, 1, 7, 1, 3, 4, 5), (32, 96, 3, 3, 3, 3, 3, 3), (1,) * 6, (1, 0, 1, 0, 2, 1), (1,) * 6, 1)),
+    ("fp32", 0, ((1, 12, 3, 5, 1, 2, 2, 2, 5), (128, 3, 3, 3, 3, 3, 1, 3, 1), (1,) * 7, (0, 2, 1, 1, 0, 1, 0), (1,) * 7, 4)),
+    ("fp32", 0, ((2, 4, 2, 10, 3, 5, 11), (80, 2, 3, 3, 3, 2, 4), (2,) * 5, (1, 1, 1, 0, 1), (1,) * 5, 2)),
+    ("fp32", 1, ((3, 32, 5, 5, 2, 7, 2, 2, 6), (64, 8, 3, 3, 3, 3, 1, 3, 2), (1,) * 7, (0, 0, 2, 2, 0, 1, 0), (1,) * 7, 4)),
+]
+
+
+@pytest.mark.parametrize(("dtype", "which", "args"), NO_PLAIN_PLAN + PLAIN_PLAN)
+def test_calls_without_tables(lib, dtype, which, args):
+    """Without tables, an MFMA plan whose problem has no plain plan goes on to the direct kernel
+    (which such problems had before); any other fails for its tables."""
+    dt = {"bf16": _capi.BFLOAT16, "fp32": _capi.FLOAT32}[dtype]
+    problem = _capi.Problem.make(*args)
+    ref = ctypes.byref(problem)
+    assert lib.convnd_hip_plan_name(ref, dt, which) == b"mfma"
+    if which == 0:
+        need = lib.convnd_hip_forward_workspace_size(ref, dt)
+        status = lib.convnd_hip_forward(ref, dt, NOWHERE, NOWHERE, None, NOWHERE, NOWHERE, need, None)
+    else:
+        need = lib.convnd_hip_backward_workspace_size(ref, dt, 1, 0, 0)
+        status = lib.convnd_hip_backward(ref, dt, NOWHERE, NOWHERE, NOWHERE, NOWHERE, None, None, NOWHERE, need, None)
+    assert status == _capi.LAUNCH_FAILED
+    message = lib.convnd_hip_last_error().decode()
+    if (dtype, which, args) in NO_PLAIN_PLAN:
+        assert message.startswith("direct "), message
+    else:
+        assert message.startswith("geometry tables"), message

@@ -251,7 +251,7 @@ struct IgemmPlan {
   // Problems that calls without scratch or geometry tables (the allocation-free entry beyond
   // its scratch, a first call under stream capture) run on the direct kernels, which need
   // neither, instead of being refused: padded ones, wide or large split-precision ones, and
-  // halos that only fit LDS in odd boxes or with split taps.
+  // halos that only fit LDS in odd boxes or with split taps (plain_plan_exists).
   bool or_direct = false;
   double conflict = 1;      // lanes per 16-byte bank slot in a B-fragment read (1 = none)
   double cost = 0.0;
@@ -387,23 +387,6 @@ std::vector<IgemmBoxShape> igemm_boxes(int R, const int* J, const int* sigma, co
   return out;
 }
 
-// Whether some box of exactly box_vol positions with power-of-two extents has a halo (of one octet)
-// that fits LDS.
-bool pow2_box_fits(int R, const int* J, const int* sigma, const int* span, int box_vol) {
-  int limit[kFastRank];
-  for (int a = 0; a < R; ++a) {
-    limit[a] = 1;
-    while (limit[a] < J[a] && limit[a] < box_vol) limit[a] *= 2;
-  }
-  bool fits = false;
-  for_each_box(R, limit, box_vol, [&](const int* b) {
-    int64_t bytes = 16;
-    for (int a = 0; a < R; ++a) bytes *= (b[a] - 1) * sigma[a] + span[a] + 1;
-    fits = fits || bytes <= kLdsBudget;
-  });
-  return fits;
-}
-
 // Halo pitches: hpitch[R-1] = 1 and hpitch[a] = hpitch[a+1] * padded extent of axis a+1.
 // The two innermost padded extents are searched (0..15 extra positions each), smallest plane
 // first; returned are the smallest plane and every larger one with fewer bank conflicts than
@@ -470,6 +453,90 @@ std::vector<IgemmPitches> choose_pitches(int R, const int* sigma, const IgemmBox
     }
   }
   return out;
+}
+
+// Whether a plain plan exists: a power-of-two box of 64 (from four output-channel tiles on), 128 or
+// 256 positions whose halo of one octet, with the pitches of the fewest bank conflicts, row table,
+// box offsets and tap offsets (`ntaps` taps) fits LDS. Problems without one could only run on the
+// direct kernels before boxes of any extents and split taps, so their calls without tables or
+// scratch still do (IgemmPlan::or_direct): the line is exact, so that no call that was taken is
+// refused for a plan that has become faster.
+bool plain_plan_exists(int R, const int* J, const int* sigma, const int* span, int64_t ntaps,
+                       int mtiles) {
+  auto aligned = [](int64_t bytes) { return static_cast<int64_t>(align_up(static_cast<size_t>(bytes))); };
+  const int64_t taps = aligned(16 * (((ntaps * 8 + 31) / 32 + kTapPad + 3) / 4 * 4));
+  bool fits = false;
+  for (int box_vol = mtiles >= 4 ? 64 : 128; box_vol <= 256; box_vol *= 2) {
+    int limit[kFastRank];
+    for (int a = 0; a < R; ++a) {
+      limit[a] = 1;
+      while (limit[a] < J[a] && limit[a] < box_vol && (R <= 4 || limit[a] < 64)) limit[a] *= 2;
+    }
+    for_each_box(R, limit, box_vol, [&](const int* b) {
+      if (fits) return;
+      int hext[kFastRank];
+      int64_t hvol = 1, rows = 1;
+      for (int a = 0; a < R; ++a) {
+        const int64_t h = (int64_t)(b[a] - 1) * sigma[a] + span[a] + 1;
+        if (h > (a < R - 1 ? 64 : 255)) return;
+        hext[a] = static_cast<int>(h);
+        hvol *= h;
+        if (a < R - 1) rows *= h;
+        if (hvol * 16 > kLdsBudget) return;
+      }
+      const int64_t room = kLdsBudget - aligned(rows * 8) - aligned(box_vol * 4) - taps;
+      auto plane_fits = [&](int64_t positions) { return aligned(positions * 16) <= room; };
+      if (!plane_fits(hvol)) return;
+      // Pitches as choose_pitches searches them, by the worst block of 16 positions.
+      const int mid = R >= 3 ? R - 2 : -1, last = R >= 2 ? R - 1 : -1;
+      struct Candidate {
+        int64_t size;
+        int p1, p2;
+      };
+      std::vector<Candidate> cands;
+      for (int p1 = 0; p1 <= (last >= 0 ? 15 : 0); ++p1)
+        for (int p2 = 0; p2 <= (mid >= 0 ? 15 : 0); ++p2) {
+          int64_t size = 1;
+          for (int a = 0; a < R; ++a)
+            size *= hext[a] + (a == last ? p1 : 0) + (a == mid ? p2 : 0);
+          cands.push_back({size, p1, p2});
+        }
+      std::stable_sort(cands.begin(), cands.end(),
+                       [](const Candidate& x, const Candidate& y) { return x.size < y.size; });
+      if (plane_fits(cands.back().size)) {
+        fits = true;
+        return;
+      }
+      int best = 1 << 30;
+      int64_t chosen = hvol;
+      for (const Candidate& c : cands) {
+        int pitch[kFastRank];
+        pitch[R - 1] = 1;
+        for (int a = R - 2; a >= 0; --a)
+          pitch[a] = pitch[a + 1] * (hext[a + 1] + (a + 1 == last ? c.p1 : 0) + (a + 1 == mid ? c.p2 : 0));
+        int worst = 1;
+        for (int q0 = 0; q0 < box_vol && worst < best; q0 += 16) {
+          int count[16] = {0};
+          for (int q = q0; q < q0 + 16; ++q) {
+            int r = q, off = 0;
+            for (int a = R - 1; a >= 0; --a) {
+              off += r % b[a] * sigma[a] * pitch[a];
+              r /= b[a];
+            }
+            worst = std::max(worst, ++count[off & 15]);
+          }
+        }
+        if (worst < best) {
+          best = worst;
+          chosen = c.size;
+          if (best == 1) break;
+        }
+      }
+      fits = plane_fits(chosen);
+    });
+    if (fits) break;
+  }
+  return fits;
 }
 
 // Optional launch-plan override for tuning sweeps, read once per process from
@@ -892,7 +959,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     IgemmArgs& A = plan.args;
     plan.padded = padded;
     plan.or_direct = padded || wide || (split && !staged_fits(gemm_cin)) ||
-                     !pow2_box_fits(R, J, sigma, span, mtiles >= 4 ? 64 : 128);
+                     !plain_plan_exists(R, J, sigma, span, ntaps_max, mtiles);
     plan.wpk_elems = (size_t)A.nphase * A.groups * A.tcount * A.nchunk * A.kc_max * A.parts * A.mtiles_padded * 64 * 8;
     plan.staged_elems = (size_t)A.batch * A.in_vol * A.cin_total;
     // Byte offsets into the staged operand are 32-bit (buffer loads, an offset of 0xffffffe0
