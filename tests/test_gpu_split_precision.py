@@ -1,0 +1,84 @@
+"""Precision of fp32 layers that run on bf16 parts where fp32 products of the direct kernels served
+before (marked ``gpu``): no larger error against float64 than those products' sums have.
+
+A sum of n products added one by one, each addition rounded to fp32, has a relative error
+(2-norm over many outputs) of about r * sqrt(n / 2) for terms of zero mean and r * sqrt(n / 3)
+for terms of one sign, with r = 2^-23.5 / sqrt(12), the root mean square of one rounding: the
+partial sum at step k carries sqrt(k / n) or k / n of the result. Six truncated part products
+in one accumulator are ten times further off on same-sign data (1.4e-5 against 1.1e-6 at
+n = 7776) and twice as far on sparse data.
+"""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+import helpers
+from torch_convnd import _build, _capi, conv_nd, load_native
+
+pytestmark = pytest.mark.gpu
+
+ROUNDING = 2.0**-23.5 / math.sqrt(12.0)
+SPARSE = 0.004  # share of non-zero inputs
+
+# x shape, w shape, stride, passes on eight products (y, dx, dw), operand layout of the forward
+CASES = {
+    "wide": ((1, 72, 4, 4, 4, 5), (80, 72, 3, 3, 3, 3), 1, ("y", "dx"), 3),
+    "few_positions": ((1, 32, 2, 3, 2, 4), (33, 32, 3, 3, 3, 3), 1, ("y", "dx"), 3),
+    "strided_rank5": ((1, 16, 7, 7, 7, 7, 9), (40, 16, 3, 3, 3, 3, 3), 2, ("y",), 3),
+    # The planes of three parts fit LDS in no box: copies of the channels, whole octets or not.
+    "copies": ((1, 8, 4, 4, 4, 4, 5, 6), (14, 8, 3, 3, 3, 3, 3, 3), 2, ("y",), 1),
+    "copies_odd": ((2, 3, 4, 5, 4, 5, 4, 5), (8, 3, 3, 3, 3, 3, 3, 3), 2, ("y",), 1),
+}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def native():
+    load_native()
+
+
+def draw(kind, shape, generator):
+    if kind == "same_sign":
+        return torch.rand(shape, generator=generator) + 2.0**-20
+    x = torch.randn(shape, generator=generator)
+    if kind == "sparse":
+        x = torch.where(torch.rand(shape, generator=generator) < SPARSE, x, torch.zeros(()))
+    return x
+
+
+def bound(kind, n):
+    """One rounding of the result at least, and a tenth for the scatter of the estimate."""
+    terms = n / 3 if kind == "same_sign" else (SPARSE * n if kind == "sparse" else n) / 2
+    return 1.1 * ROUNDING * math.sqrt(terms + 1)
+
+
+@pytest.mark.parametrize("kind", ["dense", "same_sign", "sparse"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_split_products_are_no_further_off_than_fp32_products(name, kind):
+    x_shape, w_shape, stride, passes, parts = CASES[name]
+    rank = len(x_shape) - 2
+    args = ((stride,) * rank, (1,) * rank, (1,) * rank, 1)
+    print(f"[precision] {name} {kind} x={x_shape} w={w_shape}", flush=True)
+    lib = _build.hip_library()
+    assert lib.convnd_hip_plan_check(ctypes.byref(_capi.Problem.make(x_shape, w_shape, *args)),
+                                     _capi.FLOAT32) == _capi.SUCCESS
+    plans = dict(zip(("y", "dx", "dw"), _capi.plan_details(lib, x_shape, w_shape, *args, torch.float32)))
+    assert plans["y"]["parts"] == parts, plans["y"]
+    for p in passes:
+        assert plans[p].get("products") == 8 or (p == "dw" and plans[p]["kernel"] == "mfma_wgrad_cm"), plans[p]
+    g = torch.Generator().manual_seed(81)
+    x = draw(kind, x_shape, g)
+    w = draw("same_sign" if kind == "same_sign" else "dense", w_shape, g)
+    ref_y = helpers.oracle_forward(x, w, None, *args)
+    dy = draw(kind, ref_y.shape, g)
+    ref_dx, ref_dw, _ = helpers.oracle_backward(dy, x, w, *args)
+    dev = [t.cuda().requires_grad_() for t in (x, w)]
+    y = conv_nd(dev[0], dev[1], None, *args, backend="native")
+    dx, dw = torch.autograd.grad(y, dev, dy.cuda())
+    taps = math.prod(w_shape[2:])
+    for p, got, ref, n in (("y", y, ref_y, w_shape[1] * taps), ("dx", dx, ref_dx, w_shape[0] * taps)):
+        if p in passes:
+            error = ((got.detach().double().cpu() - ref).norm() / ref.norm()).item()
+            assert error <= bound(kind, n), (p, error, bound(kind, n))

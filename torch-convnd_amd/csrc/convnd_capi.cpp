@@ -687,6 +687,14 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     }
   }
   const int mtiles = (gemm_cout + 15) / 16;
+  const bool plain = plain_plan_exists(R, J, sigma, span, ntaps_max, mtiles);
+  // Split-precision problems that the direct kernels' fp32 products served before keep that
+  // precision: eight products per K step from the three parts, the cross products in accumulators
+  // of their own (or, as copies, added before the large one's). With six in one accumulator, what is
+  // truncated or lost beside a large sum shows. Relative error (2-norm) of 96 -> 96 channels, 3^4
+  // taps on 8^4, for dense / same-sign / sparse data: direct 1.4e-6 / 1.1e-6 / 6.9e-8, six
+  // 1.3e-6 / 1.4e-5 / 1.6e-7, eight 4.9e-7 / 4.0e-7 / 3.1e-8; time 10.5 ms, 80 us, 90 us.
+  const bool eight = split && (wide || !staged_fits(gemm_cin) || !plain);
   // Direct staging (16-bit data): the kernel reads the caller's channels-first tensor and
   // double-buffers the chunk halos; otherwise (split-precision fp32, or halos too large to
   // double-buffer) a prologue copies the operand octet-major first, which costs its HBM
@@ -703,7 +711,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     if (filter.nbuf != 2) staging_options.push_back({true, 1});
   }
   if (filter.ds != 1 && filter.nbuf != 2) staging_options.push_back({false, 1});
-  // Operand layouts of split precision (IgemmArgs::parts): the parts once each, or the six
+  // Operand layouts of split precision (IgemmArgs::parts): the parts once each, or the
   // copies as one K dimension, whose few channels fill whole octets better (3 channels: 24
   // channels along K against 6 products x 8). Channel chunk: 1, 2, 3, 4, 6, 8, 12 or 16 octets dividing
   // the channels along K.
@@ -724,15 +732,19 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     const int nbuf = staging.second;
     const int mb = tile[0], nb = tile[1], wm = tile[2], wn = waves / wm;
     // Eight-wave workgroups (one per CU, two waves per SIMD) exist for direct staging.
-    if ((waves == 8 && !direct) || !igemm_tile_supported(mb, nb, wm, waves, parts)) continue;
+    const int products = split ? (eight ? 8 : kSplit) : 1;
+    if ((waves == 8 && !direct) || !igemm_tile_supported(mb, nb, wm, waves, parts, products)) continue;
     if (filter.parts && filter.parts != parts) continue;
-    const int kcin = parts == 3 ? real_octs * 8 : gemm_cin;  // channels along K
-    const int products = parts == 3 ? kSplit : 1;            // MFMAs per K32 step and fragment pair
-    const int staged_cin = parts == 3 ? 3 * kcin : gemm_cin; // staged channels per group
+    const int step_mfmas = parts == 3 ? products : 1;  // per K32 step and fragment pair
+    // Channels along K, and those of one copy.
+    const int copy_cin = parts == 3 || eight ? real_octs * 8 : real_cin;
+    const int kcin = parts == 3 ? copy_cin : (eight ? products * copy_cin : gemm_cin);
+    const int staged_cin = parts * kcin;  // staged channels per group
     if ((split || padded) && !staged_fits(staged_cin)) continue;
-    // Six copies: few channels, up to the width that always used them.
-    if (parts == 1 && wide) continue;
-    if (parts == 3 && real_cin < 3) continue;
+    // Six copies: few channels, up to the width that always used them. Eight: where no box holds
+    // the planes of three parts.
+    if (split && parts == 1 && (wide || (eight && plan.ok && plan.args.parts == 3))) continue;
+    if (split && parts == 3 && real_cin < 3 && !eight) continue;
     if (filter.waves && filter.waves != waves) continue;
     // Cover the output channels without idle waves: the waves' M extent may exceed the
     // channel count by less than one wave's share.
@@ -746,6 +758,8 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     for (const int noct : {16, 12, 8, 6, 4, 3, 2, 1}) {
       const int cc = noct * 8;
       if (kcin % cc != 0 || (filter.cc && filter.cc != cc)) continue;
+      // (A chunk of eight copies holds channels of one product: see IgemmArgs::taps_inner.)
+      if (eight && copy_cin % cc != 0) continue;
       const int planes = parts * noct;  // octet planes of a chunk
       const int64_t nchunk = kcin / cc;
       // Split taps (IgemmArgs::tsplit), with the octet-major copy: axes of several taps that
@@ -819,7 +833,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           // wave's own load-to-use latency, blended towards the largest.
           const double lds_factor = std::max(1.0 + 0.145 * (conflict - 1.0), noct == 1 ? 1.34 : 1.0);
           const double cu_waves = double(occ) * waves;
-          const double mfma = products * mb * nb * 16.0 * 1.03 * simd_waves;
+          const double mfma = step_mfmas * mb * nb * 16.0 * 1.03 * simd_waves;
           const double ldsc = cu_waves * parts * nb * 1024.0 / 180.0 * lds_factor;
           const double l1 = cu_waves * parts * mb * 1024.0 / 67.0;
           const double latency = (simd_waves >= 2 ? 93.0 : 105.0) + 41.5 * parts * nb * lds_factor;
@@ -897,6 +911,10 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           A.cc = cc;
           A.noct = noct;
           A.parts = parts;
+          A.products = products;
+          A.split_pitch = copy_cin;
+          A.split_other = eight ? kSplitOther8Map : kSplitOtherMap;
+          A.taps_inner = eight && parts == 1 ? 1 : 0;
           A.part_octs = A.cin_g / 8 / parts;
           A.rows = static_cast<int>(rows);
           A.hlast = hext[R - 1];
@@ -958,8 +976,7 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
   if (plan.ok) {
     IgemmArgs& A = plan.args;
     plan.padded = padded;
-    plan.or_direct = padded || wide || (split && !staged_fits(gemm_cin)) ||
-                     !plain_plan_exists(R, J, sigma, span, ntaps_max, mtiles);
+    plan.or_direct = padded || eight || !plain;
     plan.wpk_elems = (size_t)A.nphase * A.groups * A.tcount * A.nchunk * A.kc_max * A.parts * A.mtiles_padded * 64 * 8;
     plan.staged_elems = (size_t)A.batch * A.in_vol * A.cin_total;
     // Byte offsets into the staged operand are 32-bit (buffer loads, an offset of 0xffffffe0
@@ -1000,9 +1017,9 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
     S.src_cg = real_cin;
     S.dst_cg = A.cin_g;
     S.split_c = split ? real_cin : 0;
-    S.split_pitch = A.parts == 3 ? real_octs * 8 : real_cin;
-    S.split_n = A.parts == 3 ? 3 : kSplit;
-    S.split_map = A.parts == 3 ? kSplitPartsMap : kSplitDataMap;
+    S.split_pitch = A.split_pitch;
+    S.split_n = A.parts == 3 ? 3 : A.products;
+    S.split_map = A.parts == 3 ? kSplitPartsMap : (eight ? kSplitData8Map : kSplitDataMap);
     S.split_batch = 0;
     for (int a = 0; a < R; ++a) {
       S.in[a] = A.in_size[a];
@@ -2976,7 +2993,7 @@ int convnd_hip_plan_describe(const convnd_hip_problem* problem, convnd_hip_dtype
              ",\"conflict\":" + std::to_string(p.conflict) +
              ",\"boxes\":" + std::to_string(A.boxes) + ",\"phases\":" +
              std::to_string(A.nphase) + ",\"cc\":" + std::to_string(A.cc) +
-             ",\"parts\":" + std::to_string(A.parts) + ",\"tsplit\":" + std::to_string(A.tsplit) +
+             ",\"parts\":" + std::to_string(A.parts) + ",\"products\":" + std::to_string(A.products) + ",\"tsplit\":" + std::to_string(A.tsplit) +
              ",\"tcount\":" + std::to_string(A.tcount) + ",\"plen\":" + std::to_string(A.plen) +
              ",\"nchunk\":" + std::to_string(A.nchunk) + ",\"kc_max\":" +
              std::to_string(A.kc_max) + ",\"mgroups\":" + std::to_string(A.mgroups) +

@@ -57,27 +57,33 @@ __device__ __forceinline__ void unrolled(F&& body) {
   }
 }
 
-// The six part products of one K32 step, smallest first: position parts b, weight parts a.
-template <typename M, int MB, int NB>
+// The part products of one K32 step, smallest first: position parts b, weight parts a. Six of them
+// into one accumulator; with NP = 8 all but the one below 2^-28 of the product, the seven cross
+// products in an accumulator of their own, so that neither a truncated part nor a small product
+// added to a large sum is lost.
+template <typename M, int MB, int NB, int NP>
 __device__ __forceinline__ void part_products(const typename M::frag (*b)[NB],
                                               const typename M::frag (*a)[MB],
-                                              f32x4 (&acc)[MB][NB]) {
-  constexpr int kData[6] = {1, 2, 0, 1, 0, 0};
-  constexpr int kOther[6] = {1, 0, 2, 0, 1, 0};
+                                              f32x4 (&acc)[MB][NB], f32x4 (&cross)[MB][NB]) {
+  constexpr int kData[8] = {1, 2, 1, 2, 0, 1, 0, 0};
+  constexpr int kOther[8] = {2, 1, 1, 0, 2, 0, 1, 0};
 #pragma unroll
-  for (int q = 0; q < 6; ++q)
+  for (int q = 8 - NP; q < 8; ++q) {
+    f32x4(&sum)[MB][NB] = NP == 8 && q < 7 ? cross : acc;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb)
-        acc[mb][nb] = M::run(b[kData[q]][nb], a[kOther[q]][mb], acc[mb][nb]);
+        sum[mb][nb] = M::run(b[kData[q]][nb], a[kOther[q]][mb], sum[mb][nb]);
+  }
 }
 
 // T: GEMM operand type; O: output and bias type (T, or float for split-precision fp32).
-// P: bf16 parts of split-precision fp32 staged and packed once each (3), else 1.
+// P: bf16 parts of split-precision fp32 staged and packed once each (3), else 1; NP: products of
+// two parts that a K step adds (see part_products).
 // Every per-axis quantity comes from the geometry tables (IgemmArgs::tables), so the
 // kernel body is the same for every rank.
-template <typename T, typename O, int MB, int NB, int WM, bool DS, int W, int P = 1>
+template <typename T, typename O, int MB, int NB, int WM, bool DS, int W, int P = 1, int NP = 6>
 __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(igemm_waves<MB, NB>, igemm_waves<MB, NB>)))
 void igemm_kernel(IgemmArgs A) {
@@ -201,6 +207,15 @@ void igemm_kernel(IgemmArgs A) {
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Sums of the cross products (P == 3, NP == 8; unused otherwise).
+  f32x4 cross[MB][NB];
+  auto clear_cross = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) cross[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear_cross();
 
   const size_t wpart = (size_t)A.mtiles_padded * 64;  // fragments per part of a K32 step
   const size_t wstep = P * wpart;                     // fragments per K32 step
@@ -262,7 +277,7 @@ void igemm_kernel(IgemmArgs A) {
           load_b(br[(i + 1) & 1], tb);
           load_w(ar[(i + kRing - 1) % kRing], kc + i + kRing - 1);
           __builtin_amdgcn_sched_barrier(0);
-          part_products<M, MB, NB>(br[i & 1], ar[i % kRing], acc);
+          part_products<M, MB, NB, NP>(br[i & 1], ar[i % kRing], acc, cross);
           __builtin_amdgcn_sched_barrier(0);
         };
         int kc = 0;
@@ -301,7 +316,7 @@ void igemm_kernel(IgemmArgs A) {
             bt[p][nb] = __builtin_bit_cast(frag, v);
           }
         }
-        part_products<M, MB, NB>(bt, at, acc);
+        part_products<M, MB, NB, NP>(bt, at, acc, cross);
       }
       return;
     }
@@ -608,6 +623,12 @@ void igemm_kernel(IgemmArgs A) {
     }
   };
   auto store_outputs = [&]() __attribute__((always_inline)) {
+    if constexpr (P == 3 && NP == 8) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[mb][nb] += cross[mb][nb];
+    }
     switch (A.act) {
       case CONVND_HIP_ACT_RELU:
         epilogue(std::integral_constant<int, CONVND_HIP_ACT_RELU>{});
@@ -820,18 +841,22 @@ void igemm_kernel(IgemmArgs A) {
     // halo that its phases share: 128 <- 64 channels in 4 groups, stride 2 on three axes, 24^3 x 12,
     // 103 -> 79 us.
     for (int q = 0;;) {
-      for (int tc = 0; tc < A.tcount; ++tc) {
+      for (int tc = 0, ck = 0, last = 0;;) {
         // Every wave is past the staging that read the rows (the last chunk's barrier).
-        if (tc > 0) fill_rows(tc);
-        for (int ck = 0; ck < A.nchunk; ++ck) {
-          if (q == 0) {
-            // Row table written, and every wave done reading the chunk before.
-            __syncthreads();
-            stage(ck);
-            __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads have landed in LDS
-            __syncthreads();
-          }
-          mma_chunk(tc * A.nchunk + ck, lds, []() {});
+        if (tc != last) fill_rows(tc);
+        last = tc;
+        if (q == 0) {
+          // Row table written, and every wave done reading the chunk before.
+          __syncthreads();
+          stage(ck);
+          __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads have landed in LDS
+          __syncthreads();
+        }
+        mma_chunk(tc * A.nchunk + ck, lds, []() {});
+        // Chunks of a split tap, then the next tap; or the taps of a chunk (IgemmArgs::taps_inner).
+        if (A.taps_inner ? ++tc == A.tcount : ++ck == A.nchunk) {
+          if (A.taps_inner ? ++ck == A.nchunk : ++tc == A.tcount) break;
+          (A.taps_inner ? tc : ck) = 0;
         }
       }
       store_outputs();
@@ -848,6 +873,7 @@ void igemm_kernel(IgemmArgs A) {
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      clear_cross();
     }
   }
 }
@@ -862,23 +888,31 @@ void igemm_kernel(IgemmArgs A) {
 #define CONVND_IGEMM_TILES8(X) \
   X(4, 4, 1) X(2, 4, 1) X(4, 2, 1) X(2, 8, 1) X(1, 8, 1) X(1, 4, 1) X(1, 2, 1) X(2, 2, 1)
 
-// Split precision from three parts (two waves per SIMD, 256 registers each).
+// Split precision from three parts (two waves per SIMD, 256 registers each); with the second
+// accumulators of eight products, the tiles that fit them without scratch.
+#define CONVND_IGEMM_TILES_P3X8(X) \
+  X(1, 2, 1) X(1, 4, 1) X(2, 2, 1) X(1, 4, 2) X(2, 2, 2) X(1, 4, 4)
 #define CONVND_IGEMM_TILES_P3(X) \
-  X(1, 2, 1) X(1, 4, 1) X(2, 2, 1) X(2, 4, 1) X(1, 4, 2) X(2, 4, 2) X(2, 2, 2) X(1, 4, 4) X(4, 2, 1)
+  CONVND_IGEMM_TILES_P3X8(X) X(2, 4, 1) X(2, 4, 2) X(4, 2, 1)
 
 hipError_t igemm_dispatch_p3(int mb, int nb, const IgemmArgs& a, size_t lds, hipStream_t s) {
   const dim3 grid(a.boxes, a.groups * a.mgroups, a.batch * (a.nphase / a.plen));
-#define CONVND_IGEMM_CASE(MBV, NBV, WMV)                                                       \
-  if (mb == MBV && nb == NBV && a.wm == WMV && a.waves == 4) {                                 \
-    auto fn = igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3>;                         \
+#define CONVND_IGEMM_CASE_NP(MBV, NBV, WMV, NPV)                                               \
+  if (mb == MBV && nb == NBV && a.wm == WMV && a.waves == 4 && a.products == NPV) {            \
+    auto fn = igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3, NPV>;                    \
     hipError_t err =                                                                           \
-        ensure_dynamic_lds<igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3>>(lds);      \
+        ensure_dynamic_lds<igemm_kernel<__bf16, float, MBV, NBV, WMV, false, 4, 3, NPV>>(lds); \
     if (err != hipSuccess) return err;                                                         \
     hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, a);                                        \
     return hipGetLastError();                                                                  \
   }
+#define CONVND_IGEMM_CASE(MBV, NBV, WMV) CONVND_IGEMM_CASE_NP(MBV, NBV, WMV, 6)
+#define CONVND_IGEMM_CASE_X8(MBV, NBV, WMV) CONVND_IGEMM_CASE_NP(MBV, NBV, WMV, 8)
   CONVND_IGEMM_TILES_P3(CONVND_IGEMM_CASE)
+  CONVND_IGEMM_TILES_P3X8(CONVND_IGEMM_CASE_X8)
+#undef CONVND_IGEMM_CASE_X8
 #undef CONVND_IGEMM_CASE
+#undef CONVND_IGEMM_CASE_NP
   return hipErrorInvalidValue;
 }
 
@@ -912,11 +946,13 @@ hipError_t igemm_dispatch(int mb, int nb, const IgemmArgs& a, size_t lds, hipStr
 
 }  // namespace
 
-bool igemm_tile_supported(int mb, int nb, int wm, int waves, int parts) {
+bool igemm_tile_supported(int mb, int nb, int wm, int waves, int parts, int products) {
 #define CONVND_IGEMM_HAS(MBV, NBV, WMV) \
   if (mb == MBV && nb == NBV && wm == WMV) return true;
   if (parts == 3) {
-    if (waves == 4) {
+    if (waves == 4 && products == 8) {
+      CONVND_IGEMM_TILES_P3X8(CONVND_IGEMM_HAS)
+    } else if (waves == 4) {
       CONVND_IGEMM_TILES_P3(CONVND_IGEMM_HAS)
     }
     return false;

@@ -145,11 +145,17 @@ struct IgemmArgs {
   int k[kFastRank], s[kFastRank], p[kFastRank], d[kFastRank];
   int k_vol;
   int split_c;     // split-precision fp32: real channels per group in the GEMM-input role
-  // Split-precision fp32 operand layout. parts 1: six copies of the channels (one per part
-  // product) as one K dimension. parts 3: the three bf16 parts of every channel once, cin_g =
+  // Split-precision fp32 operand layout. parts 1: a copy of the channels per part product (the weights'
+  // parts by split_other, split_pitch channels from one to the next) as one K dimension. parts 3: the three bf16 parts of every channel once, cin_g =
   // 3 * part_octs * 8 staged channels per group (part slowest) and three weight fragments per
-  // (step, M tile); every K32 step runs the six part products from registers. 16-bit data: 1.
+  // (step, M tile); every K32 step runs the part products from registers. 16-bit data: 1.
   int parts;
+  int products;    // part products: 6, or 8 (part_products); 16-bit data: 1
+  int split_pitch;
+  unsigned split_other;
+  // Eight copies: the channel chunks, smallest products first, run over all split taps each, so that
+  // the sums of the small products are complete before the large one's are added to them.
+  int taps_inner;
   int part_octs;   // octets of one part's channels per group (all of them: cin_g / 8 / parts)
   int in_bytes;    // bytes of the staged operand (unsigned bit pattern, below 0xffffffe0)
   // Geometry tables in device memory, built once per plan by the host (convnd_geometry.h)
@@ -481,6 +487,9 @@ int64_t prologue_sum_blocks(int64_t batch, int64_t volume);
 constexpr int kSplitBlocks = 6;
 constexpr unsigned kSplitDataMap = 0x120100u;   // 0, 0, 1, 0, 2, 1
 constexpr unsigned kSplitOtherMap = 0x102010u;  // 0, 1, 0, 2, 0, 1
+// Eight products, smallest first (all but (2, 2)): data parts 1 2 1 2 0 1 0 0 with 2 1 1 0 2 0 1 0.
+constexpr unsigned kSplitData8Map = 0x00102121u;
+constexpr unsigned kSplitOther8Map = 0x01020112u;
 constexpr unsigned kSplitPartsMap = 0x210u;     // 0, 1, 2
 struct IgemmArgs;
 struct WgradArgs;
@@ -540,8 +549,8 @@ hipError_t launch_igemm(convnd_hip_dtype dtype, int mb, int nb, const IgemmArgs&
                         size_t lds_bytes, hipStream_t stream);
 // Whether launch_igemm has a compiled kernel for this wave tile (mb x nb fragments), wave
 // arrangement (wm waves along output channels), workgroup size (waves: 4, or 8 with direct
-// staging) and operand layout (parts).
-bool igemm_tile_supported(int mb, int nb, int wm, int waves, int parts);
+// staging), operand layout (parts) and part products per K step.
+bool igemm_tile_supported(int mb, int nb, int wm, int waves, int parts, int products);
 // stg: staging slots per thread (8, 16 or 24); multi: the item's staging takes
 // several batches of 8 slots (only the first is prefetched).
 hipError_t launch_wgrad_mfma(convnd_hip_dtype dtype, int mb, int stg, bool multi,

@@ -16,8 +16,8 @@ namespace stage {
 // Packed weights: unit u = ((((phase*G + g)*tcount*nchunk + chunk)*kc_max + kc)*parts*mtiles_padded
 // + part*mtiles_padded + mt)*64 + lane holds the 8 A-fragment elements W'[m][k], m = mt*16 + lane%16,
 // k = kc*32 + (lane/16)*8 + i (i < 8), zero where m or k is padding.
-// S = float (split precision): GEMM channel ci is part split_other_part(ci / split_c) of
-// channel ci % split_c of the fp32 weight (zero past kSplitProducts copies); with parts == 3
+// S = float (split precision): GEMM channel ci is part split_map_part(split_other, ci / split_pitch)
+// of channel ci % split_pitch of the fp32 weight (zero from split_c on, past the copies); with parts == 3
 // channel ci of part `part` (zero from split_c on).
 template <typename T, typename S>
 __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w, T* wpk,
@@ -76,10 +76,10 @@ __device__ __forceinline__ void igemm_pack_blocks(const IgemmArgs& A, const S* w
       if (A.parts == 3) {
         live = live && ci < A.split_c;
       } else {
-        const int sp = ci / A.split_c;
-        live = live && sp < kSplitProducts;
-        ci -= sp * A.split_c;
-        part = split_other_part(sp);
+        const int sp = ci / A.split_pitch;
+        ci -= sp * A.split_pitch;
+        live = live && sp < A.products && ci < A.split_c;
+        part = split_map_part(A.split_other, sp);
       }
     } else {
       // Zero channels that fill the last octet of the GEMM input.
