@@ -82,3 +82,46 @@ def test_split_products_are_no_further_off_than_fp32_products(name, kind):
         if p in passes:
             error = ((got.detach().double().cpu() - ref).norm() / ref.norm()).item()
             assert error <= bound(kind, n), (p, error, bound(kind, n))
+
+
+# Strided last axes whose halo only the channel-major weight gradient holds.
+WEIGHT_CASES = {
+    "small": ((1, 16, 7, 7, 7, 7, 9), (8, 16, 3, 3, 3, 3, 3)),
+    "ragged": ((2, 8, 9, 7, 7, 7, 5), (24, 8, 3, 3, 3, 3, 3)),
+    "many_boxes": ((2, 8, 11, 11, 9, 9, 9), (16, 8, 3, 3, 3, 3, 3)),
+}
+
+
+def weight_bound(kind, positions):
+    """Position i in thread i mod 256, then a tree of eight levels, whose partial sums carry
+    1 (zero mean) or 2^-level (one sign) of the squared result together."""
+    chain = positions / 256
+    if kind == "same_sign":
+        terms = chain / 768 + 2
+    else:
+        share = SPARSE if kind == "sparse" else 1.0
+        terms = share * chain / 2 + min(8, share * positions)
+    return 1.1 * ROUNDING * math.sqrt(terms + 1)
+
+
+@pytest.mark.parametrize("kind", ["dense", "same_sign", "sparse"])
+@pytest.mark.parametrize("name", list(WEIGHT_CASES))
+def test_strided_weight_gradient_is_no_further_off_than_fp32_products(name, kind):
+    x_shape, w_shape = WEIGHT_CASES[name]
+    args = ((2,) * 5, (1,) * 5, (1,) * 5, 1)
+    print(f"[precision] weight gradient {name} {kind} x={x_shape} w={w_shape}", flush=True)
+    lib = _build.hip_library()
+    assert lib.convnd_hip_plan_check(ctypes.byref(_capi.Problem.make(x_shape, w_shape, *args)),
+                                     _capi.FLOAT32) == _capi.SUCCESS
+    assert _capi.plan_details(lib, x_shape, w_shape, *args, torch.float32)[2]["kernel"] == "mfma_wgrad_cm"
+    g = torch.Generator().manual_seed(82)
+    x = draw(kind, x_shape, g)
+    w = draw("dense", w_shape, g)
+    out = tuple((n - 1) // 2 + 1 for n in x_shape[2:])
+    dy = draw("dense" if kind == "sparse" else kind, (x_shape[0], w_shape[0], *out), g)
+    ref = helpers.oracle_backward(dy, x, w, *args)[1]
+    dev = [t.cuda().requires_grad_() for t in (x, w)]
+    y = conv_nd(dev[0], dev[1], None, *args, backend="native")
+    dw = torch.autograd.grad(y, dev[1], dy.cuda())[0]
+    error = ((dw.double().cpu() - ref).norm() / ref.norm()).item()
+    assert error <= weight_bound(kind, x_shape[0] * math.prod(out)), (error, weight_bound(kind, x_shape[0] * math.prod(out)))

@@ -1077,12 +1077,22 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
     return false;
   // The planar copy's source is addressed by 32-bit byte offsets.
   if (g.batch * g.channels * g.in_vol * element_size(dt) > 0xffffffe0ll) return false;
-  // Split precision: the GEMM runs over kSplit part products per image, read from copies that
+  // Split precision: the GEMM runs over the part products of each image, read from copies that
   // hold each of the three bf16 parts once (of the input and of grad_output).
-  const int64_t batch = split ? g.batch * kSplit : g.batch;
-  const int64_t sbatch = split ? g.batch * 3 : g.batch;
   const int R = g.rank;
   const int ls = static_cast<int>(g.s[R - 1]);
+  // Strided fp32 layers, which the direct kernel's fp32 products served before, keep that precision:
+  // eight products, smallest first, and short position chunks. A box adds eight K steps to a sum, the
+  // direct kernel one position per 256 to each of the 256 threads' sums, which a tree then adds:
+  // chunks of positions / (12 * 256) boxes have two thirds of its chain, and at most eight boxes hold
+  // against its tree where the chains are long; their sums are added in double. Relative error
+  // (2-norm) of 16 -> 32 channels on 11^5, stride 2, for dense / same-sign / sparse data: direct
+  // 1.1e-7 / 4.1e-8 / 2.5e-8, six products in two chunks 2.3e-7 / 1.1e-7 / 7.6e-8, now
+  // 6.7e-8 / 2.8e-8 / 2.5e-8; time 3.8 ms, 143 us, 244 us.
+  const bool eight = split && ls != 1;
+  const int64_t products = split ? (eight ? 8 : kSplit) : 1;
+  const int64_t batch = g.batch * products;
+  const int64_t sbatch = split ? g.batch * 3 : g.batch;
   if (ls > kMaxLastStride) return false;
   const int cin_g = static_cast<int>(g.cin_g), cout_g = static_cast<int>(g.cout_g);
   const int k_vol = static_cast<int>(g.k_vol);
@@ -1208,12 +1218,16 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         if (xi > 64 || dyt_bytes + xi * 1024 > kWgradCmBuffer) continue;
         const int64_t per_chunk_wgs = (int64_t)ncq * g.groups * mgroups;
         int64_t npc = std::min<int64_t>(std::max<int64_t>(1, 256 / per_chunk_wgs), items);
-        const int64_t ipc = (items + npc - 1) / npc;
+        int64_t ipc = (items + npc - 1) / npc;
+        if (eight)
+          ipc = std::min(ipc, std::clamp<int64_t>(g.batch * g.out_vol / (12 * box_vol), 2, 8));
         npc = (items + ipc - 1) / ipc;
         const int64_t lds_items = align_up((int64_t)(box_vol / 8) * 4);
         const int64_t lds = lds_items + ipc * 8;
         if (lds > dyn_budget) continue;
         if (npc * per_chunk_wgs > INT32_MAX) continue;
+        // (Partial sums of the short chunks: at most 1 GiB.)
+        if (eight && npc * per_chunk_wgs * 4 * mb * nt * 64 * 16 > (int64_t{1} << 30)) continue;
         for (const bool parity : {false, true})
         for (const int waves : {8, 4}) {
         if (!wgrad_cm_supported(mb, nt, waves)) continue;
@@ -1266,6 +1280,8 @@ bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
         C.rank = R;
         C.batch = static_cast<int>(batch);
         C.split_n = split ? static_cast<int>(g.batch) : 0;
+        C.split_data = eight ? kSplitData8Map : kSplitDataMap;
+        C.split_other = eight ? kSplitOther8Map : kSplitOtherMap;
         C.groups = static_cast<int>(g.groups);
         C.cin_g = cin_g;
         C.cout_g = cout_g;

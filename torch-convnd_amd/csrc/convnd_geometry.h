@@ -733,13 +733,13 @@ inline void wgrad_cm_build_tables(const WgradCmArgs& A, unsigned char* tab) {
   for (int it = 0; it < A.items; ++it) {
     const int n = it / boxes;
     int bb = it - n * boxes;
-    // Split precision: batch block s pairs part split_data_part(s) of the input with part
-    // split_other_part(s) of grad_output, each copy holding the three parts once.
+    // Split precision: batch block s pairs one part of the input with one of grad_output, each
+    // copy holding the three parts once.
     int xn = n, dn = n;
     if (A.split_n > 0) {
       const int s = n / A.split_n, i = n - s * A.split_n;
-      xn = split_data_part(s) * A.split_n + i;
-      dn = split_other_part(s) * A.split_n + i;
+      xn = split_map_part(A.split_data, s) * A.split_n + i;
+      dn = split_map_part(A.split_other, s) * A.split_n + i;
     }
     long long xbase = (long long)xn * A.cin_total * A.pvol;
     long long dbase = (long long)dn * A.cout_total * A.dvol;

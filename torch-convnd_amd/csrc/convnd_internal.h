@@ -325,9 +325,10 @@ struct WgradCmArgs {
   int kvp, tpc, cpc;
   int npc, items, items_per_pc;
   // Split-precision fp32: images per part block (0 otherwise). Item n of batch block s reads
-  // part split_data_part(s) of image n % split_n from the padded input's part copies and
-  // part split_other_part(s) from grad_output's (three part images each).
+  // part split_map_part(split_data, s) of image n % split_n from the padded input's part copies and
+  // part split_map_part(split_other, s) from grad_output's (three part images each).
   int split_n;
+  unsigned split_data, split_other;
   int lds_items;        // dynamic LDS byte offset of the item records (after the run table)
   int box[kFastRank], nbox[kFastRank], dext[kFastRank], hext[kFastRank], pe[kFastRank];
   int k[kFastRank], s[kFastRank], d[kFastRank];

@@ -28,6 +28,8 @@
 //     partial sums of its range of items; a second pass adds them in a fixed order into the
 //     weight layout (deterministic, no atomics).
 
+#include <type_traits>
+
 #include "convnd_internal.h"
 #include "convnd_stage.h"
 #include "convnd_types.h"
@@ -376,13 +378,15 @@ __global__ __launch_bounds__(kThreads) void wgrad_cm_reduce_kernel(const f32x4* 
     stage::bias_from_sums<T>(bs, blockIdx.x - rblocks);
     return;
   }
-  __shared__ f32x4 wsum[3][64];
+  // fp32 results: the partials are added in double and rounded once.
+  using V = std::conditional_t<sizeof(T) == 4, f64x4, f32x4>;
+  __shared__ V wsum[3][64];
   const int wave = static_cast<int>(threadIdx.x) >> 6;
   const int lane = static_cast<int>(threadIdx.x) & 63;
   // 32-bit slot arithmetic (the launcher keeps nslots below 2^31).
   const int s = static_cast<int>(blockIdx.x) * 64 + lane;
   const bool live = s < nslots;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  V acc = {0, 0, 0, 0};
   for (int i0 = wave; i0 < A.npc; i0 += 32) {
     f32x4 v[8];
 #pragma unroll
@@ -392,7 +396,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_cm_reduce_kernel(const f32x4* 
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (i0 + 4 * k < A.npc) acc += v[k];
+      if (i0 + 4 * k < A.npc) acc += __builtin_convertvector(v[k], V);
   }
   if (wave > 0) wsum[wave - 1][lane] = acc;
   __syncthreads();
