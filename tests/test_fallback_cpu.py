@@ -9,6 +9,7 @@ buffers are addresses that are never read. Skipped where a GPU is present.
 import ctypes
 import math
 import random
+import time
 
 import pytest
 import torch
@@ -122,3 +123,19 @@ def test_calls_without_tables(lib, dtype, which, args):
         assert message.startswith("direct "), message
     else:
         assert message.startswith("geometry tables"), message
+
+
+def noalloc(lib, problem, dt):
+    return lib.convnd_hip_forward_noalloc(ctypes.byref(problem), dt, NOWHERE, NOWHERE, None, NOWHERE, None)
+
+
+def test_noalloc_plans_a_geometry_once(lib):
+    """A plan search takes milliseconds, a lookup microseconds: only the first call of a geometry
+    searches, also where neither its three-part plan nor six copies fit the scratch."""
+    problem = _capi.Problem.make((32, 48, 18, 17, 16, 7), (48, 48, 3, 3, 3, 3), (1,) * 4, (1,) * 4, (1,) * 4, 1)
+    times = []
+    for _ in range(12):
+        start = time.perf_counter()
+        assert noalloc(lib, problem, _capi.FLOAT32) == _capi.WORKSPACE_TOO_SMALL
+        times.append(time.perf_counter() - start)
+    assert min(times[1:]) < times[0] / 10, times

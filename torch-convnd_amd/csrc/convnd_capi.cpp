@@ -1863,6 +1863,30 @@ ForwardSetup setup_forward(const Geom& g, convnd_hip_dtype dt) {
   return cached_plan(cache, plan_key(g, dt, 0), [&] { return make_forward(g, dt); });
 }
 
+// The forward of the allocation-free entry, whose scratch holds [geometry tables | the workspace
+// regions of convnd_hip_forward]: the forward's own plan where that fits; where it does not, the
+// direct kernel for or_direct plans, and for split precision from three parts six copies if they
+// fit (the call fails if the plan returned does not).
+ForwardSetup setup_noalloc(const Geom& g, convnd_hip_dtype dt) {
+  static PlanCache<ForwardSetup> cache;
+  return cached_plan(cache, plan_key(g, dt, 0), [&] {
+    auto fits = [](const ForwardSetup& f) {
+      return align_up(static_cast<size_t>(f.ig.args.tab_bytes)) + f.bytes <= kNoAllocScratchBytes;
+    };
+    ForwardSetup f = setup_forward(g, dt);
+    if (!f.ig.ok || fits(f)) return f;
+    if (f.ig.or_direct) {
+      f.ig.ok = false;
+    } else if (f.ig.args.parts == 3) {
+      PlanFilter six;
+      six.parts = 1;
+      const ForwardSetup other = layout_forward(plan_igemm_filtered(g, dt, 0, six));
+      if (other.ig.ok && fits(other)) f = other;
+    }
+    return f;
+  });
+}
+
 // The input gradient's staging pass can add grad_output's channel sums: 16-bit data, and fp32
 // read once for its three parts.
 bool staging_sums(const IgemmPlan& dg, convnd_hip_dtype dt) {
@@ -2613,25 +2637,11 @@ int convnd_hip_forward_noalloc(const convnd_hip_problem* problem, convnd_hip_dty
   if (st != CONVND_HIP_SUCCESS) return st;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   if (g.batch == 0) return CONVND_HIP_SUCCESS;
-  ForwardSetup f = setup_forward(g, dtype);
-  // Scratch: [geometry tables | the workspace regions of convnd_hip_forward].
-  size_t tab = f.ig.ok ? align_up(static_cast<size_t>(f.ig.args.tab_bytes)) : 0;
-  if (f.ig.ok && tab + f.bytes > kNoAllocScratchBytes) {
-    if (f.ig.or_direct) {
-      f.ig.ok = false;
-    } else if (f.ig.args.parts == 3) {
-      // Split precision whose three-part plan exceeds the scratch: six copies may still fit.
-      PlanFilter six;
-      six.parts = 1;
-      const IgemmPlan ig = plan_igemm_filtered(g, dtype, 0, six);
-      const ForwardSetup f6 = layout_forward(ig);
-      if (ig.ok && align_up(static_cast<size_t>(ig.args.tab_bytes)) + f6.bytes <= kNoAllocScratchBytes) f = f6;
-    }
-  }
+  const ForwardSetup f = setup_noalloc(g, dtype);
   if (!f.ig.ok)  // the direct kernels use no scratch
     return run_forward(g, dtype, f, input, weight, bias, output, CONVND_HIP_ACT_NONE, nullptr,
                        nullptr, nullptr, false, stream);
-  tab = align_up(static_cast<size_t>(f.ig.args.tab_bytes));
+  const size_t tab = align_up(static_cast<size_t>(f.ig.args.tab_bytes));
   if (tab + f.bytes > kNoAllocScratchBytes)
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "convnd_hip_forward_noalloc: this problem needs " + std::to_string(tab + f.bytes) +
