@@ -212,11 +212,12 @@ int convnd_hip_partial_rescale(convnd_hip_dtype dtype, const void* raw, const vo
 /* convnd_hip_forward without a workspace and without any device allocation: the staged
  * input, the packed weights and the geometry tables live in a file-scope device array of
  * CONVND_HIP_NOALLOC_SCRATCH_BYTES per GPU, held from the library's load until the process
- * ends; the call itself makes no hipMalloc / hipFree. Problems whose scratch needs exceed it
- * fail with CONVND_HIP_WORKSPACE_TOO_SMALL and a message naming the size. Every call on one
+ * ends; the call itself makes no hipMalloc / hipFree. Problems for which no
+ * plan's scratch fits it fail with CONVND_HIP_WORKSPACE_TOO_SMALL and a message naming the size. Every call on one
  * GPU shares that GPU's array and leaves its contents behind (each call rewrites all it
  * reads), so calls that overlap on one GPU (other streams, other threads) race: serialise
- * them. Same results as convnd_hip_forward (the same kernels).
+ * them. Results are convnd_hip_forward's bit for bit where its own plan fits the scratch; where
+ * it does not, another plan that fits or the direct kernels run, which add in another order.
  * No counterpart in the reference: for callers that cannot allocate device memory -- code
  * under stream capture, serving loops that must not allocate, harnesses that forbid
  * hipMalloc. */

@@ -139,3 +139,24 @@ def test_noalloc_plans_a_geometry_once(lib):
         assert noalloc(lib, problem, _capi.FLOAT32) == _capi.WORKSPACE_TOO_SMALL
         times.append(time.perf_counter() - start)
     assert min(times[1:]) < times[0] / 10, times
+
+
+# Layers whose plan stages a copy larger than the scratch, while another, staged straight from the
+# input, needs little (all but the last, whose packed weights alone exceed it).
+@pytest.mark.parametrize(
+    ("x_shape", "w_shape", "stride", "padding", "dilation", "groups", "taken"),
+    [
+        ((8, 128, 11, 10, 11, 10, 13), (8, 128, 3, 3, 3, 3, 3), (1,) * 5, (1,) * 5, (1,) * 5, 1, True),
+        ((8, 32, 16, 13, 11, 13, 15), (8, 32, 3, 3, 3, 3, 3), (1,) * 5, (1,) * 5, (1,) * 5, 1, True),
+        ((8, 40, 7, 7, 7, 7, 7, 7), (1, 40, 3, 3, 2, 3, 1, 2), (1,) * 6, (3, 1, 1, 2, 0, 0), (3, 1, 3, 2, 3, 1), 1, True),
+        ((8, 64, 6, 6, 6, 6, 6, 6, 6), (192, 32, 3, 1, 3, 3, 3, 3, 1), (2,) * 7, (1, 0, 1, 1, 1, 1, 0), (1,) * 7, 2, True),
+        ((1, 1024, 4, 4, 4, 4), (1024, 1024, 3, 3, 3, 3), (1,) * 4, (1,) * 4, (1,) * 4, 1, False),
+    ],
+)
+def test_noalloc_takes_plans_that_fit_its_scratch(lib, x_shape, w_shape, stride, padding, dilation, groups, taken):
+    problem = _capi.Problem.make(x_shape, w_shape, stride, padding, dilation, groups)
+    need = lib.convnd_hip_forward_workspace_size(ctypes.byref(problem), _capi.BFLOAT16)
+    assert need > _capi.NOALLOC_SCRATCH_BYTES
+    status = noalloc(lib, problem, _capi.BFLOAT16)
+    # (Taken: the call goes on to the device, which is not there.)
+    assert status == (_capi.LAUNCH_FAILED if taken else _capi.WORKSPACE_TOO_SMALL)

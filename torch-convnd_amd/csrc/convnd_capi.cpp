@@ -547,6 +547,7 @@ bool plain_plan_exists(int R, const int* J, const int* sigma, const int* span, i
 // ignores the override when none does.
 struct PlanFilter {
   int mb = 0, nb = 0, wm = 0, cc = 0, occ = 0, cm = -1, ds = -1, nbuf = 0, waves = 0, parts = 0, ts = -1, parity = -1, plen = 0;
+  size_t max_bytes = 0;  // of the tables and workspace (0: any)
   std::vector<int> box;
   bool active = false;
 };
@@ -887,6 +888,23 @@ IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
           const int* hpitch = pitches.hpitch;
           const int64_t plane_bytes = plane_align(pitches.plane_pos * 16);
           const int tap_row = static_cast<int>((kc + kTapPad + 3) / 4 * 4);
+          if (filter.max_bytes > 0) {
+            IgemmArgs T{};  // what the table layout reads
+            T.nphase = nphase;
+            T.tap_row = tap_row;
+            T.box_vol = box_vol;
+            T.rows = static_cast<int>(rows);
+            T.direct = direct ? 1 : 0;
+            T.plane_bytes = static_cast<int>(plane_bytes);
+            T.tcount = static_cast<int>(tcount);
+            T.boxes = static_cast<int>(boxes);
+            T.kc_max = static_cast<int>(kc);
+            const size_t packed = (size_t)nphase * g.groups * tcount * nchunk * kc * parts *
+                                  (mgroups * wm * mb) * 512 * 2;
+            const size_t staged = direct ? 0 : (size_t)in_positions * staged_cin * 2;
+            if (align_up(igemm_table_layout(T)) + align_up(staged) + align_up(packed) > filter.max_bytes)
+              continue;
+          }
           best = cost;
           plan.ok = true;
           plan.mb = mb;
@@ -1865,25 +1883,22 @@ ForwardSetup setup_forward(const Geom& g, convnd_hip_dtype dt) {
 
 // The forward of the allocation-free entry, whose scratch holds [geometry tables | the workspace
 // regions of convnd_hip_forward]: the forward's own plan where that fits; where it does not, the
-// direct kernel for or_direct plans, and for split precision from three parts six copies if they
-// fit (the call fails if the plan returned does not).
+// direct kernel for or_direct plans, else the cheapest plan that fits (16-bit data staged straight
+// from the input, fp32 as six copies; the call fails if there is none).
 ForwardSetup setup_noalloc(const Geom& g, convnd_hip_dtype dt) {
   static PlanCache<ForwardSetup> cache;
   return cached_plan(cache, plan_key(g, dt, 0), [&] {
-    auto fits = [](const ForwardSetup& f) {
-      return align_up(static_cast<size_t>(f.ig.args.tab_bytes)) + f.bytes <= kNoAllocScratchBytes;
-    };
     ForwardSetup f = setup_forward(g, dt);
-    if (!f.ig.ok || fits(f)) return f;
+    if (!f.ig.ok || align_up(static_cast<size_t>(f.ig.args.tab_bytes)) + f.bytes <= kNoAllocScratchBytes)
+      return f;
     if (f.ig.or_direct) {
       f.ig.ok = false;
-    } else if (f.ig.args.parts == 3) {
-      PlanFilter six;
-      six.parts = 1;
-      const ForwardSetup other = layout_forward(plan_igemm_filtered(g, dt, 0, six));
-      if (other.ig.ok && fits(other)) f = other;
+      return f;
     }
-    return f;
+    PlanFilter within;
+    within.max_bytes = kNoAllocScratchBytes;
+    const IgemmPlan ig = plan_igemm_filtered(g, dt, 0, within);
+    return ig.ok ? layout_forward(ig) : f;
   });
 }
 
