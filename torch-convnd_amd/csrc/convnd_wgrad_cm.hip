@@ -28,8 +28,6 @@
 //     partial sums of its range of items; a second pass adds them in a fixed order into the
 //     weight layout (deterministic, no atomics).
 
-#include <type_traits>
-
 #include "convnd_internal.h"
 #include "convnd_stage.h"
 #include "convnd_types.h"
@@ -367,8 +365,9 @@ void wgrad_cm_kernel(WgradCmArgs A) {
 // four output channels of one column. A block covers 64 consecutive slots (lane = slot): its
 // wave w adds the partials w, w + 4, w + 8, ... (loads in flight eight at a time), and the
 // four waves' sums are added in order through LDS (a fixed order: deterministic). Blocks past
-// the reduction's: the bias gradient from the staging pass's sums.
-template <typename T>
+// the reduction's: the bias gradient from the staging pass's sums. V: the type
+// of the sums.
+template <typename T, typename V>
 __global__ __launch_bounds__(kThreads) void wgrad_cm_reduce_kernel(const f32x4* part, T* dw,
                                                                    WgradCmArgs A, int mbv,
                                                                    int64_t nslots, int rblocks,
@@ -378,8 +377,6 @@ __global__ __launch_bounds__(kThreads) void wgrad_cm_reduce_kernel(const f32x4* 
     stage::bias_from_sums<T>(bs, blockIdx.x - rblocks);
     return;
   }
-  // fp32 results: the partials are added in double and rounded once.
-  using V = std::conditional_t<sizeof(T) == 4, f64x4, f32x4>;
   __shared__ V wsum[3][64];
   const int wave = static_cast<int>(threadIdx.x) >> 6;
   const int lane = static_cast<int>(threadIdx.x) & 63;
@@ -501,13 +498,18 @@ hipError_t launch_wgrad_cm_reduce(convnd_hip_dtype dtype, int mb, const WgradCmA
   const int rb = static_cast<int>(rblocks);
   const f32x4* part = reinterpret_cast<const f32x4*>(a.partial);
   if (dtype == CONVND_HIP_BFLOAT16) {
-    hipLaunchKernelGGL(wgrad_cm_reduce_kernel<__bf16>, grid, dim3(kThreads), 0, stream, part,
+    hipLaunchKernelGGL((wgrad_cm_reduce_kernel<__bf16, f32x4>), grid, dim3(kThreads), 0, stream, part,
                        static_cast<__bf16*>(dw), a, mb, nslots, rb, bs);
   } else if (dtype == CONVND_HIP_FLOAT16) {
-    hipLaunchKernelGGL(wgrad_cm_reduce_kernel<_Float16>, grid, dim3(kThreads), 0, stream, part,
+    hipLaunchKernelGGL((wgrad_cm_reduce_kernel<_Float16, f32x4>), grid, dim3(kThreads), 0, stream, part,
                        static_cast<_Float16*>(dw), a, mb, nslots, rb, bs);
+  } else if (dtype == CONVND_HIP_FLOAT32 && a.split_data == kSplitData8Map) {
+    // The short chunks of eight products: added in double, rounded once (elsewhere it would cost
+    // 1.5 us of 260 at [2,24,13,11,10,15] -> 48 channels).
+    hipLaunchKernelGGL((wgrad_cm_reduce_kernel<float, f64x4>), grid, dim3(kThreads), 0, stream, part,
+                       static_cast<float*>(dw), a, mb, nslots, rb, bs);
   } else if (dtype == CONVND_HIP_FLOAT32) {
-    hipLaunchKernelGGL(wgrad_cm_reduce_kernel<float>, grid, dim3(kThreads), 0, stream, part,
+    hipLaunchKernelGGL((wgrad_cm_reduce_kernel<float, f32x4>), grid, dim3(kThreads), 0, stream, part,
                        static_cast<float*>(dw), a, mb, nslots, rb, bs);
   } else {
     return hipErrorInvalidValue;
