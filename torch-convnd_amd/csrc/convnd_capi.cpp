@@ -2406,8 +2406,6 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
     // them into the six products).
     if (dtype == CONVND_HIP_FLOAT32) {
       pp.split_batch = static_cast<int>(g.batch);
-      pp.pp_blocks = 3;
-      pp.pp_part_map = kSplitPartsMap;
       pp.dy_part_map = kSplitPartsMap;
     }
     CA.partial = reinterpret_cast<float*>(ws + b.off_partial);

@@ -477,15 +477,13 @@ int64_t prologue_sum_blocks(int64_t batch, int64_t volume);
 //   octets:     zero-padded octet-major input for the weight gradient (pad);
 //   dy_pad:     grad_output padded to whole boxes for the weight gradient (wg);
 //   planar pad: zero-padded channels-first input for the channel-major weight gradient
-//               (pp; an fp32 source gives pp_batch = pp_blocks x split_batch bf16 part
-//               images, image n holding part split_map_part(pp_part_map, n / split_batch)
-//               of image n % split_batch);
+//               (pp; an fp32 source gives pp_batch = 3 x split_batch bf16 part images,
+//               image n holding part n / split_batch of image n % split_batch);
 //   sums:       channel partial sums of a channels-first 16-bit tensor (bias gradient).
 // Split-precision part maps: 4 bits per image block, block s of a copy holding bf16 part
 // (map >> 4 s) & 15 of every source image. kSplitDataMap / kSplitOtherMap: the six products'
 // parts of the data and the other operand (blocks 0..5, the order of split_data_part /
 // split_other_part); kSplitPartsMap: a copy of the three parts themselves.
-constexpr int kSplitBlocks = 6;
 constexpr unsigned kSplitDataMap = 0x120100u;   // 0, 0, 1, 0, 2, 1
 constexpr unsigned kSplitOtherMap = 0x102010u;  // 0, 1, 0, 2, 0, 1
 // Eight products, smallest first (all but (2, 2)): data parts 1 2 1 2 0 1 0 0 with 2 1 1 0 2 0 1 0.
@@ -515,8 +513,6 @@ struct PrologueParts {
   const PlanarPadArgs* pp = nullptr;  // zero-padded channels-first input (x -> x_pp)
   void* x_pp = nullptr;
   int64_t pp_batch = 0;
-  int pp_blocks = kSplitBlocks;       // fp32 source: part blocks of x_pp
-  unsigned pp_part_map = kSplitDataMap;  // and the part each holds
   // Channel partial sums of a channels-first 16-bit tensor [sum_batch][sum_channels]
   // [sum_volume] in the layout of the GEMM-input copy's sums (octet_sum_blocks per channel).
   const void* sum_src = nullptr;

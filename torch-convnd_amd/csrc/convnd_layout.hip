@@ -64,10 +64,9 @@ struct DevPrologue {
   int64_t e_total;
   int e_blocks;
   int e_split_nc;  // split precision: source (image, channel) rows of each part block
-  unsigned e_part_map;  // and the part each block holds
-  int e_nc_copy;        // (image, channel) rows of one copy
+  int e_nc_copy;   // (image, channel) rows of one copy
   // The three parts of an fp32 source from one read of it, for each of the copies.
-  bool a_all_parts, d_all_parts, e_all_parts;
+  bool a_all_parts, d_all_parts;
   // Channel partial sums of a channels-first 16-bit tensor (bias gradient): block (image,
   // channel, run of kSumRun positions) -> f_sums[c * (batch * f_nrun) + n * f_nrun + run].
   const void* f_src;
@@ -181,7 +180,7 @@ void prologue_kernel(DevPrologue P) {
     if constexpr (SPLIT) {
       stage::pad_planar_split_blocks(static_cast<const float*>(P.xpp_src),
                                      static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total,
-                                     P.e_split_nc, P.e_part_map, P.e_nc_copy, P.e_all_parts, b);
+                                     P.e_split_nc, P.e_nc_copy, b);
     } else {
       stage::pad_planar16_blocks(static_cast<const unsigned short*>(P.xpp_src),
                                  static_cast<unsigned short*>(P.x_pp), P.ppa, P.e_total,
@@ -511,12 +510,10 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
     total += P.d_blocks;
   }
   if (p.x_pp != nullptr && p.pp != nullptr) {
-    // Split precision: pp_batch = pp_blocks x split_batch part images.
-    if (split && (p.split_batch <= 0 || p.pp_blocks < 1 || p.pp_blocks > kSplitProducts ||
-                  p.pp_batch != (int64_t)p.pp_blocks * p.split_batch))
+    // Split precision: three part images per image.
+    if (split && (p.split_batch <= 0 || p.pp_batch != (int64_t)3 * p.split_batch))
       return hipErrorInvalidValue;
     P.e_split_nc = split ? p.split_batch * p.pp->channels : 0;
-    P.e_part_map = p.pp_part_map;
     P.ppa = *p.pp;
     P.xpp_src = p.x;
     P.x_pp = p.x_pp;
@@ -527,10 +524,9 @@ hipError_t launch_prologue(convnd_hip_dtype dtype, const PrologueParts& p, hipSt
                                    (p.pp->copies == 2 && p.pp->shift[1] != 1)))
       return hipErrorInvalidValue;
     P.e_nc_copy = static_cast<int>(p.pp_batch * p.pp->channels);
-    P.e_all_parts = split && p.pp->last_stride == 1 && p.pp_blocks == 3 &&
-                    p.pp_part_map == kSplitPartsMap;
-    P.e_total = p.pp->copies * (P.e_all_parts ? p.split_batch : p.pp_batch) * p.pp->channels *
-                (p.pp->pvol / 8);
+    // (One read of a run for its three parts, but for a strided last axis.)
+    P.e_total = p.pp->copies * (split && p.pp->last_stride == 1 ? p.split_batch : p.pp_batch) *
+                p.pp->channels * (p.pp->pvol / 8);
     if (P.e_total > 0x7fffffff) return hipErrorInvalidValue;  // 32-bit run indices
     const int64_t per = (int64_t)stage::kPlanarRuns * kThreads;
     P.e_blocks = static_cast<int>((P.e_total + per - 1) / per);

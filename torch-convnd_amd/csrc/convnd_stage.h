@@ -532,8 +532,7 @@ __device__ __forceinline__ PlanarRunSrc planar_run_src(const PlanarPadArgs& P, i
 template <typename Src>
 __device__ __forceinline__ void pad_planar_strided_blocks(const Src* src, unsigned short* dst,
                                                           const PlanarPadArgs& P, int ntotal,
-                                                          int nc_copy, int split_nc,
-                                                          unsigned part_map, int block) {
+                                                          int nc_copy, int split_nc, int block) {
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
@@ -548,9 +547,8 @@ __device__ __forceinline__ void pad_planar_strided_blocks(const Src* src, unsign
     }
     int part = 0;
     if constexpr (sizeof(Src) == 4) {
-      const int s = nc / split_nc;
-      nc -= s * split_nc;
-      part = split_map_part(part_map, s);
+      part = nc / split_nc;
+      nc -= part * split_nc;
     }
     int srow = 0, istr = P.last_in;
     bool ok = true;
@@ -616,7 +614,7 @@ __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
   // 32-bit run indices: the planner keeps the copy and the source below 2^31 elements.
   const int ntotal = static_cast<int>(total);
   if (P.last_stride > 1) {
-    pad_planar_strided_blocks<unsigned short>(src, dst, P, ntotal, nc_copy, 0, 0u, block);
+    pad_planar_strided_blocks<unsigned short>(src, dst, P, ntotal, nc_copy, 0, block);
     return;
   }
   // The two aligned 16-byte chunks that cover each run's 8 source elements (starting at
@@ -667,39 +665,28 @@ __device__ __forceinline__ void pad_planar16_blocks(const unsigned short* src,
   }
 }
 
-// Split-precision form: an fp32 source of split_nc (image, channel) rows gives blocks of
-// split_nc destination rows, destination row block s holding bf16 part
-// split_map_part(part_map, s) of every source element. A run's 8 fp32 elements start at
-// element o of
-// the first of three aligned 16-byte chunks (the buffer's per-dword range check reads zero
-// past the source's end). With all_parts (three blocks, parts 0, 1, 2; unit last stride) the
+// Split-precision form: an fp32 source of split_nc (image, channel) rows gives three blocks of
+// split_nc destination rows per copy, block s holding bf16 part s of every source element. A
+// run's 8 fp32 elements start at element o of the first of three aligned 16-byte chunks (the
+// buffer's per-dword range check reads zero past the source's end). With a unit last stride the
 // runs are those of one block per copy, each read once and written to all three.
 __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsigned short* dst,
                                                         const PlanarPadArgs& P, int64_t total,
-                                                        int split_nc, unsigned part_map,
-                                                        int nc_copy, bool all_parts,
-                                                        int block) {
+                                                        int split_nc, int nc_copy, int block) {
   const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(src), static_cast<short>(0), static_cast<int>(P.src_bytes), 0x00020000);
   const int64_t nbytes = static_cast<int64_t>(P.src_bytes);
   const int ntotal = static_cast<int>(total);
   if (P.last_stride > 1) {
-    pad_planar_strided_blocks<float>(src, dst, P, ntotal, nc_copy, split_nc, part_map, block);
+    pad_planar_strided_blocks<float>(src, dst, P, ntotal, nc_copy, split_nc, block);
     return;
   }
   u32x4 c0[kPlanarRuns], c1[kPlanarRuns], c2[kPlanarRuns];
-  int o[kPlanarRuns], lo[kPlanarRuns], hi[kPlanarRuns], part[kPlanarRuns];
+  int o[kPlanarRuns], lo[kPlanarRuns], hi[kPlanarRuns];
 #pragma unroll
   for (int q = 0; q < kPlanarRuns; ++q) {
     const int t = (block * kPlanarRuns + q) * kThreads + static_cast<int>(threadIdx.x);
-    PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, all_parts ? split_nc : nc_copy);
-    part[q] = 0;
-    if (!all_parts) {
-      // Destination row block s reads source row nc - s * split_nc.
-      const int s = r.nc / split_nc;
-      r.first -= (int64_t)s * split_nc * P.in_vol;
-      part[q] = split_map_part(part_map, s);
-    }
+    const PlanarRunSrc r = planar_run_src(P, t < ntotal ? t : 0, split_nc);
     const bool live = t < ntotal && r.lo < r.hi;
     const int64_t chunk = r.first >= 0 ? r.first >> 2 : -((3 - r.first) >> 2);  // floor(/4)
     o[q] = static_cast<int>(r.first - chunk * 4);
@@ -724,22 +711,14 @@ __device__ __forceinline__ void pad_planar_split_blocks(const float* src, unsign
         if (o[q] == k) x = d[e + k];
       f[e] = e >= lo[q] && e < hi[q] ? __builtin_bit_cast(float, x) : 0.f;
     }
-    if (all_parts) {
-      // Run t of one block's runs per copy: its three part images lie a block apart.
-      const int64_t block_runs = ntotal / P.copies;
-      const int64_t copy = t / block_runs;
-      unsigned short* dt = dst + (copy * 2 * block_runs + t) * 8;
-      u32x4 w[3];
-      split_parts8(f, w);
+    // Run t of one block's runs per copy: its three part images lie a block apart.
+    const int64_t block_runs = ntotal / P.copies;
+    const int64_t copy = t / block_runs;
+    unsigned short* dt = dst + (copy * 2 * block_runs + t) * 8;
+    u32x4 w[3];
+    split_parts8(f, w);
 #pragma unroll
-      for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dt + p * block_runs * 8) = w[p];
-      continue;
-    }
-    unsigned h[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = bf16_part_bits(f[e], part[q]);
-    *reinterpret_cast<u32x4*>(dst + (size_t)t * 8) =
-        u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+    for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x4*>(dt + p * block_runs * 8) = w[p];
   }
 }
 
