@@ -486,9 +486,12 @@ int64_t prologue_sum_blocks(int64_t batch, int64_t volume);
 // split_other_part); kSplitPartsMap: a copy of the three parts themselves.
 constexpr unsigned kSplitDataMap = 0x120100u;   // 0, 0, 1, 0, 2, 1
 constexpr unsigned kSplitOtherMap = 0x102010u;  // 0, 1, 0, 2, 0, 1
-// Eight products, smallest first (all but (2, 2)): data parts 1 2 1 2 0 1 0 0 with 2 1 1 0 2 0 1 0.
+// Eight products, smallest first (all but (2, 2)): data parts 1 2 1 2 0 1 0 0 with 2 1 1 0 2 0 1 0;
+// without the first two, the six above in that order.
 constexpr unsigned kSplitData8Map = 0x00102121u;
 constexpr unsigned kSplitOther8Map = 0x01020112u;
+constexpr unsigned kSplitData6Map = kSplitData8Map >> 8;
+constexpr unsigned kSplitOther6Map = kSplitOther8Map >> 8;
 constexpr unsigned kSplitPartsMap = 0x210u;     // 0, 1, 2
 struct IgemmArgs;
 struct WgradArgs;
