@@ -840,6 +840,7 @@ void igemm_kernel(IgemmArgs A) {
     // chunk, staged for the first. Half of a strided input gradient's workgroup was staging the
     // halo that its phases share: 128 <- 64 channels in 4 groups, stride 2 on three axes, 24^3 x 12,
     // 103 -> 79 us.
+    const bool taps_inner = P == 1 && std::is_same<O, float>::value && A.taps_inner;
     for (int q = 0;;) {
       for (int tc = 0, ck = 0, last = 0;;) {
         // Every wave is past the staging that read the rows (the last chunk's barrier).
@@ -854,9 +855,9 @@ void igemm_kernel(IgemmArgs A) {
         }
         mma_chunk(tc * A.nchunk + ck, lds, []() {});
         // Chunks of a split tap, then the next tap; or the taps of a chunk (IgemmArgs::taps_inner).
-        if (A.taps_inner ? ++tc == A.tcount : ++ck == A.nchunk) {
-          if (A.taps_inner ? ++ck == A.nchunk : ++tc == A.tcount) break;
-          (A.taps_inner ? tc : ck) = 0;
+        if (taps_inner ? ++tc == A.tcount : ++ck == A.nchunk) {
+          if (taps_inner ? ++ck == A.nchunk : ++tc == A.tcount) break;
+          (taps_inner ? tc : ck) = 0;
         }
       }
       store_outputs();
