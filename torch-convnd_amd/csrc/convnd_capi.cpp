@@ -242,7 +242,7 @@ struct IgemmPlan {
   IgemmArgs args{};
   size_t lds = 0;
   size_t wpk_elems = 0;
-  size_t staged_elems = 0;  // channels-last copy of the GEMM's input operand
+  size_t staged_elems = 0;  // octet-major copy of the GEMM's input operand
   size_t table_bytes = 0;   // geometry tables (IgemmArgs::tables)
   PadArgs stage{};          // octet-major copy of the GEMM input (no padding)
   // 16-bit GEMM input whose channels per group are no whole octets: staged with zero channels
@@ -608,9 +608,10 @@ const PlanFilter& plan_filter(int mode) {
 // see convnd_types.h), when the real channel count per group is small enough to stage.
 constexpr int kSplit = 6;
 constexpr int kSplitMaxChannels = 64;
-// Wider layers (three-part layout only) from one full tile of output channels on (72 -> 16
-// channels, 3^4 taps, 4x4x4x8: 2809 -> 65 us; 96 -> 96 on 8^4, both directions: 25.2 -> 0.44 ms).
-// Narrower ones are pinned to the direct kernels by the plan test.
+// Wider layers (three-part layout only) from one full tile of output channels on (one call of 72 ->
+// 16 channels, 3^4 taps, 4x4x4x8: 2815 us on the direct kernel, 55 us here; 96 -> 96 on 8^4: 10.5 ms,
+// 90 us). Narrower ones run on the direct kernels, as the plan test has it; this side of the line
+// is not measured.
 constexpr int kSplitWideOut = 16;
 
 IgemmPlan plan_igemm_filtered(const Geom& g, convnd_hip_dtype dt, int mode,
@@ -1076,9 +1077,9 @@ struct WgradPlan {
   size_t dy_pad_elems = 0;   // grad_output padded to whole boxes (used when needed)
   size_t partial_elems = 0;
   double cost = 0.0;
-  // Channel-major kernel (convnd_wgrad_cm.hip) in place of the octet-major one: reads the
-  // caller's input directly (no staged copy); `args` then only describes grad_output for
-  // the padded copy (rank, extents, batch, channels).
+  // Channel-major kernel (convnd_wgrad_cm.hip) in place of the octet-major one: reads zero-padded
+  // channels-first copies of the input; `args` then only describes grad_output for the padded
+  // copy (rank, extents, batch, channels).
   bool cm = false;
   bool or_direct = false;  // as IgemmPlan::or_direct
   WgradCmArgs cm_args{};
@@ -1086,8 +1087,8 @@ struct WgradPlan {
 };
 
 // Channel-major weight-gradient plan: 16-bit data, or split-precision fp32 (kSplit bf16 part
-// images per image, both operands read from part copies), and a unit stride along the last
-// axis (the runs of a halo row are contiguous in the padded input).
+// images per image, both operands read from part copies); a strided last axis reads a copy of
+// the padded input per stride phase (the runs of a halo row are contiguous in each).
 bool plan_wgrad_cm(const Geom& g, convnd_hip_dtype dt, const PlanFilter& filter,
                    WgradPlan* out) {
   const bool split = dt == CONVND_HIP_FLOAT32;
@@ -2407,7 +2408,7 @@ int run_backward(const Geom& g, convnd_hip_dtype dtype, const BackwardSetup& b,
     pp.x_pp = ws + b.off_x_stage;
     pp.pp_batch = WA.batch;
     // Split-precision fp32: the three bf16 part images of both operands (the item table pairs
-    // them into the six products).
+    // them into the products).
     if (dtype == CONVND_HIP_FLOAT32) {
       pp.split_batch = static_cast<int>(g.batch);
       pp.dy_part_map = kSplitPartsMap;

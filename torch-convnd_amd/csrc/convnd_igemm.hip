@@ -58,7 +58,7 @@ __device__ __forceinline__ void unrolled(F&& body) {
 }
 
 // The part products of one K32 step, smallest first: position parts b, weight parts a. Six of them
-// into one accumulator; with NP = 8 all but the one below 2^-28 of the product, the seven cross
+// into one accumulator; with NP = 8 all but the one below 2^-30 of the product, the seven cross
 // products in an accumulator of their own, so that neither a truncated part nor a small product
 // added to a large sum is lost.
 template <typename M, int MB, int NB, int NP>

@@ -38,9 +38,11 @@ __device__ __forceinline__ T narrow(A v) {
 // every subtraction is exact), so v = p0 + p1 + p2 exactly for fp32 v and every part has
 // the sign of v, |p1| < 2^-7 |v|, |p2| < 2^-15 |v|. A product x*w keeps the six part
 // products (0,0) (0,1) (1,0) (0,2) (2,0) (1,1) accumulated in fp32 (the dropped ones are
-// below 2^-21 |x w| together): the GEMM runs over six copies of the channel (or batch)
-// dimension, the data operand contributing parts kSplitData[s] and the other operand parts
-// kSplitOther[s].
+// below 2^-21 |x w| together): the GEMM runs over the three parts of both operands, or over
+// six copies of the channel (or batch) dimension, copy s of the data operand holding part
+// split_data_part(s) and of the other operand part split_other_part(s). Layers that fp32
+// products served before keep (1,2) and (2,1) too, eight products (below 2^-30 dropped), and add
+// the small ones up first or apart (part_products in the implicit GEMM, kSplitData8Map).
 // Non-finite values and the other operand: a non-finite v gives v in all three parts, and a
 // part of a finite nonzero v that would be zero is replaced by p0 * 2^-40 (same sign), so
 // every product that meets an infinity carries the sign of x*w and a zero only meets it
