@@ -2074,6 +2074,9 @@ TablesRef device_tables(const std::string& key, size_t bytes, hipStream_t stream
   e->bytes = bytes;
   if (hipHostMalloc(&e->host, bytes, hipHostMallocDefault) != hipSuccess ||
       hipMalloc(&e->dev, bytes) != hipSuccess) {
+    // The runtime keeps the error until it is read, and the launch check of a direct kernel that
+    // runs instead (or_direct) would find it.
+    (void)hipGetLastError();
     fail(CONVND_HIP_LAUNCH_FAILED, "geometry tables: device allocation failed");
     return nullptr;
   }
