@@ -43,6 +43,8 @@ __device__ __forceinline__ T narrow(A v) {
 // split_data_part(s) and of the other operand part split_other_part(s). Layers that fp32
 // products served before keep (1,2) and (2,1) too, eight products (below 2^-30 dropped), and add
 // the small ones up first or apart (part_products in the implicit GEMM, kSplitData8Map).
+// bf16 ends at 2^-133: of a value below about 2^-110 (1e-33) the smallest part is cut short, a
+// relative error of up to 2^-133 / |v| (measured: 5e-6 at 1e-35, 5e-3 at 1e-38).
 // Non-finite values and the other operand: a non-finite v gives v in all three parts, and a
 // part of a finite nonzero v that would be zero is replaced by p0 * 2^-40 (same sign), so
 // every product that meets an infinity carries the sign of x*w and a zero only meets it
