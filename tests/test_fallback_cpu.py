@@ -160,3 +160,24 @@ def test_noalloc_takes_plans_that_fit_its_scratch(lib, x_shape, w_shape, stride,
     status = noalloc(lib, problem, _capi.BFLOAT16)
     # (Taken: the call goes on to the device, which is not there.)
     assert status == (_capi.LAUNCH_FAILED if taken else _capi.WORKSPACE_TOO_SMALL)
+
+
+@pytest.mark.parametrize(
+    ("x_shape", "w_shape", "plan"),
+    [
+        ((1, 1, 6, 5, 7, 5, 5), (72, 1, 1, 1, 1, 1, 1), b"direct"),
+        ((1, 1, 8, 8, 8, 8), (40, 1, 2, 1, 1, 1), b"direct"),
+        ((1, 4, 4, 4, 4, 4), (60, 4, 1, 1, 1, 1), b"direct"),
+        # Just more outputs, or products.
+        ((1, 2, 6, 5, 7, 5, 5), (72, 2, 1, 1, 1, 1, 1), b"mfma"),
+        ((1, 1, 8, 8, 8, 9), (40, 1, 2, 2, 1, 1), b"mfma"),
+        ((1, 5, 4, 4, 4, 4), (60, 5, 1, 1, 1, 1), b"mfma"),
+    ],
+)
+def test_forwards_of_a_few_products_take_one_launch(lib, x_shape, w_shape, plan):
+    rank = len(x_shape) - 2
+    problem = _capi.Problem.make(x_shape, w_shape, (1,) * rank, (0,) * rank, (1,) * rank, 1)
+    ref = ctypes.byref(problem)
+    assert lib.convnd_hip_plan_name(ref, _capi.BFLOAT16, 0) == plan
+    # (The workspace is the GEMM's: with an activation, applied before the one rounding, it runs.)
+    assert lib.convnd_hip_forward_workspace_size(ref, _capi.BFLOAT16) > 0

@@ -2229,6 +2229,18 @@ int run_forward(const Geom& g, convnd_hip_dtype dtype, const ForwardSetup& f, co
   return st;
 }
 
+// Forwards without activation of a few products per output and few outputs, of the layers that the
+// direct kernel served before, run there (channels-last ones too, on their copies: the same results):
+// its one launch is shorter than the two of packing and GEMM where calls follow each other. In such a
+// stream, 1 / 2 / 4 / 9 -> 72 channels, no taps, on 6x5x7x5x5 (378,000 outputs): direct 15.6 / 19.6 /
+// 27.4 / 47.4 us a call, implicit GEMM 19.2 each; 1 -> 40 channels, two taps, on 8^4 (143,360
+// outputs): 14.7 against 19.5. (A call waited for by itself: 35.6 against 32.9, 29.5 against 29.6.)
+bool one_launch_forward(const Geom& g, const IgemmPlan& ig, int activation) {
+  const int64_t products = g.cin_g * g.k_vol;
+  return ig.ok && ig.or_direct && activation == CONVND_HIP_ACT_NONE && products <= 4 &&
+         products * g.batch * g.out_channels * g.out_vol <= (int64_t{1} << 19);
+}
+
 // The forward plan's geometry tables (kept null for the plans without any). A first call under
 // stream capture has none: an or_direct plan then becomes the direct kernel's, any other fails.
 bool forward_tables(const Geom& g, convnd_hip_dtype dtype, ForwardSetup* f, hipStream_t stream,
@@ -2616,7 +2628,10 @@ const char* convnd_hip_plan_name(const convnd_hip_problem* problem, convnd_hip_d
     const TinyPlan t = plan_tiny(g, dtype, which == 1 ? 1 : 0);
     if (t.ok && (which != 2 || t.wlds > 0)) return "tiny";
   }
-  if (which == 0) return plan_igemm(g, dtype, 0).ok ? "mfma" : "direct";
+  if (which == 0) {
+    const IgemmPlan p = plan_igemm(g, dtype, 0);
+    return p.ok && !one_launch_forward(g, p, CONVND_HIP_ACT_NONE) ? "mfma" : "direct";
+  }
   if (which == 1) return plan_igemm(g, dtype, 1).ok ? "mfma" : "direct";
   return plan_wgrad(g, dtype).ok ? "mfma" : "direct";
 }
@@ -2644,6 +2659,7 @@ int convnd_hip_forward_act(const convnd_hip_problem* problem, convnd_hip_dtype d
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "device workspace is smaller than convnd_hip_forward_workspace_size");
   TablesRef tables;  // held until the kernels that read them are enqueued
+  if (one_launch_forward(g, f.ig, activation)) f.ig.ok = false;
   if (!forward_tables(g, dtype, &f, stream, &tables)) return CONVND_HIP_LAUNCH_FAILED;
   return run_forward(g, dtype, f, input, weight, bias, output, activation,
                      static_cast<char*>(workspace), tables ? tables->dev : nullptr, nullptr, true,
@@ -2658,7 +2674,8 @@ int convnd_hip_forward_noalloc(const convnd_hip_problem* problem, convnd_hip_dty
   if (st != CONVND_HIP_SUCCESS) return st;
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   if (g.batch == 0) return CONVND_HIP_SUCCESS;
-  const ForwardSetup f = setup_noalloc(g, dtype);
+  ForwardSetup f = setup_noalloc(g, dtype);
+  if (one_launch_forward(g, f.ig, CONVND_HIP_ACT_NONE)) f.ig.ok = false;
   if (!f.ig.ok)  // the direct kernels use no scratch
     return run_forward(g, dtype, f, input, weight, bias, output, CONVND_HIP_ACT_NONE, nullptr,
                        nullptr, nullptr, false, stream);
@@ -2741,6 +2758,7 @@ int convnd_hip_forward_layout(const convnd_hip_problem* problem, convnd_hip_dtyp
     return fail(CONVND_HIP_WORKSPACE_TOO_SMALL,
                 "device workspace is smaller than convnd_hip_forward_workspace_size_layout");
   TablesRef tables;  // held until the kernels that read them are enqueued
+  if (one_launch_forward(g, f.ig, activation)) f.ig.ok = false;
   if (!forward_tables(g, dtype, &f, stream, &tables)) return CONVND_HIP_LAUNCH_FAILED;
   char* ws = static_cast<char*>(workspace);
   const void* tab = tables ? tables->dev : nullptr;
