@@ -1,8 +1,8 @@
 // Direct N-d convolution kernels for gfx950 with 64-bit index arithmetic.
 //
 // They serve every shape the MFMA and tiny-channel kernels do not: float64, ranks above eight,
-// huge strides/dilations/padding, and calls of other shapes that cannot have the MFMA kernels'
-// scratch or geometry tables. Each output
+// huge strides/dilations/padding, forwards of a few products per output, and calls of other shapes
+// that cannot have the MFMA kernels' scratch or geometry tables. Each output
 // element is computed by one thread (forward, input gradient) or one workgroup
 // (weight gradient) in a fixed summation order, so results are deterministic.
 //
